@@ -2730,15 +2730,16 @@ static int mlp_features_impl(dhip_mlp *q, const double *const hist[4], int32_t n
     return DHIP_OK;
 }
 
-// gradient (double, q->grad) and loss of a minibatch; returns the tile count
+// gradient (double, q->grad) and loss of a minibatch
 static int mlp_grad_impl(dhip_mlp *q, const float *X, const float *T, const int32_t *idx, int64_t B) {
     dhip_ctx *c = q->ctx;
-    const int64_t tiles = (B + TS - 1) / TS;
-    DHIP_HIPCHK(c, q->part.ensure(sizeof(float) * (size_t)(tiles + 1) * (MLP_NPARAM + 1)));
+    // four waves of 16 samples a block, one block per CU at most (the blocks walk the tiles)
+    const int64_t blocks = std::min<int64_t>((B + TSW * TW - 1) / (TSW * TW), c->cu_count);
+    DHIP_HIPCHK(c, q->part.ensure(sizeof(float) * (size_t)blocks * (MLP_NPARAM + 1)));
     TrainArgs ta{X, T, idx, B, q->theta.as<float>(), q->part.as<float>()};
-    DHIP_LAUNCH(c, "mlp_train", k_mlp_train, (unsigned)tiles, TRAIN_T, 0, ta);
-    DHIP_LAUNCH(c, "mlp_reduce", k_mlp_reduce, blocks_for(MLP_NPARAM + 1, 256), 256, 0, q->part.as<float>(),
-                (int)tiles, q->grad.as<double>());
+    DHIP_LAUNCH(c, "mlp_train", k_mlp_train, (unsigned)blocks, TRAIN_T, TRAIN_LDS, ta);
+    DHIP_LAUNCH(c, "mlp_reduce", k_mlp_reduce, blocks_for(MLP_NPARAM + 1, 64), 64 * MLP_RED_G, 0,
+                q->part.as<float>(), (int)blocks, q->grad.as<double>());
     return DHIP_OK;
 }
 
@@ -2761,6 +2762,13 @@ int dhip_mlp_create(dhip_ctx_t *c, dhip_mlp_t **out) {
         for (DevBuf *x : b) x->release();
         delete q;
         return set_error(c, DHIP_E_NOMEM, "network buffers");
+    }
+    if (hipFuncSetAttribute((const void *)k_mlp_train, hipFuncAttributeMaxDynamicSharedMemorySize,
+                            (int)TRAIN_LDS) != hipSuccess) {
+        DevBuf *b[] = {&q->theta, &q->m, &q->v, &q->packed, &q->grad};
+        for (DevBuf *x : b) x->release();
+        delete q;
+        return set_error(c, DHIP_E_HIP, "the training kernel's LDS");
     }
     *out = q;
     return DHIP_OK;

@@ -7,12 +7,13 @@
 //                   normalised, stored float32 [S][12].
 //   k_mlp_infer     matrix cores: one wave per 16 DOFs, v_mfma_f32_16x16x32_bf16 for every layer
 //                   (bf16 weights and layer inputs, float32 accumulation); weights staged in LDS.
-//   k_mlp_train     training tile of 32 samples per block: forward with the same rounding points
-//                   as k_mlp_infer (float32 FMA on bf16-rounded operands), backward, and the
-//                   tile's gradient written to its own slot (no atomics).
-//   k_mlp_reduce    gradient = sum of the tile slots in tile order; k_mlp_adam the update.
+//   k_mlp_train     matrix cores: 16 samples per wave, forward with k_mlp_infer's rounding points,
+//                   backward in float32, gradients accumulated in registers over the wave's tiles;
+//                   a block's gradient goes to its own slot (no atomics).
+//   k_mlp_reduce    gradient = sum of the block slots in slot order; k_mlp_adam the update.
 #pragma once
 
+#include "dhip_assembly.hpp"
 #include "dhip_common.hpp"
 
 namespace dhip {
@@ -285,153 +286,368 @@ __global__ void __launch_bounds__(64 * INFER_WAVES) k_mlp_infer(const float *X, 
 
 // ---------------------------------------------------------------------------------------------
 // training
-constexpr int TS = 32;        // samples per block
-constexpr int TRAIN_T = 256;  // threads per block
+//
+// One wave owns 16 samples at a time and keeps them in registers from the forward pass to the last
+// weight gradient; nothing waits for another wave until the block's gradients are added up.
+//   * Products are taken with the units as the matrix rows and the samples as the columns, so a lane
+//     holds units 16 t + 4 q + i (q = lane / 16, i = 0..3) of sample lane % 16, and that register file is
+//     the B operand of the next product when its contraction index is enumerated in the same order: the
+//     forward weights are staged in that order, the backward ones are read through it.
+//   * Forward: bf16 weights and layer inputs, v_mfma_f32_16x16x32_bf16 (as k_mlp_infer).  Backward: the
+//     float32 deltas meet float32 copies of the rounded weights and inputs in v_mfma_f32_16x16x4_f32, so
+//     no operand is rounded further.
+//   * Weight gradients contract over the samples: delta and layer input go through LDS once per layer
+//     (rows of 68 floats: the lanes' four sample rows 4 q + kk lie 16 banks apart), into 160
+//     accumulators that live as long as the wave.
+// A block adds its waves' sums in LDS and writes one slot; k_mlp_reduce adds the slots in float64.
+// Bound by the float32 matrix rate and the tanh evaluations, about 9,500 matrix cycles per 16 samples.
+// At 65,536 samples on 256 CUs 82 us (27 of it the staged weights, the block sums and the launch, 13.5 per
+// tile of a wave); 32 samples a block with every product on the vector units and one slot per 32 samples
+// took 350 us.
+constexpr int TW = 4;               // waves per block
+constexpr int TRAIN_T = 64 * TW;    // threads per block
+constexpr int TSW = 16;             // samples per wave and pass
+constexpr int TLD = 68;             // row length of the LDS tiles and of the float32 weights
 
 struct TrainArgs {
     const float *X, *T;       // [S][12], [S][2]
     const int32_t *idx;       // minibatch sample ids
     int64_t B;                // minibatch size
     const float *theta;
-    float *part;              // [tiles][MLP_NPARAM + 1] (last: loss)
+    float *part;              // [blocks][MLP_NPARAM + 1] (last: loss)
 };
 
-// out[s][n] (+)= sum_k A[s][k] * Wt[n][k], tile TS x 64: thread -> 2 samples x 4 outputs
-template <int K>
-__device__ inline void fwd_gemm(const float (*A)[MLP_H], const float *Wt, const float *b, float (*Hout)[MLP_H]) {
-    const int t = threadIdx.x, s0 = 2 * (t >> 4), n0 = 4 * (t & 15);
-    float acc[2][4];
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = 0.f;
-    for (int k = 0; k < K; ++k) {
-        const float a0 = bfround(A[s0][k]), a1 = bfround(A[s0 + 1][k]);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const float w = Wt[(n0 + j) * K + k];
-            acc[0][j] = __fmaf_rn(a0, w, acc[0][j]);
-            acc[1][j] = __fmaf_rn(a1, w, acc[1][j]);
-        }
-    }
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) Hout[s0 + i][n0 + j] = tanhf(acc[i][j] + b[n0 + j]);
+// bf16 forward weights as A fragments of v_mfma_f32_16x16x32_bf16: [fragment][lane][8].
+constexpr int TF_1 = 0, TF_2 = 4, TF_3 = 12, TF_4 = 20, TF_N = 22;
+
+struct TrainShared {
+    __align__(16) uint16_t frag[TF_N * 64 * 8];
+    float w2[MLP_H * TLD], w3[MLP_H * TLD];   // rounded weights [out][in] for the backward products
+    float w4[MLP_NO * MLP_H];
+    float bias[3 * MLP_H + MLP_NO];
+    __align__(16) float dz[TW][TSW * TLD], in[TW][TSW * TLD];
+    __align__(16) float theta[MLP_NPARAM];
+};
+// the waves' gradients at the end take the same LDS
+constexpr size_t TRAIN_LDS = sizeof(TrainShared) > sizeof(float) * TW * (MLP_NPARAM + 1)
+                                 ? sizeof(TrainShared) : sizeof(float) * TW * (MLP_NPARAM + 1);
+
+// weight of out unit n at in unit k (layer 1: k >= 12 is padding; layer 4: n >= 2)
+__device__ inline float train_weight(const float *th, int layer, int n, int k) {
+    if (layer == 1) return k < MLP_NF ? th[MLP_W1 + n * MLP_NF + k] : 0.f;
+    if (layer == 4) return n < MLP_NO ? th[MLP_W4 + n * MLP_H + k] : 0.f;
+    return th[(layer == 2 ? MLP_W2 : MLP_W3) + n * MLP_H + k];
 }
 
 __global__ void __launch_bounds__(TRAIN_T) k_mlp_train(TrainArgs a) {
-    __shared__ float Wr[MLP_NPARAM];               // bf16-rounded weights, float32 biases
-    __shared__ float A0[TS][MLP_H];                // inputs (first 12 columns)
-    __shared__ float H[3][TS][MLP_H];              // tanh outputs (unrounded)
-    __shared__ float D0[TS][MLP_H], D1[TS][MLP_H];  // backward buffers
-    __shared__ float dY[TS][MLP_NO];
-    __shared__ float lsum[TS];
-    const int t = threadIdx.x;
-    for (int p = t; p < MLP_NPARAM; p += TRAIN_T) {
-        const bool isw = (p < MLP_B1) || (p >= MLP_W2 && p < MLP_B2) || (p >= MLP_W3 && p < MLP_B3) ||
-                         (p >= MLP_W4 && p < MLP_B4);
-        Wr[p] = isw ? bfround(a.theta[p]) : a.theta[p];
-    }
-    const int64_t base = (int64_t)blockIdx.x * TS;
-    for (int e = t; e < TS * MLP_NF; e += TRAIN_T) {
-        const int s = e / MLP_NF, k = e % MLP_NF;
-        const int64_t g = base + s;
-        A0[s][k] = g < a.B ? a.X[(int64_t)a.idx[g] * MLP_NF + k] : 0.f;
-    }
-    __syncthreads();
-    fwd_gemm<MLP_NF>(A0, Wr + MLP_W1, Wr + MLP_B1, H[0]);
-    __syncthreads();
-    fwd_gemm<MLP_H>(H[0], Wr + MLP_W2, Wr + MLP_B2, H[1]);
-    __syncthreads();
-    fwd_gemm<MLP_H>(H[1], Wr + MLP_W3, Wr + MLP_B3, H[2]);
-    __syncthreads();
-    // output, residual, loss (0.5 |y - t|^2 per sample), dY = (y - t) / B
-    if (t < TS * MLP_NO) {
-        const int s = t / MLP_NO, o = t % MLP_NO;
-        const int64_t g = base + s;
-        float y = 0.f;
-        for (int k = 0; k < MLP_H; ++k) y = __fmaf_rn(bfround(H[2][s][k]), Wr[MLP_W4 + o * MLP_H + k], y);
-        y += Wr[MLP_B4 + o];
-        const float d = g < a.B ? y - a.T[(int64_t)a.idx[g] * MLP_NO + o] : 0.f;
-        dY[s][o] = d / (float)a.B;
-        D0[s][o] = 0.5f * d * d;  // scratch for the loss
-    }
-    __syncthreads();
-    if (t < TS) lsum[t] = D0[t][0] + D0[t][1];
-    __syncthreads();
-    float *G = a.part + (size_t)blockIdx.x * (MLP_NPARAM + 1);
-    if (t == 0) {
-        float l = 0.f;
-        for (int s = 0; s < TS; ++s) l += lsum[s];
-        G[MLP_NPARAM] = l;
-    }
-    // output layer gradients
-    for (int p = t; p < MLP_NO * MLP_H; p += TRAIN_T) {
-        const int o = p / MLP_H, k = p % MLP_H;
-        float g = 0.f;
-        for (int s = 0; s < TS; ++s) g = __fmaf_rn(dY[s][o], bfround(H[2][s][k]), g);
-        G[MLP_W4 + p] = g;
-    }
-    if (t < MLP_NO) {
-        float g = 0.f;
-        for (int s = 0; s < TS; ++s) g += dY[s][t];
-        G[MLP_B4 + t] = g;
-    }
-    // dZ3 = (dY W4) * (1 - h3^2) into D0
-    for (int e = t; e < TS * MLP_H; e += TRAIN_T) {
-        const int s = e / MLP_H, k = e % MLP_H;
-        float v = 0.f;
+    extern __shared__ __align__(16) unsigned char train_lds[];
+    TrainShared &sh = *reinterpret_cast<TrainShared *>(train_lds);
+    const int t = threadIdx.x, lane = t & 63, wv = t >> 6, col = lane & 15, q = lane >> 4;
+    // the parameters once into LDS, every load in flight before the first use
+    {
+        constexpr int NV = (MLP_NPARAM / 2 + TRAIN_T - 1) / TRAIN_T;
+        float2 v[NV];
 #pragma unroll
-        for (int o = 0; o < MLP_NO; ++o) v = __fmaf_rn(dY[s][o], Wr[MLP_W4 + o * MLP_H + k], v);
-        const float h = H[2][s][k];
-        D0[s][k] = v * (1.f - h * h);
+        for (int u = 0; u < NV; ++u) {
+            const int e = t + u * TRAIN_T;
+            if (e < MLP_NPARAM / 2) v[u] = reinterpret_cast<const float2 *>(a.theta)[e];
+        }
+#pragma unroll
+        for (int u = 0; u < NV; ++u) {
+            const int e = t + u * TRAIN_T;
+            if (e < MLP_NPARAM / 2) reinterpret_cast<float2 *>(sh.theta)[e] = v[u];
+        }
     }
     __syncthreads();
-    // hidden layers 3, 2, 1: weight/bias gradients and the next dZ
-    float (*Dz)[MLP_H] = D0;
-    float (*Dn)[MLP_H] = D1;
-    for (int layer = 2; layer >= 0; --layer) {
-        const int wofs = layer == 2 ? MLP_W3 : layer == 1 ? MLP_W2 : MLP_W1;
-        const int bofs = layer == 2 ? MLP_B3 : layer == 1 ? MLP_B2 : MLP_B1;
-        const int K = layer == 0 ? MLP_NF : MLP_H;
-        const float (*In)[MLP_H] = layer == 0 ? A0 : H[layer - 1];
-        // dW[n][k] = sum_s dZ[s][n] * bf(In[s][k])
-        for (int p = t; p < MLP_H * K; p += TRAIN_T) {
-            const int nn = p / K, k = p % K;
-            float g = 0.f;
-            for (int s = 0; s < TS; ++s) g = __fmaf_rn(Dz[s][nn], bfround(In[s][k]), g);
-            G[wofs + p] = g;
+    const float *theta = sh.theta;
+    for (int e = t; e < TF_N * 512; e += TRAIN_T) {
+        const int f = e >> 9, ln = (e >> 3) & 63, x = e & 7, row = ln & 15, j = ln >> 4;
+        int layer, n, k;
+        if (f < TF_2) {
+            layer = 1;
+            n = 16 * f + row;
+            k = 8 * j + x;
+        } else {
+            layer = f < TF_3 ? 2 : f < TF_4 ? 3 : 4;
+            const int g = f - (layer == 2 ? TF_2 : layer == 3 ? TF_3 : TF_4);
+            n = 16 * (g >> 1) + row;
+            k = 16 * (2 * (g & 1) + (x >> 2)) + 4 * j + (x & 3);
         }
-        if (t < MLP_H) {
-            float g = 0.f;
-            for (int s = 0; s < TS; ++s) g += Dz[s][t];
-            G[bofs + t] = g;
+        sh.frag[e] = f2bf(train_weight(theta, layer, n, k));
+    }
+    for (int e = t; e < MLP_H * MLP_H; e += TRAIN_T) {
+        const int n = e / MLP_H, k = e % MLP_H;
+        sh.w2[n * TLD + k] = bfround(theta[MLP_W2 + e]);
+        sh.w3[n * TLD + k] = bfround(theta[MLP_W3 + e]);
+    }
+    for (int e = t; e < MLP_NO * MLP_H; e += TRAIN_T) sh.w4[e] = bfround(theta[MLP_W4 + e]);
+    for (int e = t; e < MLP_H; e += TRAIN_T) {
+        sh.bias[e] = theta[MLP_B1 + e];
+        sh.bias[MLP_H + e] = theta[MLP_B2 + e];
+        sh.bias[2 * MLP_H + e] = theta[MLP_B3 + e];
+    }
+    if (t < MLP_NO) sh.bias[3 * MLP_H + t] = theta[MLP_B4 + t];
+    __syncthreads();
+
+    floatx4_t g1[4], g2[4][4], g3[4][4], g4[4];   // dW tiles [out tile][in tile]; layer 1's column 12 is its bias
+    float gb2[16], gb3[16], gb4[2] = {0.f, 0.f}, loss = 0.f;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        g1[i] = g4[i] = floatx4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int j = 0; j < 4; ++j) g2[i][j] = g3[i][j] = floatx4_t{0.f, 0.f, 0.f, 0.f};
+    }
+#pragma unroll
+    for (int i = 0; i < 16; ++i) gb2[i] = gb3[i] = 0.f;
+
+    float *dz = sh.dz[wv], *in = sh.in[wv];
+    auto frag = [&](int f) { return *reinterpret_cast<const bf16x8_t *>(&sh.frag[(f * 64 + lane) * 8]); };
+    // tanh of a layer's products, in place
+    auto activate = [&](float (&h)[4][4], const float *b) {
+#pragma unroll
+        for (int nt = 0; nt < 4; ++nt)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) h[nt][i] = tanhf(h[nt][i] + b[16 * nt + 4 * q + i]);
+    };
+    // the rounded layer inputs of contraction step ks
+    auto act_frag = [&](const float (&h)[4][4], int ks) {
+        bf16x8_t v;
+#pragma unroll
+        for (int x = 0; x < 8; ++x) v[x] = __builtin_bit_cast(__bf16, f2bf(h[2 * ks + (x >> 2)][x & 3]));
+        return v;
+    };
+    auto forward = [&](const float (&hin)[4][4], int f0, float (&hout)[4][4]) {
+        const bf16x8_t b0 = act_frag(hin, 0), b1 = act_frag(hin, 1);
+#pragma unroll
+        for (int nt = 0; nt < 4; ++nt) {
+            floatx4_t d = {0.f, 0.f, 0.f, 0.f};
+            d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(frag(f0 + 2 * nt), b0, d, 0, 0, 0);
+            d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(frag(f0 + 2 * nt + 1), b1, d, 0, 0, 0);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) hout[nt][i] = d[i];
         }
-        if (layer > 0) {
-            // dZ_prev[s][k] = (sum_n dZ[s][n] * W[n][k]) * (1 - h^2)
-            for (int e = t; e < TS * MLP_H; e += TRAIN_T) {
-                const int s = e / MLP_H, k = e % MLP_H;
-                float v = 0.f;
-                for (int nn = 0; nn < MLP_H; ++nn) v = __fmaf_rn(Dz[s][nn], Wr[wofs + nn * MLP_H + k], v);
-                const float h = H[layer - 1][s][k];
-                Dn[s][k] = v * (1.f - h * h);
+    };
+    auto store = [&](float *buf, const float (&v)[4][4], bool round) {
+#pragma unroll
+        for (int nt = 0; nt < 4; ++nt) {
+            floatx4_t x;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) x[i] = round ? bfround(v[nt][i]) : v[nt][i];
+            *reinterpret_cast<floatx4_t *>(&buf[col * TLD + 16 * nt + 4 * q]) = x;
+        }
+    };
+    // g[nt][kt] += dz^T in over the wave's 16 samples (sample 4 q + kk at step kk)
+    auto weight_grad = [&](floatx4_t (&g)[4][4]) {
+#pragma unroll
+        for (int kk = 0; kk < 4; ++kk) {
+            float av[4], bv[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                av[i] = dz[(4 * q + kk) * TLD + 16 * i + col];
+                bv[i] = in[(4 * q + kk) * TLD + 16 * i + col];
             }
-            __syncthreads();
-            float (*tmp)[MLP_H] = Dz;
-            Dz = Dn;
-            Dn = tmp;
+#pragma unroll
+            for (int nt = 0; nt < 4; ++nt)
+#pragma unroll
+                for (int kt = 0; kt < 4; ++kt)
+                    g[nt][kt] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[nt], bv[kt], g[nt][kt], 0, 0, 0);
         }
+    };
+    // delta of the layer below: (W^T d) (1 - h^2), the contraction index n = 16 nt + 4 q + i from d's registers
+    auto backward = [&](const float *w, const float (&d)[4][4], const float (&h)[4][4], float (&out)[4][4]) {
+        floatx4_t acc[4];
+#pragma unroll
+        for (int kt = 0; kt < 4; ++kt) acc[kt] = floatx4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int nt = 0; nt < 4; ++nt)
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int kt = 0; kt < 4; ++kt)
+                    acc[kt] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[(16 * nt + 4 * q + i) * TLD + 16 * kt + col],
+                                                                   d[nt][i], acc[kt], 0, 0, 0);
+#pragma unroll
+        for (int kt = 0; kt < 4; ++kt)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) out[kt][i] = acc[kt][i] * (1.f - h[kt][i] * h[kt][i]);
+    };
+
+    const int64_t ntile = (a.B + TSW - 1) / TSW;
+    for (int64_t tile = (int64_t)blockIdx.x * TW + wv; tile < ntile; tile += (int64_t)gridDim.x * TW) {
+        const int64_t g = tile * TSW + col;
+        const int64_t sid = g < a.B ? (int64_t)a.idx[g] : -1;
+        // features 8 q .. 8 q + 7 of the lane's sample (12 real ones, zero padding)
+        float x0[8];
+#pragma unroll
+        for (int x = 0; x < 8; ++x) {
+            const int k = 8 * q + x;
+            x0[x] = sid >= 0 && k < MLP_NF ? bfround(a.X[sid * MLP_NF + k]) : 0.f;
+        }
+        float tv[2] = {0.f, 0.f};
+        if (sid >= 0) {
+            tv[0] = a.T[sid * MLP_NO];
+            tv[1] = a.T[sid * MLP_NO + 1];
+        }
+        float h1[4][4], h2[4][4], h3[4][4];
+        {
+            bf16x8_t b;
+#pragma unroll
+            for (int x = 0; x < 8; ++x) b[x] = __builtin_bit_cast(__bf16, f2bf(x0[x]));
+#pragma unroll
+            for (int nt = 0; nt < 4; ++nt) {
+                floatx4_t d = {0.f, 0.f, 0.f, 0.f};
+                d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(frag(TF_1 + nt), b, d, 0, 0, 0);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) h1[nt][i] = d[i];
+            }
+        }
+        activate(h1, sh.bias);
+        forward(h1, TF_2, h2);
+        activate(h2, sh.bias + MLP_H);
+        forward(h2, TF_3, h3);
+        activate(h3, sh.bias + 2 * MLP_H);
+        // output (units 0 and 1 in lanes q = 0), residual, loss, dY = (y - t) / B
+        float dy[2];
+        {
+            floatx4_t d = {0.f, 0.f, 0.f, 0.f};
+            d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(frag(TF_4), act_frag(h3, 0), d, 0, 0, 0);
+            d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(frag(TF_4 + 1), act_frag(h3, 1), d, 0, 0, 0);
+#pragma unroll
+            for (int o = 0; o < MLP_NO; ++o) {
+                const float y = __shfl(d[o], col, 64) + sh.bias[3 * MLP_H + o];
+                const float r = sid >= 0 ? y - tv[o] : 0.f;
+                dy[o] = r / (float)a.B;
+                if (q == 0) loss += 0.5f * r * r;
+                if (q == 0) gb4[o] += dy[o];
+            }
+        }
+        // layer 4: weights and the delta of layer 3
+        store(in, h3, true);
+        float d3[4][4], d2[4][4], d1[4][4];
+#pragma unroll
+        for (int nt = 0; nt < 4; ++nt)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int n = 16 * nt + 4 * q + i;
+                const float v = __fmaf_rn(dy[1], sh.w4[MLP_H + n], dy[0] * sh.w4[n]);
+                d3[nt][i] = v * (1.f - h3[nt][i] * h3[nt][i]);
+                gb3[4 * nt + i] += d3[nt][i];
+            }
+        wave_sync_lds();
+#pragma unroll
+        for (int kk = 0; kk < 4; ++kk) {
+            const float e0 = __shfl(dy[0], 4 * q + kk, 64), e1 = __shfl(dy[1], 4 * q + kk, 64);
+            const float av = col == 0 ? e0 : col == 1 ? e1 : 0.f;
+#pragma unroll
+            for (int kt = 0; kt < 4; ++kt)
+                g4[kt] = __builtin_amdgcn_mfma_f32_16x16x4f32(av, in[(4 * q + kk) * TLD + 16 * kt + col], g4[kt], 0, 0, 0);
+        }
+        wave_sync_lds();
+        // layer 3
+        store(in, h2, true);
+        store(dz, d3, false);
+        wave_sync_lds();
+        weight_grad(g3);
+        wave_sync_lds();
+        backward(sh.w3, d3, h2, d2);
+#pragma unroll
+        for (int e = 0; e < 16; ++e) gb2[e] += d2[e >> 2][e & 3];
+        // layer 2
+        store(in, h1, true);
+        store(dz, d2, false);
+        wave_sync_lds();
+        weight_grad(g2);
+        wave_sync_lds();
+        backward(sh.w2, d2, h1, d1);
+        // layer 1: inputs 0..11, a one in column 12 for the bias
+        store(dz, d1, false);
+        if (q < 2) {
+#pragma unroll
+            for (int x = 0; x < 8; ++x) in[col * TLD + 8 * q + x] = 8 * q + x == MLP_NF ? 1.f : x0[x];
+        }
+        wave_sync_lds();
+#pragma unroll
+        for (int kk = 0; kk < 4; ++kk) {
+            const float bv = in[(4 * q + kk) * TLD + col];
+#pragma unroll
+            for (int nt = 0; nt < 4; ++nt)
+                g1[nt] = __builtin_amdgcn_mfma_f32_16x16x4f32(dz[(4 * q + kk) * TLD + 16 * nt + col], bv, g1[nt], 0, 0, 0);
+        }
+        wave_sync_lds();
+    }
+
+    // sums over the 16 lanes that share units
+    auto over_samples = [&](float v) {
+#pragma unroll
+        for (int o = 8; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+        return v;
+    };
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+        gb2[e] = over_samples(gb2[e]);
+        gb3[e] = over_samples(gb3[e]);
+    }
+    gb4[0] = over_samples(gb4[0]);
+    gb4[1] = over_samples(gb4[1]);
+    loss = over_samples(loss);
+    __syncthreads();
+    // every wave's gradient to LDS (over the weights and tiles), then their sum in wave order
+    float *G = reinterpret_cast<float *>(train_lds) + wv * (MLP_NPARAM + 1);
+#pragma unroll
+    for (int nt = 0; nt < 4; ++nt)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int n = 16 * nt + 4 * q + i;
+            if (col < MLP_NF) G[MLP_W1 + n * MLP_NF + col] = g1[nt][i];
+            else if (col == MLP_NF) G[MLP_B1 + n] = g1[nt][i];
+#pragma unroll
+            for (int kt = 0; kt < 4; ++kt) {
+                G[MLP_W2 + n * MLP_H + 16 * kt + col] = g2[nt][kt][i];
+                G[MLP_W3 + n * MLP_H + 16 * kt + col] = g3[nt][kt][i];
+            }
+            if (col == 0) {
+                G[MLP_B2 + n] = gb2[4 * nt + i];
+                G[MLP_B3 + n] = gb3[4 * nt + i];
+            }
+        }
+    if (q == 0) {
+#pragma unroll
+        for (int kt = 0; kt < 4; ++kt)
+#pragma unroll
+            for (int o = 0; o < MLP_NO; ++o) G[MLP_W4 + o * MLP_H + 16 * kt + col] = g4[kt][o];
+    }
+    if (lane == 0) {
+        G[MLP_B4] = gb4[0];
+        G[MLP_B4 + 1] = gb4[1];
+        G[MLP_NPARAM] = loss;
+    }
+    __syncthreads();
+    const float *W = reinterpret_cast<const float *>(train_lds);
+    float *P = a.part + (size_t)blockIdx.x * (MLP_NPARAM + 1);
+    for (int e = t; e < MLP_NPARAM + 1; e += TRAIN_T) {
+        float v = W[e];
+#pragma unroll
+        for (int w = 1; w < TW; ++w) v += W[w * (MLP_NPARAM + 1) + e];
+        P[e] = v;
     }
 }
 
-// grad[p] = sum over tiles (tile order) of part[tile][p]; p = MLP_NPARAM is the loss
-__global__ void k_mlp_reduce(const float *part, int ntiles, double *grad) {
-    const int p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p > MLP_NPARAM) return;
-    double s = 0.0;
-    for (int b = 0; b < ntiles; ++b) s += (double)part[(size_t)b * (MLP_NPARAM + 1) + p];
-    grad[p] = s;
+// grad[p] = sum over the block slots of part[slot][p] in float64; p = MLP_NPARAM is the loss.  64 columns
+// per block, 16 threads a column that take every 16th slot, added in order: 9 us for 256 slots (one thread a column over the 2,048 slots that
+// 32 samples a block left: 500 us).
+constexpr int MLP_RED_G = 16;
+__global__ void __launch_bounds__(64 * MLP_RED_G) k_mlp_reduce(const float *part, int nslot, double *grad) {
+    __shared__ double s[MLP_RED_G][64];
+    const int c = threadIdx.x & 63, g = threadIdx.x >> 6, p = blockIdx.x * 64 + c;
+    double v = 0.0;
+    if (p <= MLP_NPARAM)
+        for (int b = g; b < nslot; b += MLP_RED_G) v += (double)part[(size_t)b * (MLP_NPARAM + 1) + p];
+    s[g][c] = v;
+    __syncthreads();
+    if (g == 0 && p <= MLP_NPARAM) {
+        for (int k = 1; k < MLP_RED_G; ++k) v += s[k][c];
+        grad[p] = v;
+    }
 }
 
 struct AdamArgs {

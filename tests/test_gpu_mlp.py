@@ -50,6 +50,32 @@ def test_features_match_oracle(ctx):
     mlp.close()
 
 
+@pytest.mark.parametrize("B", [1, 15, 16, 17, 63, 65, 1000, 16384, 16389, 40000])
+def test_grad_tile_edges(ctx, B):
+    """The training kernel takes 16 samples a wave, 64 a block and walks the blocks over larger
+    minibatches: gradient and loss at the edges of each, repeated samples included.  The bound is the
+    float32 sums' (2^-24 times the square root of the terms) and one bfloat16 neighbour in a layer input
+    of the few samples whose float32 activation rounds the other way."""
+    print(f"[gpu mlp] gradient, {B} samples", flush=True)
+    rng = np.random.default_rng(B)
+    th = (M.init_params(2) + rng.normal(scale=0.05, size=M.NPARAM)).astype(np.float32).astype(np.float64)
+    S = max(B // 2, 3)
+    X = rng.normal(size=(S, 12)).astype(np.float32)
+    T = (0.5 * rng.normal(size=(S, 2))).astype(np.float32)
+    idx = rng.integers(0, S, size=B).astype(np.int32)
+    mlp = ctx.mlp(th)
+    ptrs = [upload(ctx, v) for v in (X, T, idx)]
+    loss, g = mlp.grad(*ptrs, B)
+    lo, go = M.loss_and_grad(th, X[idx].astype(np.float64), T[idx].astype(np.float64))
+    assert abs(loss - lo) <= 1e-4 * lo
+    assert np.linalg.norm(g - go) <= 1e-3 * np.linalg.norm(go)
+    again, g2 = mlp.grad(*ptrs, B)
+    assert again == loss and np.array_equal(g, g2)
+    for p in ptrs:
+        ctx.free(p)
+    mlp.close()
+
+
 def test_grad_and_inference_match_oracle(ctx):
     print("[gpu mlp] gradient / inference", flush=True)
     rng = np.random.default_rng(1)
