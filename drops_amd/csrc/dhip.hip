@@ -1916,13 +1916,11 @@ int dhip_tune(dhip_ctx_t *c, const char *key, int64_t value) {
     }
     if (!std::strcmp(key, "batch_split")) {
         if (value != 0 && value != 1) return set_error(c, DHIP_E_ARG, "batch_split must be 0 or 1");
-        c->batch_split = (int)value;
         return DHIP_OK;
     }
     if (!std::strcmp(key, "batch_solve_threads")) {
         if (value != 256 && value != 512 && value != 1024)
             return set_error(c, DHIP_E_ARG, "batch_solve_threads must be 256, 512 or 1024");
-        c->batch_solve_threads = (int)value;
         return DHIP_OK;
     }
     if (!std::strcmp(key, "batch_prepass")) {
@@ -3023,8 +3021,7 @@ struct dhip_batch {
     int32_t max_cells = 0;
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
-    int g_threads = 0, g_grid = 0, g_max_iter = 0, g_rel = 0, g_prepass = -1, g_split = -1, g_sthreads = 0;
-    int64_t g_lds = 0;
+    int g_threads = 0, g_grid = 0, g_max_iter = 0, g_rel = 0, g_prepass = -1;
     double g_tol = 0.0;
 };
 
@@ -3046,26 +3043,13 @@ static const void *batch_kernel(int threads) {
                           : threads == 512 ? (const void *)k_batch<512> : (const void *)k_batch<256>;
 }
 
-static const void *batch_solve_kernel(int threads) {
-    return threads == 1024 ? (const void *)k_batch_solve<1024>
-                           : threads == 512 ? (const void *)k_batch_solve<512> : (const void *)k_batch_solve<256>;
-}
-
-// Dynamic LDS (the search direction) and grid of a per-problem batch kernel at a residency of
-// `per_cu_want` workgroups per CU.
-static int batch_launch_shape(dhip_ctx *c, const void *k, int threads, int per_cu_want, int32_t nprob, int64_t *lds,
+// Grid of a per-problem batch kernel at a residency of at most `per_cu_want` workgroups per CU.
+static int batch_launch_shape(dhip_ctx *c, const void *k, int threads, int per_cu_want, int32_t nprob, int64_t lds,
                               int *grid) {
-    int maxs = 0;
-    hipFuncAttributes fa{};
-    DHIP_HIPCHK(c, hipDeviceGetAttribute(&maxs, hipDeviceAttributeMaxSharedMemoryPerMultiprocessor, c->device));
-    DHIP_HIPCHK(c, hipFuncGetAttributes(&fa, k));
-    int64_t l = ((int64_t)maxs / per_cu_want - (int64_t)fa.sharedSizeBytes - 1024) & ~(int64_t)255;
-    l = std::max<int64_t>(0, std::min<int64_t>(l, 128 * 1024));
-    if (l > 64 * 1024) DHIP_HIPCHK(c, hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)l));
+    if (lds > 0) DHIP_HIPCHK(c, hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     int per_cu = 0;
-    DHIP_HIPCHK(c, hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k, threads, (size_t)l));
+    DHIP_HIPCHK(c, hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k, threads, (size_t)lds));
     if (per_cu < 1) return set_error(c, DHIP_E_HIP, "batched kernel cannot be resident");
-    *lds = l;
     *grid = (int)std::min<int64_t>(nprob, (int64_t)c->cu_count * std::min(per_cu, per_cu_want));
     return DHIP_OK;
 }
@@ -3161,7 +3145,7 @@ int dhip_batch_create(dhip_ctx_t *c, int32_t nprob, const dhip_batch_problem_t *
         cut_tot += P.ncut_cap;
         row_tot += P.row_cap;
         nz_tot += P.nz_cap;
-        sell_tot += 15 * 64 * ((P.row_cap + 63) / 64);
+        sell_tot += BP_W * (64 * ((P.row_cap + 63) / 64) + (P.row_cap > 8 * BPT ? BPT : 0));   // + a padding slot
         slice_tot += (P.row_cap + 63) / 64 + 1;
         if (P.nz_cap >= ((int64_t)1 << 31)) return fail(set_error(c, DHIP_E_CAPACITY, "problem %d too large", i));
     }
@@ -3277,22 +3261,12 @@ int dhip_batch_solve(dhip_batch_t *b, int32_t max_iter, double tol, int32_t rel,
     DHIP_HIPCHK(c, hipSetDevice(c->device));
     const int threads = c->batch_threads;
     const void *k = batch_kernel(threads);
-    // dynamic LDS for the search direction: what the requested residency leaves of the CU's LDS
-    int64_t lds = 0;
-    int grid = 0;
-    int rc = batch_launch_shape(c, k, threads, c->batch_blocks_per_cu, b->nprob, &lds, &grid);
+    int grid = 0, sgrid = 0;
+    int rc = batch_launch_shape(c, k, threads, c->batch_blocks_per_cu, b->nprob, 0, &grid);
     if (rc) return rc;
-    const int split = c->batch_split;
-    const int sthreads = c->batch_solve_threads;
-    const void *ks = batch_solve_kernel(sthreads);
-    int64_t slds = 0;
-    int sgrid = 0;
-    if (split) {
-        rc = batch_launch_shape(c, ks, sthreads, 1, b->nprob, &slds, &sgrid);
-        if (rc) return rc;
-    }
-    b->args.split = split;
-    b->args.lds_floats = (split ? slds : lds) / 4;
+    const void *ks = (const void *)k_batch_solve;
+    rc = batch_launch_shape(c, ks, BPT, 1, b->nprob, BP_LDS, &sgrid);
+    if (rc) return rc;
     b->args.max_iter = max_iter;
     b->args.tol = tol;
     b->args.rel = rel;
@@ -3316,17 +3290,16 @@ int dhip_batch_solve(dhip_batch_t *b, int32_t max_iter, double tol, int32_t rel,
         }
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
-        e = hipLaunchKernel(k, dim3(grid), dim3(threads), argv, split ? 0 : (size_t)lds, c->stream);
-        if (e != hipSuccess || !split) return e;
-        return hipLaunchKernel(ks, dim3(sgrid), dim3(sthreads), argv, (size_t)slds, c->stream);
+        e = hipLaunchKernel(k, dim3(grid), dim3(threads), argv, 0, c->stream);
+        if (e != hipSuccess) return e;
+        return hipLaunchKernel(ks, dim3(sgrid), dim3(BPT), argv, (size_t)BP_LDS, c->stream);
     };
     if (!use_graph) {
         ProfScope ps(c, "batch");
         DHIP_HIPCHK(c, enqueue());
     } else {
         const bool same = b->exec && b->g_threads == threads && b->g_grid == grid && b->g_max_iter == max_iter &&
-                          b->g_tol == tol && b->g_rel == rel && b->g_lds == lds && b->g_prepass == a.prepass &&
-                          b->g_split == split && b->g_sthreads == sthreads;
+                          b->g_tol == tol && b->g_rel == rel && b->g_prepass == a.prepass;
         if (!same) {
             if (b->exec) (void)hipGraphExecDestroy(b->exec);
             if (b->graph) (void)hipGraphDestroy(b->graph);
@@ -3345,10 +3318,7 @@ int dhip_batch_solve(dhip_batch_t *b, int32_t max_iter, double tol, int32_t rel,
             b->g_max_iter = max_iter;
             b->g_tol = tol;
             b->g_rel = rel;
-            b->g_lds = lds;
             b->g_prepass = a.prepass;
-            b->g_split = split;
-            b->g_sthreads = sthreads;
         }
         ProfScope ps(c, "batch_graph");
         DHIP_HIPCHK(c, hipGraphLaunch(b->exec, c->stream));

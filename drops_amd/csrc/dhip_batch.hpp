@@ -1,9 +1,9 @@
 // dhip_batch.hpp -- many independent P1 trace-FEM problems assembled and solved in one launch.
 //
 // Each problem has its own Kuhn brick, level set and sizes.  One workgroup owns one problem at a
-// time and runs the whole path for it with workgroup barriers only (no grid synchronisation):
-// classification + compaction, local matrices, first-encounter numbering, CSR rows, and a Jacobi
-// PCG with FP32 inner iterations and FP64 refinement.  Workgroups take problems from a queue
+// time with workgroup barriers only (no grid synchronisation): classification + compaction, local
+// matrices, first-encounter numbering and CSR rows, and in a second launch a Jacobi PCG with FP32
+// inner iterations and FP64 refinement.  Workgroups take problems from a queue
 // ordered largest first (longest-processing-time order), so uneven sizes balance over the grid.
 // The per-item code is the single-problem path's (cell_cut_mask, local_p1_one, qualify_one,
 // first_one, rowcount_one, rowfill_one), so every assembled array equals what the single-problem
@@ -12,11 +12,8 @@
 //   k_batch_cells / k_batch_verts   planning: cut tets and cut-tet vertices per problem (sizes of
 //                                   the per-problem scratch; the rows of a problem are at most its
 //                                   cut-tet vertices, each row has at most 15 entries)
-//   k_batch<BB>                     the persistent solve, BB threads per problem
-//   k_batch_solve<BB>               with the tuning key batch_split: k_batch stops after assembly and
-//                                   this second launch runs the PCGs, BB (up to 1024) threads per
-//                                   problem, largest first; the solve is bandwidth-bound per problem,
-//                                   so more threads than the assembly's workgroup shorten the span
+//   k_batch<BB>                     assembly, BB threads per problem
+//   k_batch_solve                   the PCGs, one problem per CU at a time, largest first
 #pragma once
 
 #include "dhip_assembly.hpp"
@@ -35,7 +32,7 @@ struct BatchProb {
     int64_t nz_off;     // first entry slot (capacity nz_cap)
     int64_t nz_cap;
     double lc[3];       // the solved operator combination
-    int64_t sell_off;   // first SELL-64 slot (capacity 15 * 64 * ceil(row_cap / 64))
+    int64_t sell_off;   // first SELL-64 slot (capacity 16 * 64 * ceil(row_cap / 64) + 16 * BPT)
     int64_t slice_off;  // first slice offset (capacity ceil(row_cap / 64) + 1)
 };
 
@@ -218,9 +215,8 @@ struct BatchArgs {
     double *vm, *vl, *vs, *vc;
     double *rhs, *diag, *x, *r64;
     float *d32, *r32, *z32, *p32, *q32;
-    int32_t *scol, *soff;       // SELL-64 copy of the FP32 inner matrix
+    int32_t *scol, *soff;       // FP32 inner matrix in memory: streamed rows, or a SELL-64 copy of the whole
     float *sval;
-    int64_t lds_floats;         // dynamic LDS of the launch: the search direction when it fits
     BatchStat *stat;
     double coef0, coef1, coef2;
     int rhs_kind;
@@ -233,7 +229,6 @@ struct BatchArgs {
     double inner_tol;
     int inner_max;
     int prepass = 0;            // 1: cut lists, cell words, flags and local data come from the pre-pass
-    int split = 0;              // 1: k_batch assembles only, k_batch_solve runs the PCGs
     const int32_t *pre_zero = nullptr, *pre_err = nullptr;
 };
 
@@ -308,13 +303,9 @@ __device__ __forceinline__ double sell_spmv_group(const int32_t *soff, const int
     return p_lam;
 }
 
+// Assembly of problem p; its stat entry carries the sizes and the status to k_batch_solve.
 template <int BB>
-__device__ void batch_pcg(const BatchArgs &a, int p, float *lds_p, BatchStat &st);
-
-// Assembly of problem p, then (solve) its PCG; without solve the stat entry records the assembly
-// and k_batch_solve runs the PCG.
-template <int BB>
-__device__ void batch_problem(const BatchArgs &a, int p, float *lds_p, bool solve) {
+__device__ void batch_problem(const BatchArgs &a, int p) {
     __shared__ int sh_zero, sh_err;   // workgroup flags (LDS: no stale cache lines)
     const BatchProb P = a.prob[p];
     const MeshP m = P.m;
@@ -328,9 +319,7 @@ __device__ void batch_problem(const BatchArgs &a, int p, float *lds_p, bool solv
     int32_t *rowowner = a.rowowner + P.row_off, *rowlen = a.rowlen + P.row_off, *rowptr = a.rowptr + P.row_off + p;
     int32_t *col = a.col + P.nz_off;
     double *vm = a.vm + P.nz_off, *vl = a.vl + P.nz_off, *vs = a.vs + P.nz_off, *vc = a.vc + P.nz_off;
-    double *rhs = a.rhs + P.row_off, *diag = a.diag + P.row_off, *x = a.x + P.row_off, *r64 = a.r64 + P.row_off;
-    float *d32 = a.d32 + P.row_off, *r32 = a.r32 + P.row_off, *z32 = a.z32 + P.row_off;
-    float *p32 = a.p32 + P.row_off, *q32 = a.q32 + P.row_off;
+    double *rhs = a.rhs + P.row_off, *diag = a.diag + P.row_off;
     BatchStat st{};
     st.t0 = wall_clock64();
     st.status = DHIP_OK;
@@ -420,46 +409,19 @@ __device__ void batch_problem(const BatchArgs &a, int p, float *lds_p, bool solv
     if (st.status == DHIP_OK) {
         RowArgs ra{m, cut, ncut, cellinfo, flags, dofs, rowowner, nd, loc, rowlen, rowptr, col,
                    vm, vl, vs, vc, rhs, diag, P.lc[0], P.lc[1], P.lc[2]};
-        for (int64_t r = tid; r < nd; r += BB) {
-            rowfill_one(ra, r);
-            x[r] = 0.0;
-        }
-        __syncthreads();
-        // SELL-64 copy of the FP32 matrix: entry k of row r at soff[r / 64] + 64 k + r % 64, so the
-        // thread-per-row loads of a wave (64 consecutive rows) coalesce
-        int32_t *scol = a.scol + P.sell_off, *soff = a.soff + P.slice_off;
-        float *sval = a.sval + P.sell_off;
-        const int64_t nsl = (nd + 63) / 64;
-        for (int64_t sl = tid; sl < nsl; sl += BB) {
-            int32_t w = 0;
-            for (int64_t r = 64 * sl; r < 64 * sl + 64 && r < nd; ++r) {
-                const int32_t len = rowptr[r + 1] - rowptr[r];
-                w = len > w ? len : w;
-            }
-            soff[sl] = 64 * w;
-        }
-        __syncthreads();
-        wg_scan_inplace<BB>(soff, nsl);
-        for (int64_t r = tid; r < nd; r += BB) {
-            const int64_t base = (int64_t)soff[r >> 6] + (r & 63);
-            for (int32_t e = rowptr[r], k = 0; e < rowptr[r + 1]; ++e, ++k) {
-                scol[base + 64 * (int64_t)k] = col[e];
-                sval[base + 64 * (int64_t)k] = (float)vc[e];
-            }
-        }
+        for (int64_t r = tid; r < nd; r += BB) rowfill_one(ra, r);
         __syncthreads();
         st.t_asm = wall_clock64();
-        if (solve) batch_pcg<BB>(a, p, lds_p, st);
     }
     st.t1 = wall_clock64();
     if (tid == 0) a.stat[p] = st;
     __syncthreads();
 }
 
-// Jacobi PCG of an assembled problem: FP64 residual and refinement, FP32 inner iterations on the
-// SELL-64 copy; st receives iterations, residual and status.
+// The same PCG for a problem whose search direction does not fit the workgroup's LDS: every vector in
+// memory, the inner matrix as a SELL-64 copy.
 template <int BB>
-__device__ void batch_pcg(const BatchArgs &a, int p, float *lds_p, BatchStat &st) {
+__device__ __noinline__ void batch_pcg_memory(const BatchArgs &a, int p, BatchStat &st) {
     const BatchProb P = a.prob[p];
     const int tid = threadIdx.x;
     const int64_t nd = st.ndof;
@@ -470,11 +432,32 @@ __device__ void batch_pcg(const BatchArgs &a, int p, float *lds_p, BatchStat &st
     double *x = a.x + P.row_off, *r64 = a.r64 + P.row_off;
     float *d32 = a.d32 + P.row_off, *r32 = a.r32 + P.row_off, *z32 = a.z32 + P.row_off;
     float *p32 = a.p32 + P.row_off, *q32 = a.q32 + P.row_off;
-    const int32_t *scol = a.scol + P.sell_off, *soff = a.soff + P.slice_off;
-    const float *sval = a.sval + P.sell_off;
+    // SELL-64 copy of the FP32 matrix: entry k of row r at soff[r / 64] + 64 k + r % 64, so the
+    // thread-per-row loads of a wave (64 consecutive rows) coalesce
+    int32_t *scol = a.scol + P.sell_off, *soff = a.soff + P.slice_off;
+    float *sval = a.sval + P.sell_off;
+    const int64_t nsl = (nd + 63) / 64;
+    for (int64_t sl = tid; sl < nsl; sl += BB) {
+        int32_t w = 0;
+        for (int64_t r = 64 * sl; r < 64 * sl + 64 && r < nd; ++r) {
+            const int32_t len = rowptr[r + 1] - rowptr[r];
+            w = len > w ? len : w;
+        }
+        soff[sl] = 64 * w;
+    }
+    __syncthreads();
+    wg_scan_inplace<BB>(soff, nsl);
+    for (int64_t r = tid; r < nd; r += BB) {
+        const int64_t base = (int64_t)soff[r >> 6] + (r & 63);
+        for (int32_t e = rowptr[r], k = 0; e < rowptr[r + 1]; ++e, ++k) {
+            scol[base + 64 * (int64_t)k] = col[e];
+            sval[base + 64 * (int64_t)k] = (float)vc[e];
+        }
+    }
+    __syncthreads();
+    for (int64_t r = tid; r < nd; r += BB) x[r] = 0.0;
+    __syncthreads();
     {
-
-        // ---- Jacobi PCG: FP64 residual and refinement, FP32 inner iterations ----
         int total_it = 0, outer = 0, status = 1;
         double normb = 1.0, resid = 0.0;
         bool firstpass = true;
@@ -482,7 +465,7 @@ __device__ void batch_pcg(const BatchArgs &a, int p, float *lds_p, BatchStat &st
             double p_rr = 0.0, p_bb = 0.0;
             for (int64_t r = tid; r < nd; r += BB) {
                 const double s =
-                    row_product<double, (BB >= 1024 ? 8 : MAXR)>(rowptr, col, vc, 0, r, [&](int32_t c) { return x[c]; });
+                    row_product<double, 8>(rowptr, col, vc, 0, r, [&](int32_t c) { return x[c]; });
                 const double bv = rhs[r];
                 const double rv = bv - s;
                 r64[r] = rv;
@@ -502,8 +485,7 @@ __device__ void batch_pcg(const BatchArgs &a, int p, float *lds_p, BatchStat &st
             if (total_it >= a.max_iter) { status = 1; break; }
             ++outer;
             const double scale = 1.0 / rnorm;
-            // the search direction lives in LDS when the problem fits (the SpMV gathers read it)
-            float *pv = nd <= a.lds_floats ? lds_p : p32;
+            float *pv = p32;
             double p_zr = 0.0;
             for (int64_t r = tid; r < nd; r += BB) {
                 const float rin = (float)(r64[r] * scale);
@@ -518,7 +500,7 @@ __device__ void batch_pcg(const BatchArgs &a, int p, float *lds_p, BatchStat &st
             float beta = 0.0f;
             for (int it = 1; it <= a.inner_max && total_it < a.max_iter; ++it) {
                 ++total_it;
-                constexpr int GU = BB >= 1024 ? 4 : 8;   // rows per group of the vector loops
+                constexpr int GU = 4;   // rows per group of the vector loops
                 for (int64_t r0 = tid; r0 < nd; r0 += (int64_t)GU * BB) {
                     float zl[GU], pl[GU];
 #pragma unroll
@@ -537,7 +519,7 @@ __device__ void batch_pcg(const BatchArgs &a, int p, float *lds_p, BatchStat &st
                 }
                 __syncthreads();
                 const double lam =
-                    block_sum<BB>(sell_spmv_group<BB, (BB >= 1024 ? 1 : 4)>(soff, scol, sval, rowptr, pv, q32, nd));
+                    block_sum<BB>(sell_spmv_group<BB, 2>(soff, scol, sval, rowptr, pv, q32, nd));
                 const float alpha = (float)(rho / lam);
                 double p_rr2 = 0.0, p_zr2 = 0.0;
                 for (int64_t r0 = tid; r0 < nd; r0 += (int64_t)GU * BB) {
@@ -584,9 +566,457 @@ __device__ void batch_pcg(const BatchArgs &a, int p, float *lds_p, BatchStat &st
     }
 }
 
+// ---------------------------------------------------------------------------
+// the PCG of a problem inside one CU
+//
+// One workgroup of BPT threads runs a problem's Jacobi PCG with FP32 inner iterations and FP64
+// refinement (residuals, dot products and the solution in FP64).  What an inner iteration touches stays
+// on the CU: the search direction in LDS, and of thread t's rows t, t + BPT, ... the first R with their
+// matrix entries (16 values, 16 column indices of 16 bits) and their vectors in registers, the next L with
+// their entries in LDS.  The rows of larger problems beyond these are streamed each iteration from a copy laid
+// out for their own thread (four values and four columns a load, 96 B a row); S rows a thread of those keep
+// their vectors in registers, and past 19 rows a thread (MEM) the vectors are streamed too.  The classes are
+// what 256 registers hold without spilling.
+// An iteration is three barriers, two workgroup sums and the LDS gathers of the search direction (about 7
+// cycles a wave's 64 against 2 without bank conflicts).  Measured a row count's iteration with 200 problems at
+// once: 765 rows 1.9 us, 1,543 2.5, 2,471 3.4, 3,555 4.7, 4,682 9.7, 7,604 13.7, 9,372 20, 12,936 30; with
+// every vector and the matrix in memory 15 to 60 us.  512 problems of 16^3 to 64^3 cells: all PCGs 70 -> 18.5 ms.
+// ---------------------------------------------------------------------------
+constexpr int BPT = 512;
+constexpr int BPW = BPT / 64;
+constexpr int BP_W = 16, BP_Q = BP_W / 4;   // entries per row (a P1 interface row has at most 15), in quads
+constexpr int BP_G = 4;               // streamed rows whose vector loads are issued together
+constexpr int BP_MAX_SLOTS = 76;      // rows per thread: 76 * 512 floats of search direction fit the LDS
+struct BpShared {
+    double red[2][BPW][2];
+    uint8_t quads[BP_MAX_SLOTS * BPW];
+    __align__(16) unsigned char end[16];
+};
+
+// bytes of LDS: the search direction of `slots` rows a thread, and l rows' entries
+constexpr int64_t bp_lds(int64_t slots, int l) {
+    return (int64_t)sizeof(BpShared) + slots * BPT * 4 + (int64_t)l * BP_Q * BPT * 24;
+}
+
+// dynamic LDS of k_batch_solve: its largest class, on a CU of 160 KiB
+constexpr int64_t BP_LDS = bp_lds(BP_MAX_SLOTS, 0) > bp_lds(28, 2) ? bp_lds(BP_MAX_SLOTS, 0) : bp_lds(28, 2);
+static_assert(BP_LDS + 2048 <= 160 * 1024, "k_batch_solve's LDS");
+
+// sum over the wave in lane 63 (row shifts, then the row broadcasts)
+template <int CTRL, int ROWS>
+__device__ __forceinline__ double dpp_add(double v) {
+    const uint64_t b = __builtin_bit_cast(uint64_t, v);
+    const int lo = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)b, CTRL, ROWS, 0xf, true);
+    const int hi = __builtin_amdgcn_update_dpp(0, (int)(uint32_t)(b >> 32), CTRL, ROWS, 0xf, true);
+    return v + __builtin_bit_cast(double, ((uint64_t)(uint32_t)hi << 32) | (uint32_t)lo);
+}
+__device__ __forceinline__ double wave_sum_last(double v) {
+    v = dpp_add<0x111, 0xf>(v);
+    v = dpp_add<0x112, 0xf>(v);
+    v = dpp_add<0x114, 0xf>(v);
+    v = dpp_add<0x118, 0xf>(v);
+    v = dpp_add<0x142, 0xa>(v);
+    return dpp_add<0x143, 0xc>(v);
+}
+
+// Workgroup sums of u and v in every thread: the eight waves' sums go through LDS once, every lane takes one
+// of them and the lanes add up in a fixed pattern.  One barrier: successive calls use the two halves of `red`
+// in turn, and a half is written again only after the other half's barrier.
+__device__ __forceinline__ void bp_sum2(double (*red)[2], double &u, double &v) {
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    u = wave_sum_last(u);
+    v = wave_sum_last(v);
+    if (lane == 63) {
+        red[w][0] = u;
+        red[w][1] = v;
+    }
+    __syncthreads();
+    u = red[lane & 7][0];
+    v = red[lane & 7][1];
+    u = dpp_add<0xB1, 0xf>(u);    // lane ^ 1
+    v = dpp_add<0xB1, 0xf>(v);
+    u = dpp_add<0x4E, 0xf>(u);    // lane ^ 2
+    v = dpp_add<0x4E, 0xf>(v);
+    u = dpp_add<0x141, 0xf>(u);   // the other half of the eight
+    v = dpp_add<0x141, 0xf>(v);
+}
+static_assert(BPW == 8, "bp_sum2 adds eight waves");
+
+// u / v for positive normal v, to a rounding of FP64 (the quotient is used as FP32)
+__device__ __forceinline__ double bp_quot(double u, double v) {
+    double r = __builtin_amdgcn_rcp(v);
+    r = __builtin_fma(__builtin_fma(-v, r, 1.0), r, r);
+    r = __builtin_fma(__builtin_fma(-v, r, 1.0), r, r);
+    return u * r;
+}
+
+// Global pointers of a called function: without the address space the loads would be flat ones, which wait
+// for every load in flight.
+template <class T>
+using GlobalPtr = __attribute__((address_space(1))) T *;
+typedef float BpF4 __attribute__((ext_vector_type(4)));
+typedef uint32_t BpU2 __attribute__((ext_vector_type(2)));
+
+// A row's FP32 entries and columns, four at a time; entries past the row's end are (0, column 0).  Every load
+// is issued (an index past the row's end is clamped to it), so that a row's loads overlap.
+struct BpQuad {
+    BpF4 v;
+    BpU2 c;
+};
+__device__ __forceinline__ BpQuad bp_load_quad(GlobalPtr<const int32_t> col, GlobalPtr<const double> vc, int32_t e,
+                                               int32_t end) {
+    double v[4];
+    uint32_t cc[4];
+    const int32_t last = end > 0 ? end - 1 : 0;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        const int32_t i = e + k < last ? e + k : last;
+        v[k] = vc[i];
+        cc[k] = (uint32_t)col[i];
+    }
+    BpQuad q;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        const bool in = e + k < end;
+        q.v[k] = in ? (float)v[k] : 0.0f;
+        cc[k] = in ? cc[k] : 0u;
+    }
+    q.c[0] = cc[0] | cc[1] << 16;
+    q.c[1] = cc[2] | cc[3] << 16;
+    return q;
+}
+__device__ __forceinline__ float bp_quad_dot(float s, const BpF4 &v, const BpU2 &c, const float *pv) {
+    s = __builtin_fmaf(v[0], pv[c[0] & 0xffffu], s);
+    s = __builtin_fmaf(v[1], pv[c[0] >> 16], s);
+    s = __builtin_fmaf(v[2], pv[c[1] & 0xffffu], s);
+    return __builtin_fmaf(v[3], pv[c[1] >> 16], s);
+}
+// (A x)_r in FP64, in column order
+__device__ __forceinline__ double bp_row64(GlobalPtr<const int32_t> col, GlobalPtr<const double> vc, int32_t e,
+                                           int32_t end, GlobalPtr<const double> x) {
+    constexpr int B = 8;
+    double s = 0.0;
+    for (; e < end; e += B) {
+        double v[B], xx[B];
+        int32_t cc[B];
+#pragma unroll
+        for (int k = 0; k < B; ++k) {
+            const int32_t i = e + k < end ? e + k : end - 1;
+            cc[k] = col[i];
+            v[k] = vc[i];
+        }
+#pragma unroll
+        for (int k = 0; k < B; ++k) xx[k] = x[cc[k]];
+#pragma unroll
+        for (int k = 0; k < B; ++k)
+            if (e + k < end) s += v[k] * xx[k];
+    }
+    return s;
+}
+
+// the widest row of the wave's 64, in quads (uniform)
+__device__ __forceinline__ int bp_wave_quads(int len) {
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+        const int t = __shfl_xor(len, o, 64);
+        len = t > len ? t : len;
+    }
+    return __builtin_amdgcn_readfirstlane((len + 3) >> 2);
+}
+
+template <int R, int L, int S, bool MEM>
+__device__ __noinline__ void batch_pcg_chip(const BatchArgs &a, int p, BatchStat &st) {
+    extern __shared__ __align__(16) unsigned char lds[];
+    BpShared &sh = *reinterpret_cast<BpShared *>(lds);
+    float *pv = reinterpret_cast<float *>(lds + sizeof(BpShared));
+    double (*red)[BPW][2] = sh.red;
+    uint8_t *quads = sh.quads;
+    constexpr int V0 = R + L;   // rows per thread whose entries are on the CU
+    constexpr int V = V0 + S;   // rows per thread whose vectors are in registers
+    const double inner_tol2 = a.inner_tol * a.inner_tol;
+    const BatchProb &P = a.prob[p];
+    int tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));   // nothing of one size's code is formed ahead of the queue loop
+    const int wv = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+    const int nd = st.ndof;
+    const int slots = MEM ? (nd + BPT - 1) / BPT : V;
+    const auto rowptr = (GlobalPtr<const int32_t>)(a.rowptr + P.row_off + p);
+    const auto col = (GlobalPtr<const int32_t>)(a.col + P.nz_off);
+    const auto vc = (GlobalPtr<const double>)(a.vc + P.nz_off);
+    const auto rhs = (GlobalPtr<const double>)(a.rhs + P.row_off);
+    const auto diag = (GlobalPtr<const double>)(a.diag + P.row_off);
+    const auto x = (GlobalPtr<double>)(a.x + P.row_off);
+    const auto r64 = (GlobalPtr<double>)(a.r64 + P.row_off);
+    // streamed rows: entries as four floats / four uint16 per (slice, quad, lane); MEM: the vectors too (z32
+    // holds the inverse diagonal)
+    const auto d32 = (GlobalPtr<float>)(a.d32 + P.row_off), r32 = (GlobalPtr<float>)(a.r32 + P.row_off);
+    const auto z32 = (GlobalPtr<float>)(a.z32 + P.row_off), q32 = (GlobalPtr<float>)(a.q32 + P.row_off);
+    const auto sv = (GlobalPtr<BpF4>)(a.sval + P.sell_off);
+    const auto sc = (GlobalPtr<BpU2>)(a.scol + P.sell_off);
+    // LDS rows: the same quads behind the search direction
+    BpF4 *lv = reinterpret_cast<BpF4 *>(pv + slots * BPT);
+    BpU2 *lc = reinterpret_cast<BpU2 *>(lv + L * BP_Q * BPT);
+
+    // entries of the LDS and streamed rows, once per problem
+    for (int u = R; u < slots; ++u) {
+        const int r = tid + u * BPT;
+        int32_t e = 0, end = 0;
+        if (r < nd) {
+            e = rowptr[r];
+            end = rowptr[r + 1];
+            if (MEM && u >= V) z32[r] = 1.0f / (float)diag[r];
+        }
+        const int w = bp_wave_quads(end - e);
+        if (lane == 0) quads[u * BPW + wv] = (uint8_t)w;
+        for (int q = 0; q < (S > 0 || MEM ? BP_Q : w); ++q) {   // (streamed rows are loaded whole, padding included)
+            const BpQuad b = bp_load_quad(col, vc, e + 4 * q, end);
+            const BpF4 bv = b.v;
+            const BpU2 bc = b.c;
+            if (u < V0) {
+                lv[((u - R) * BP_Q + q) * BPT + tid] = bv;
+                lc[((u - R) * BP_Q + q) * BPT + tid] = bc;
+            } else {
+                const int64_t at = (int64_t)(((u - V0) * BPW + wv) * BP_Q + q) * 64 + lane;
+                sv[at] = bv;
+                sc[at] = bc;
+            }
+        }
+    }
+    int total_it = 0, outer = 0, status = 1;
+    double normb = 1.0, resid = 0.0;
+    bool firstpass = true;
+    for (;;) {
+        // ---- FP64 residual (the start is x = 0: b itself) ----
+        double p_rr = 0.0, p_bb = 0.0;
+        for (int r = tid; r < nd; r += BPT) {
+            const double bv = rhs[r];
+            double rv = bv;
+            if (firstpass) {
+                x[r] = 0.0;
+                p_bb += bv * bv;
+            } else {
+                rv = bv - bp_row64(col, vc, rowptr[r], rowptr[r + 1], x);
+            }
+            r64[r] = rv;
+            p_rr += rv * rv;
+        }
+        bp_sum2(red[0], p_rr, p_bb);
+        if (firstpass) {
+            normb = sqrt(p_bb);
+            if (normb == 0.0 || !a.rel) normb = 1.0;
+            firstpass = false;
+        }
+        const double rnorm = sqrt(p_rr);
+        resid = rnorm / normb;
+        if (resid <= a.tol) { status = 0; break; }
+        if (total_it >= a.max_iter) { status = 1; break; }
+        ++outer;
+        const double scale = 1.0 / rnorm;
+        // ---- the register rows' entries and vectors ----
+        BpF4 val[R][BP_Q];
+        BpU2 cc[R][BP_Q];
+        float rv[V], dv[V], di[V], qv[V];
+        int wq[V];
+        double p_zr = 0.0, unused = 0.0;
+        int t0 = tid;
+        asm volatile("" : "+v"(t0));   // (row addresses are formed here, not kept over the iterations)
+#pragma unroll
+        for (int u = 0; u < V; ++u) {
+            const int r = t0 + u * BPT;
+            int32_t e = 0, end = 0;
+            rv[u] = dv[u] = di[u] = 0.0f;
+            if (r < nd) {
+                e = rowptr[r];
+                end = rowptr[r + 1];
+                rv[u] = (float)(r64[r] * scale);
+                di[u] = 1.0f / (float)diag[r];
+            }
+            wq[u] = bp_wave_quads(end - e);
+            if (u < R) {
+#pragma unroll
+                for (int q = 0; q < BP_Q; ++q) {
+                    const BpQuad b = bp_load_quad(col, vc, e + 4 * q, end);
+                    val[u < R ? u : 0][q] = b.v;
+                    cc[u < R ? u : 0][q] = b.c;
+                    if (R >= 4 && (q & 1)) __builtin_amdgcn_sched_barrier(0);   // (two quads' FP64 loads in flight)
+                }
+            }
+            pv[r] = 0.0f;
+            p_zr += (double)(rv[u] * di[u]) * (double)rv[u];
+        }
+        for (int u = V; MEM && u < slots; ++u) {
+            const int r = tid + u * BPT;
+            pv[r] = 0.0f;
+            if (r < nd) {
+                const float rin = (float)(r64[r] * scale);
+                r32[r] = rin;
+                d32[r] = 0.0f;
+                p_zr += (double)(rin * z32[r]) * (double)rin;
+            }
+        }
+        bp_sum2(red[1], p_zr, unused);
+        double rho = p_zr;
+        float beta = 0.0f;
+        for (int it = 1; it <= a.inner_max && total_it < a.max_iter; ++it) {
+            ++total_it;
+            // p = z + beta p
+#pragma unroll
+            for (int u = 0; u < V; ++u) {
+                const int r = tid + u * BPT;
+                pv[r] = __builtin_fmaf(beta, pv[r], rv[u] * di[u]);
+                if (V > 8 && u % 8 == 7) __builtin_amdgcn_sched_barrier(0);
+            }
+            for (int u0 = V; MEM && u0 < slots; u0 += BP_G) {
+                float rl[BP_G], zl[BP_G];
+#pragma unroll
+                for (int k = 0; k < BP_G; ++k) {
+                    const int r = tid + (u0 + k) * BPT;
+                    rl[k] = zl[k] = 0.0f;
+                    if (r < nd) {
+                        rl[k] = r32[r];
+                        zl[k] = z32[r];
+                    }
+                }
+#pragma unroll
+                for (int k = 0; k < BP_G; ++k) {
+                    const int r = tid + (u0 + k) * BPT;
+                    if (r < nd) pv[r] = __builtin_fmaf(beta, pv[r], rl[k] * zl[k]);
+                }
+            }
+            __syncthreads();
+            // q = A p, (p, q)
+            double lam = 0.0, none = 0.0;
+            // The streamed rows' entries are PF rows ahead of the sums.  Their loads stand under no condition:
+            // across a branch the compiler could only wait for all loads in flight.
+            constexpr int PF = S >= 16 ? 1 : 2;
+            BpF4 nv[PF][BP_Q];
+            BpU2 nc[PF][BP_Q];
+            auto fetch = [&](int u, BpF4 (&v)[BP_Q], BpU2 (&c)[BP_Q]) {
+                const int64_t at = (int64_t)((u - V0) * BPW + wv) * BP_Q * 64 + lane;
+#pragma unroll
+                for (int q = 0; q < BP_Q; ++q) {
+                    v[q] = sv[at + q * 64];
+                    c[q] = sc[at + q * 64];
+                }
+            };
+#pragma unroll
+            for (int k = 0; k < PF; ++k)
+                if (k < S || (MEM && k == 0)) fetch(V0 + k, nv[k], nc[k]);
+#pragma unroll
+            for (int u = 0; u < R; ++u) {
+                // the columns stay packed: unpacked out of the loop they would take 8 more registers a row
+#pragma unroll
+                for (int q = 0; q < BP_Q; ++q) asm volatile("" : "+v"(cc[u][q]));
+                float s = 0.0f;
+#pragma unroll
+                for (int q = 0; q < BP_Q; ++q)
+                    if (q < wq[u]) s = bp_quad_dot(s, val[u][q], cc[u][q], pv);
+                qv[u] = s;
+                lam += (double)s * (double)pv[tid + u * BPT];
+            }
+#pragma unroll
+            for (int l = 0; l < L; ++l) {
+                float s = 0.0f;
+#pragma unroll
+                for (int q = 0; q < BP_Q; ++q)
+                    if (q < wq[R + l]) s = bp_quad_dot(s, lv[(l * BP_Q + q) * BPT + tid], lc[(l * BP_Q + q) * BPT + tid], pv);
+                qv[R + l] = s;
+                lam += (double)s * (double)pv[tid + (R + l) * BPT];
+            }
+#pragma unroll
+            for (int k = 0; k < S; ++k) {
+                const int u = V0 + k;
+                float s = 0.0f;
+#pragma unroll
+                for (int q = 0; q < BP_Q; ++q)
+                    if (q < wq[u]) s = bp_quad_dot(s, nv[k % PF][q], nc[k % PF][q], pv);
+                if (k + PF < S) fetch(u + PF, nv[k % PF], nc[k % PF]);
+                qv[u] = s;
+                lam += (double)s * (double)pv[tid + u * BPT];
+                __builtin_amdgcn_sched_barrier(0);   // PF rows in registers, no more
+            }
+            for (int u = V; MEM && u < slots; ++u) {
+                const int r = tid + u * BPT;
+                const int w = __builtin_amdgcn_readfirstlane((int)quads[u * BPW + wv]);
+                BpF4 v[BP_Q];
+                BpU2 c[BP_Q];
+#pragma unroll
+                for (int q = 0; q < BP_Q; ++q) {
+                    v[q] = nv[0][q];
+                    c[q] = nc[0][q];
+                }
+                fetch(u + 1 < slots ? u + 1 : u, nv[0], nc[0]);
+                float s = 0.0f;
+#pragma unroll
+                for (int q = 0; q < BP_Q; ++q)
+                    if (q < w) s = bp_quad_dot(s, v[q], c[q], pv);
+                if (r < nd) q32[r] = s;
+                lam += (double)s * (double)pv[r];
+            }
+            bp_sum2(red[0], lam, none);
+            const float alpha = (float)bp_quot(rho, lam);
+            double p_rr2 = 0.0, p_zr2 = 0.0;
+#pragma unroll
+            for (int u = 0; u < V; ++u) {
+                dv[u] = __builtin_fmaf(alpha, pv[tid + u * BPT], dv[u]);
+                const float rin = __builtin_fmaf(-alpha, qv[u], rv[u]);
+                rv[u] = rin;
+                p_rr2 += (double)rin * (double)rin;
+                p_zr2 += (double)(rin * di[u]) * (double)rin;
+            }
+            for (int u0 = V; MEM && u0 < slots; u0 += BP_G) {
+                float dl[BP_G], rl[BP_G], ql[BP_G], zl[BP_G];
+#pragma unroll
+                for (int k = 0; k < BP_G; ++k) {
+                    const int r = tid + (u0 + k) * BPT;
+                    dl[k] = rl[k] = ql[k] = zl[k] = 0.0f;
+                    if (r < nd) {
+                        dl[k] = d32[r];
+                        rl[k] = r32[r];
+                        ql[k] = q32[r];
+                        zl[k] = z32[r];
+                    }
+                }
+#pragma unroll
+                for (int k = 0; k < BP_G; ++k) {
+                    const int r = tid + (u0 + k) * BPT;
+                    if (r < nd) {
+                        d32[r] = __builtin_fmaf(alpha, pv[r], dl[k]);
+                        const float rin = __builtin_fmaf(-alpha, ql[k], rl[k]);
+                        r32[r] = rin;
+                        p_rr2 += (double)rin * (double)rin;
+                        p_zr2 += (double)(rin * zl[k]) * (double)rin;
+                    }
+                }
+            }
+            bp_sum2(red[1], p_rr2, p_zr2);
+            if (p_rr2 <= inner_tol2) break;
+            const double rho1 = rho;
+            rho = p_zr2;
+            beta = (float)bp_quot(rho, rho1);
+        }
+        int t1 = tid;
+        asm volatile("" : "+v"(t1));
+#pragma unroll
+        for (int u = 0; u < V; ++u) {
+            const int r = t1 + u * BPT;
+            if (r < nd) x[r] += rnorm * (double)dv[u];
+            if (V > 8 && u % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+        }
+        for (int u = V; MEM && u < slots; ++u) {
+            const int r = tid + u * BPT;
+            if (r < nd) x[r] += rnorm * (double)d32[r];
+        }
+        __syncthreads();
+    }
+    st.iters = total_it;
+    st.outer = outer;
+    st.resid = resid;
+    st.status = status == 0 ? DHIP_OK : DHIP_E_NOT_CONVERGED;
+}
+
 template <int BB>
 __global__ void __launch_bounds__(BB) k_batch(BatchArgs a) {
-    extern __shared__ __align__(16) unsigned char lds[];
     __shared__ int sh_p;
     for (;;) {
         if (threadIdx.x == 0) {
@@ -597,15 +1027,12 @@ __global__ void __launch_bounds__(BB) k_batch(BatchArgs a) {
         const int p = sh_p;
         __syncthreads();
         if (p < 0) break;
-        batch_problem<BB>(a, p, reinterpret_cast<float *>(lds), !a.split);
+        batch_problem<BB>(a, p);
     }
 }
 
-// The PCG of every assembled problem (split mode): problems from the second queue counter in the
-// same largest-first order, BB threads each.
-template <int BB>
-__global__ void __launch_bounds__(BB) k_batch_solve(BatchArgs a) {
-    extern __shared__ __align__(16) unsigned char lds[];
+// The PCG of every assembled problem: problems from the second queue counter, largest first.
+__global__ void __launch_bounds__(BPT) k_batch_solve(BatchArgs a) {
     __shared__ int sh_p;
     for (;;) {
         if (threadIdx.x == 0) {
@@ -618,7 +1045,28 @@ __global__ void __launch_bounds__(BB) k_batch_solve(BatchArgs a) {
         if (p < 0) break;
         BatchStat st = a.stat[p];
         if (st.status == DHIP_OK) {
-            batch_pcg<BB>(a, p, reinterpret_cast<float *>(lds), st);
+            const int slots = (st.ndof + BPT - 1) / BPT;
+            // the smallest size class that holds the problem; the LDS of the classes up to 27 slots fits (asserted)
+            switch (slots) {
+                case 0: case 1: batch_pcg_chip<1, 0, 0, false>(a, p, st); break;
+                case 2: batch_pcg_chip<2, 0, 0, false>(a, p, st); break;
+                case 3: batch_pcg_chip<3, 0, 0, false>(a, p, st); break;
+                case 4: batch_pcg_chip<4, 0, 0, false>(a, p, st); break;
+                case 5: batch_pcg_chip<5, 0, 0, false>(a, p, st); break;
+                case 6: batch_pcg_chip<6, 0, 0, false>(a, p, st); break;
+                case 7: batch_pcg_chip<5, 2, 0, false>(a, p, st); break;
+                case 8: batch_pcg_chip<6, 2, 0, false>(a, p, st); break;
+                case 9: batch_pcg_chip<3, 2, 4, false>(a, p, st); break;
+                case 10: case 11: batch_pcg_chip<2, 2, 7, false>(a, p, st); break;
+                case 12: case 13: batch_pcg_chip<2, 2, 9, false>(a, p, st); break;
+                case 14: case 15: batch_pcg_chip<1, 2, 12, false>(a, p, st); break;
+                case 16: case 17: batch_pcg_chip<1, 2, 14, false>(a, p, st); break;
+                case 18: case 19: batch_pcg_chip<1, 2, 16, false>(a, p, st); break;
+                default:
+                    if (slots <= 28) batch_pcg_chip<4, 2, 0, true>(a, p, st);
+                    else if (slots <= BP_MAX_SLOTS) batch_pcg_chip<4, 0, 0, true>(a, p, st);
+                    else batch_pcg_memory<BPT>(a, p, st);
+            }
             st.t1 = wall_clock64();
             if (threadIdx.x == 0) a.stat[p] = st;
         }

@@ -170,8 +170,6 @@ struct dhip_ctx {
     int batch_blocks_per_cu = 2;      // resident workgroups per CU of the batched solve
     int xcd_map = 1;                  // persistent solvers: each XCD's blocks own one contiguous run of rows
     int coherent_exchange = 2;        // persistent solvers' exchange: 0 fenced, 1 coherent atomics, 2 tagged records (FP64 PCG)
-    int batch_split = 0;              // batched solve: assembly launch, then a separate PCG launch
-    int batch_solve_threads = 1024;   // threads per problem of the separate PCG launch
     int batch_prepass = 0;            // batched solve: classification and local matrices over the whole grid first
     bool coop_refused = false;        // cooperative launch unavailable: same grid, regular launch
     int probe_blocks = 0;

@@ -502,16 +502,14 @@ typedef struct {
 int dhip_batch_create(dhip_ctx_t *ctx, int32_t nprob, const dhip_batch_problem_t *probs, const double *phi,
                       int64_t phi_count, int32_t where, int32_t zero_policy, const double coef[3],
                       int32_t rhs_kind, const double *rhs_param, double omit_bound, dhip_batch_t **batch);
-/* Assembles and solves every problem in one persistent launch (relative residual tol, at most
- * max_iter inner iterations per problem).  use_graph: capture the launch into a hipGraph on the
- * first call and replay it while the arguments stay the same.  Workgroup size and residency come
- * from dhip_tune("batch_threads" 128/256/512, "batch_blocks_per_cu" 1..8); "batch_prepass" 1 runs
- * classification, compaction and local matrices of all problems over the whole grid before the
- * per-problem launch (same results; 0, the default, does them inside each problem's workgroup).
- * "batch_split" 1 ends the per-problem launch after assembly and runs the PCGs in a second
- * launch with "batch_solve_threads" (256/512/1024, default 1024) threads per problem, largest
- * first (bit-identical to the single launch when both use the same number of threads; with
- * another number the reductions add their partial sums in another order). */
+/* Assembles and solves every problem (relative residual tol, at most max_iter inner iterations per
+ * problem): one launch that assembles, one workgroup per problem, and one that runs the PCGs, one
+ * problem per CU at a time, largest first.  use_graph: capture the launches into a hipGraph on the
+ * first call and replay it while the arguments stay the same.  The assembly's workgroup size and
+ * residency come from dhip_tune("batch_threads" 128/256/512, "batch_blocks_per_cu" 1..8);
+ * "batch_prepass" 1 runs classification, compaction and local matrices of all problems over the
+ * whole grid before it (same results; 0 is the default).  The PCG has one geometry: the keys
+ * "batch_split" and "batch_solve_threads" are accepted and change nothing. */
 int dhip_batch_solve(dhip_batch_t *batch, int32_t max_iter, double tol, int32_t rel, int32_t use_graph);
 /* per-problem results of the last solve (nprob entries) */
 int dhip_batch_stats(dhip_batch_t *batch, dhip_batch_stat_t *stats);

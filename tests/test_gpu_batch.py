@@ -148,3 +148,42 @@ def test_batch_zero_node_problem_isolated(ctx):
     with pytest.raises(D.DhipError):
         b.problem(len(meshes) - 1)
     b.close()
+
+
+# rows per problem from 1 to 27 per thread of the solver's 512, beyond its register classes and beyond its LDS:
+# (cells across, radius) of spheres, about 1.86 (radius n)^2 rows
+CLASS_SIZES = [(16, 1.0), (22, 1.0), (27, 1.0), (31, 1.0), (35, 1.0), (39, 1.0), (43, 1.0), (46, 1.0), (49, 1.0),
+               (53, 1.0), (58, 1.0), (63, 1.0), (67, 1.0), (71, 1.0), (80, 1.0), (64, 1.5), (80, 1.9)]
+
+
+def test_batch_size_classes(ctx):
+    """One problem of every size class of the batched PCG, alone and together: the system of
+    dhip_assemble_p1 bit for bit, a true residual within the tolerance (1.5: the FP64 residual is summed in
+    another order here), replays bit-identical."""
+    print("[gpu batch] size classes", flush=True)
+    meshes = [KuhnMesh.box(-2.0, 2.0, n, shift=tuple(4e-3 / n * np.array([1.0, 2.0, 3.0]))) for n, _ in CLASS_SIZES]
+    phis = [m.sample_p2(sphere(radius=r)) for m, (_, r) in zip(meshes, CLASS_SIZES)]
+    off = np.concatenate([[0], np.cumsum([p.size for p in phis])[:-1]]).astype(np.int64)
+    b = make_batch(ctx, meshes, np.concatenate([p.ravel() for p in phis]), off)
+    b.solve(tol=1e-8)
+    st = b.stats()
+    assert np.all(st["status"] == D.OK)
+    slots = -(-st["ndof"] // 512)
+    assert {1, 2, 3, 4, 5, 6, 7, 8, 9} <= set(slots.tolist()) and slots.max() > 76 and 28 < np.sort(slots)[-2] <= 76
+    first = []
+    for p, m in enumerate(meshes):
+        g = b.problem(p)
+        first.append(g["x"])
+        ctx.mesh(m)
+        ctx.levelset(phis[p])
+        ctx.assemble_p1(coef=COEF, rhs_kind=D.RHS_3XY_MINUS_X3, lc=lc_of(m))
+        ref = ctx.csr()
+        for k in ("rowptr", "colind", "comb", "rhs"):
+            assert np.array_equal(g[k], ref[k]), (p, k)
+        A = sp.csr_matrix((g["comb"], g["colind"], g["rowptr"]))
+        assert np.linalg.norm(g["rhs"] - A @ g["x"]) <= 1.5e-8 * np.linalg.norm(g["rhs"]), (p, slots[p])
+    for graph in (False, True, True):
+        b.solve(tol=1e-8, graph=graph)
+        for p in range(len(meshes)):
+            assert np.array_equal(b.problem(p)["x"], first[p]), p
+    b.close()
