@@ -1911,7 +1911,6 @@ int dhip_tune(dhip_ctx_t *c, const char *key, int64_t value) {
     if (!std::strcmp(key, "batch_threads")) {
         if (value != 128 && value != 256 && value != 512)
             return set_error(c, DHIP_E_ARG, "batch_threads must be 128, 256 or 512");
-        c->batch_threads = (int)value;
         return DHIP_OK;
     }
     if (!std::strcmp(key, "batch_split")) {
@@ -1925,12 +1924,10 @@ int dhip_tune(dhip_ctx_t *c, const char *key, int64_t value) {
     }
     if (!std::strcmp(key, "batch_prepass")) {
         if (value != 0 && value != 1) return set_error(c, DHIP_E_ARG, "batch_prepass must be 0 or 1");
-        c->batch_prepass = (int)value;
         return DHIP_OK;
     }
     if (!std::strcmp(key, "batch_blocks_per_cu")) {
         if (value < 1 || value > 8) return set_error(c, DHIP_E_ARG, "batch_blocks_per_cu must be 1..8");
-        c->batch_blocks_per_cu = (int)value;
         return DHIP_OK;
     }
     return set_error(c, DHIP_E_ARG, "unknown tuning key %s", key);
@@ -3017,11 +3014,9 @@ struct dhip_batch {
     DevBuf vm, vl, vs, vc, rhs, diag, x, r64, d32, r32, z32, p32, q32, scol, sval, soff, stat;
     DevBuf pre_mask, pre_blk, pre_flag;   // pre-pass: cell masks, block counts, zero / error flags
     BatchArgs args{};
-    PrepassArgs pre{};
-    int32_t max_cells = 0;
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
-    int g_threads = 0, g_grid = 0, g_max_iter = 0, g_rel = 0, g_prepass = -1;
+    int g_max_iter = 0, g_rel = 0;
     double g_tol = 0.0;
 };
 
@@ -3036,22 +3031,6 @@ static void batch_release(dhip_batch *b) {
                       &b->z32, &b->p32, &b->q32, &b->scol, &b->sval, &b->soff, &b->stat, &b->pre_mask,
                       &b->pre_blk, &b->pre_flag};
     for (DevBuf *d : bufs) d->release();
-}
-
-static const void *batch_kernel(int threads) {
-    return threads == 128 ? (const void *)k_batch<128>
-                          : threads == 512 ? (const void *)k_batch<512> : (const void *)k_batch<256>;
-}
-
-// Grid of a per-problem batch kernel at a residency of at most `per_cu_want` workgroups per CU.
-static int batch_launch_shape(dhip_ctx *c, const void *k, int threads, int per_cu_want, int32_t nprob, int64_t lds,
-                              int *grid) {
-    if (lds > 0) DHIP_HIPCHK(c, hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    int per_cu = 0;
-    DHIP_HIPCHK(c, hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k, threads, (size_t)lds));
-    if (per_cu < 1) return set_error(c, DHIP_E_HIP, "batched kernel cannot be resident");
-    *grid = (int)std::min<int64_t>(nprob, (int64_t)c->cu_count * std::min(per_cu, per_cu_want));
-    return DHIP_OK;
 }
 
 extern "C" {
@@ -3221,28 +3200,13 @@ int dhip_batch_create(dhip_ctx_t *c, int32_t nprob, const dhip_batch_problem_t *
     a.zero_throw = zero_policy == DHIP_ZERO_THROW;
     a.inner_tol = 1e-4;
     a.inner_max = 400;
-    a.pre_zero = b->pre_flag.as<int32_t>();
-    a.pre_err = a.pre_zero + nprob;
-    PrepassArgs &q = b->pre;
-    q.prob = a.prob;
-    q.nprob = nprob;
-    q.phi = dphi;
-    q.cellmask = b->pre_mask.as<uint8_t>();
-    q.blkcnt = b->pre_blk.as<int32_t>();
-    q.max_blocks = (int32_t)blocks_for(max_cells, BPLAN);
-    q.zero = b->pre_flag.as<int32_t>();
-    q.perr = q.zero + nprob;
-    q.cellinfo = a.cellinfo;
-    q.cut = a.cut;
-    q.cut_total = cut_tot;
-    q.flags = a.flags;
-    q.loc = a.loc;
-    q.coef0 = a.coef0;
-    q.coef1 = a.coef1;
-    q.coef2 = a.coef2;
-    q.rhs_kind = a.rhs_kind;
-    q.rhs_p0 = a.rhs_p0;
-    b->max_cells = (int32_t)max_cells;
+    a.cellmask = b->pre_mask.as<uint8_t>();
+    a.blkcnt = b->pre_blk.as<int32_t>();
+    a.max_blocks = (int32_t)blocks_for(max_cells, BPLAN);
+    a.zero = b->pre_flag.as<int32_t>();
+    a.perr = a.zero + nprob;
+    a.cut_total = cut_tot;
+    a.row_total = row_tot;
     *out = b;
     return DHIP_OK;
 }
@@ -3259,47 +3223,39 @@ int dhip_batch_solve(dhip_batch_t *b, int32_t max_iter, double tol, int32_t rel,
     if (!b || max_iter < 1 || !(tol > 0.0)) return DHIP_E_ARG;
     dhip_ctx *c = b->ctx;
     DHIP_HIPCHK(c, hipSetDevice(c->device));
-    const int threads = c->batch_threads;
-    const void *k = batch_kernel(threads);
-    int grid = 0, sgrid = 0;
-    int rc = batch_launch_shape(c, k, threads, c->batch_blocks_per_cu, b->nprob, 0, &grid);
-    if (rc) return rc;
-    const void *ks = (const void *)k_batch_solve;
-    rc = batch_launch_shape(c, ks, BPT, 1, b->nprob, BP_LDS, &sgrid);
-    if (rc) return rc;
     b->args.max_iter = max_iter;
     b->args.tol = tol;
     b->args.rel = rel;
-    b->args.prepass = c->batch_prepass;
-    BatchArgs a = b->args;
-    void *argv[] = {&a};
-    const PrepassArgs q = b->pre;
+    const BatchArgs a = b->args;
+    DHIP_HIPCHK(c, hipFuncSetAttribute((const void *)k_batch_solve, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                       (int)BP_LDS));
     auto enqueue = [&]() -> hipError_t {
-        hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(64), 0, c->stream, b->queue.as<uint32_t>(), 16);
-        if (a.prepass) {
-            const int nflag = 2 * b->nprob;
-            hipLaunchKernelGGL(k_zero_u32, dim3(blocks_for(nflag, 256)), dim3(256), 0, c->stream,
-                               b->pre_flag.as<uint32_t>(), nflag);
-            const dim3 g2(q.max_blocks, b->nprob);
-            hipLaunchKernelGGL(k_batch_cut_count, g2, dim3(BPLAN), 0, c->stream, q);
-            hipLaunchKernelGGL(k_batch_cut_scan, dim3(b->nprob), dim3(BPLAN), 0, c->stream, q);
-            hipLaunchKernelGGL(k_batch_cut_fill, g2, dim3(BPLAN), 0, c->stream, q);
-            if (q.cut_total > 0)
-                hipLaunchKernelGGL(k_batch_local, dim3(blocks_for(q.cut_total, LOCAL_BLOCK)), dim3(LOCAL_BLOCK), 0,
-                                   c->stream, q);
+        hipStream_t s = c->stream;
+        const int nflag = 2 * b->nprob;
+        const dim3 cells(a.max_blocks, b->nprob);
+        hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(64), 0, s, b->queue.as<uint32_t>(), 16);
+        hipLaunchKernelGGL(k_zero_u32, dim3(blocks_for(nflag, 256)), dim3(256), 0, s, b->pre_flag.as<uint32_t>(), nflag);
+        hipLaunchKernelGGL(k_batch_cut_count, cells, dim3(BPLAN), 0, s, a);
+        hipLaunchKernelGGL(k_batch_cut_scan, dim3(b->nprob), dim3(BSCAN), 0, s, a);
+        hipLaunchKernelGGL(k_batch_cut_fill, cells, dim3(BPLAN), 0, s, a);
+        if (a.cut_total > 0) {
+            const dim3 slots(blocks_for(4 * a.cut_total, BFLAT)), rows(blocks_for(a.row_total, ROWW_WAVES));
+            hipLaunchKernelGGL(k_batch_local, dim3(blocks_for(a.cut_total, LOCAL_BLOCK)), dim3(LOCAL_BLOCK), 0, s, a);
+            hipLaunchKernelGGL(k_batch_first, slots, dim3(BFLAT), 0, s, a);
+            hipLaunchKernelGGL(k_batch_rank, dim3(b->nprob), dim3(BSCAN), 0, s, a);
+            hipLaunchKernelGGL(k_batch_dofs, slots, dim3(BFLAT), 0, s, a);
+            hipLaunchKernelGGL(k_batch_rows<false>, rows, dim3(64 * ROWW_WAVES), 0, s, a);
+            hipLaunchKernelGGL(k_batch_rowptr, dim3(b->nprob), dim3(BSCAN), 0, s, a);
+            hipLaunchKernelGGL(k_batch_rows<true>, rows, dim3(64 * ROWW_WAVES), 0, s, a);
         }
-        hipError_t e = hipGetLastError();
-        if (e != hipSuccess) return e;
-        e = hipLaunchKernel(k, dim3(grid), dim3(threads), argv, 0, c->stream);
-        if (e != hipSuccess) return e;
-        return hipLaunchKernel(ks, dim3(sgrid), dim3(BPT), argv, (size_t)BP_LDS, c->stream);
+        hipLaunchKernelGGL(k_batch_solve, dim3(std::min(b->nprob, c->cu_count)), dim3(BPT), (size_t)BP_LDS, s, a);
+        return hipGetLastError();
     };
     if (!use_graph) {
         ProfScope ps(c, "batch");
         DHIP_HIPCHK(c, enqueue());
     } else {
-        const bool same = b->exec && b->g_threads == threads && b->g_grid == grid && b->g_max_iter == max_iter &&
-                          b->g_tol == tol && b->g_rel == rel && b->g_prepass == a.prepass;
+        const bool same = b->exec && b->g_max_iter == max_iter && b->g_tol == tol && b->g_rel == rel;
         if (!same) {
             if (b->exec) (void)hipGraphExecDestroy(b->exec);
             if (b->graph) (void)hipGraphDestroy(b->graph);
@@ -3313,12 +3269,9 @@ int dhip_batch_solve(dhip_batch_t *b, int32_t max_iter, double tol, int32_t rel,
             DHIP_HIPCHK(c, e2);
             b->graph = g;
             DHIP_HIPCHK(c, hipGraphInstantiate(&b->exec, g, nullptr, nullptr, 0));
-            b->g_threads = threads;
-            b->g_grid = grid;
             b->g_max_iter = max_iter;
             b->g_tol = tol;
             b->g_rel = rel;
-            b->g_prepass = a.prepass;
         }
         ProfScope ps(c, "batch_graph");
         DHIP_HIPCHK(c, hipGraphLaunch(b->exec, c->stream));

@@ -19,8 +19,7 @@
 //                vertex in ascending tet id, loads their local entries together
 //                and sums them in that order (the order of the reference's
 //                hash-map +=), ranks the <= 15 columns and writes CSR rows, comb
-//                values and rhs.  rowcount_one / rowfill_one are the same rows
-//                for one lane each (the batched kernel's workgroup loops).
+//                values and rhs.
 // Compiled with -ffp-contract=off: every product and sum is rounded as in the
 // reference's evaluation order.
 #pragma once
@@ -784,80 +783,11 @@ struct RowArgs {
     double lc0, lc1, lc2;
 };
 
-__device__ inline void rowcount_one(const RowArgs &a, int64_t r) {
-    int64_t x1, x2, x3;
-    slot_vertex(a.m, a.cut, a.rowowner[r], x1, x2, x3);
-    uint32_t present = 0;
-    for_incident_cut_tets(a.m, a.cellinfo, x1, x2, x3, [&](int64_t ci, int k, int li) {
-        if (!(a.flags[ci] & 1)) return false;
-        for (int j = 0; j < 4; ++j)
-            if (a.dofs[ci * 4 + j] >= 0) present |= 1u << c_tab.slot[k][li][j];
-        return false;
-    });
-    a.rowlen[r] = __popc(present);
-}
-
-__device__ inline void rowfill_one(const RowArgs &a, int64_t r) {
-    int64_t x1, x2, x3;
-    slot_vertex(a.m, a.cut, a.rowowner[r], x1, x2, x3);
-    uint32_t present = 0;
-    int32_t cols[15];
-    double am[15], al[15], as[15];
-#pragma unroll
-    for (int s = 0; s < 15; ++s) {
-        cols[s] = 0;
-        am[s] = al[s] = as[s] = 0.0;
-    }
-    double rh = 0.0;
-    const int64_t N = a.ncut;
-    for_incident_cut_tets(a.m, a.cellinfo, x1, x2, x3, [&](int64_t ci, int k, int li) {
-        if (!(a.flags[ci] & 1)) return false;
-        for (int j = 0; j < 4; ++j) {
-            const int32_t dj = a.dofs[ci * 4 + j];
-            if (dj < 0) continue;
-            const int sl = c_tab.slot[k][li][j];
-            const int e = li * 4 + j;
-            const double m = a.loc[(int64_t)(LOC_MASS + e) * N + ci];
-            const double l = a.loc[(int64_t)(LOC_LB + e) * N + ci];
-            const double st = a.loc[(int64_t)(LOC_STAB + e) * N + ci];
-#pragma unroll
-            for (int s = 0; s < 15; ++s)
-                if (s == sl) {
-                    cols[s] = dj;
-                    am[s] += m;
-                    al[s] += l;
-                    as[s] += st;
-                }
-            present |= 1u << sl;
-        }
-        rh += a.loc[(int64_t)(LOC_RHS + li) * N + ci];
-        return false;
-    });
-    const int64_t base = a.rowptr[r];
-#pragma unroll
-    for (int s = 0; s < 15; ++s) {
-        if (!((present >> s) & 1u)) continue;
-        int rank = 0;
-#pragma unroll
-        for (int u = 0; u < 15; ++u)
-            rank += (((present >> u) & 1u) && cols[u] < cols[s]) ? 1 : 0;
-        const int64_t dst = base + rank;
-        a.col[dst] = cols[s];
-        a.vm[dst] = am[s];
-        a.vl[dst] = al[s];
-        a.vs[dst] = as[s];
-        const double cv = 1.0 * (a.lc0 * am[s] + a.lc1 * al[s]) + a.lc2 * as[s];
-        a.vc[dst] = cv;
-        if (cols[s] == r) a.diag[r] = cv;
-    }
-    a.rhs[r] = rh;
-}
-
-// One row per wave (rowcount_one / rowfill_one's rows with the tets' loads side by side): lanes 0-47 look at
+// One row per wave: lanes 0-47 look at
 // the (cell, Kuhn tet) candidates of the row vertex at once, lane order being for_incident_cut_tets' walk
 // order (d = 7 .. 0, then k), and list the flagged cut tets; sixteen tets at a time, lane 4 t + j loads
 // column vertex j of tet t, and the sums into the 15 neighbour slots go tet by tet, so every slot is summed
-// in walk order as rowfill_one sums it.
+// in walk order (the order of the reference's row map).
 constexpr int ROWW_WAVES = 4;
 
 struct RowWShared {
@@ -874,13 +804,8 @@ __device__ __forceinline__ void wave_sync_lds() {
 }
 
 template <bool FILL>
-__global__ void __launch_bounds__(64 * ROWW_WAVES) k_rows_w(RowArgs a) {
-    __shared__ RowWShared shm[ROWW_WAVES];
-    const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    // each XCD takes a contiguous run of rows, whose tets its L2 then shares
-    const int64_t r = (int64_t)xcd_position(blockIdx.x, gridDim.x) * ROWW_WAVES + w;
-    if (r >= a.ndof) return;
-    RowWShared &sh = shm[w];
+__device__ __forceinline__ void row_wave(const RowArgs &a, int64_t r, RowWShared &sh) {
+    const int lane = threadIdx.x & 63;
     if (lane < 16) {
         sh.pres[lane] = 0;
         sh.cols[lane] = 0;
@@ -975,6 +900,16 @@ __global__ void __launch_bounds__(64 * ROWW_WAVES) k_rows_w(RowArgs a) {
         if (cs == r) a.diag[r] = cv;
     }
     if (lane == 0) a.rhs[r] = rh;
+}
+
+template <bool FILL>
+__global__ void __launch_bounds__(64 * ROWW_WAVES) k_rows_w(RowArgs a) {
+    __shared__ RowWShared shm[ROWW_WAVES];
+    const int w = threadIdx.x >> 6;
+    // each XCD takes a contiguous run of rows, whose tets its L2 then shares
+    const int64_t r = (int64_t)xcd_position(blockIdx.x, gridDim.x) * ROWW_WAVES + w;
+    if (r >= a.ndof) return;
+    row_wave<FILL>(a, r, shm[w]);
 }
 
 }  // namespace dhip

@@ -1,18 +1,16 @@
 // dhip_batch.hpp -- many independent P1 trace-FEM problems assembled and solved in one launch.
 //
-// Each problem has its own Kuhn brick, level set and sizes.  One workgroup owns one problem at a
-// time with workgroup barriers only (no grid synchronisation): classification + compaction, local
-// matrices, first-encounter numbering and CSR rows, and in a second launch a Jacobi PCG with FP32
-// inner iterations and FP64 refinement.  Workgroups take problems from a queue
-// ordered largest first (longest-processing-time order), so uneven sizes balance over the grid.
-// The per-item code is the single-problem path's (cell_cut_mask, local_p1_one, qualify_one,
-// first_one, rowcount_one, rowfill_one), so every assembled array equals what the single-problem
-// entry points produce.
+// Each problem has its own Kuhn brick, level set and sizes.  The assembly runs step by step over all
+// problems at once with the single-problem path's per-item code (cell_cut_mask, local_p1_one, qualify_one,
+// first_one, row_wave), so every assembled array equals what the single-problem entry points produce.
+// Then one workgroup owns one problem at a time and runs a Jacobi PCG with FP32 inner iterations and FP64
+// refinement, with workgroup barriers only; workgroups take problems from a queue ordered largest first
+// (longest-processing-time order), so uneven sizes balance over the grid.
 //
 //   k_batch_cells / k_batch_verts   planning: cut tets and cut-tet vertices per problem (sizes of
 //                                   the per-problem scratch; the rows of a problem are at most its
 //                                   cut-tet vertices, each row has at most 15 entries)
-//   k_batch<BB>                     assembly, BB threads per problem
+//   k_batch_cut_count .. k_batch_rows   assembly, every step over all problems
 //   k_batch_solve                   the PCGs, one problem per CU at a time, largest first
 #pragma once
 
@@ -89,115 +87,25 @@ __global__ void __launch_bounds__(BPLAN) k_batch_verts(const BatchProb *prob, co
     if (threadIdx.x == 0 && cnt > 0.0) atomicAdd(&nvert[blockIdx.y], (int32_t)cnt);
 }
 
-// exclusive scan of a[0..n) in place by the whole workgroup; returns the total
-template <int BB>
-__device__ inline int64_t wg_scan_inplace(int32_t *a, int64_t n) {
-    int64_t carry = 0;
-    for (int64_t i0 = 0; i0 < n; i0 += BB) {
-        const int64_t i = i0 + threadIdx.x;
-        const int v = i < n ? a[i] : 0;
-        int tot;
-        const int off = block_excl_scan<BB>(v, &tot);
-        if (i < n) a[i] = (int32_t)(carry + off);
-        carry += tot;
-    }
-    __syncthreads();
-    return carry;
-}
-
 // ---------------------------------------------------------------------------
-// pre-pass (tuning key batch_prepass): classification, compaction and local matrices of every
-// problem over the whole grid, so that a large problem's most expensive per-tet work does not
-// lengthen its workgroup's span.  The same per-item functions produce the same arrays as the
-// in-kernel path.  The largest problem's assembly leaves its span, but every problem then enters its
-// solve at once and the solves slow down; which effect wins differs between runs, so the autotuner
-// decides per problem set.
+// assembly over the whole grid
+//
+// Every step of the single-problem assembly as one launch over all problems: a problem's workgroup had
+// to walk its own steps one after the other, the largest one for 8 ms while the others had long ended, and
+// kept the local matrices' and the rows' registers in one kernel (1,272 bytes of scratch a lane).  The same
+// per-item functions produce the same arrays as the single-problem entry points.
 //   k_batch_cut_count   per (problem, block of cells): cell masks, the block's cut-tet count,
 //                       the problem's exact-zero flag
-//   k_batch_cut_scan    per problem: exclusive scan of its block counts
+//   k_batch_cut_scan    per problem: exclusive scan of its block counts; opens its stat entry
 //   k_batch_cut_fill    per (problem, block of cells): cut list in cell order and cell words
-//   k_batch_local       one thread per cut tet of any problem: local_p1_one
-// ---------------------------------------------------------------------------
-struct PrepassArgs {
-    const BatchProb *prob;
-    int32_t nprob;
-    const double *phi;
-    uint8_t *cellmask;          // per problem cell (cell_off layout)
-    int32_t *blkcnt;            // [nprob][max_blocks]
-    int32_t max_blocks;
-    int32_t *zero;              // per problem: exact-zero node in a cut tet
-    int32_t *perr;              // per problem: local error bits (2: all-zero sub-tet)
-    uint32_t *cellinfo;
-    int64_t *cut;
-    int64_t cut_total;
-    uint8_t *flags;
-    double *loc;
-    double coef0, coef1, coef2;
-    int rhs_kind;
-    double rhs_p0;
-};
-
-__global__ void __launch_bounds__(BPLAN) k_batch_cut_count(PrepassArgs a) {
-    const int p = blockIdx.y;
-    const BatchProb &P = a.prob[p];
-    const int64_t cell = (int64_t)blockIdx.x * BPLAN + threadIdx.x;
-    int mk = 0;
-    bool z = false;
-    if (cell < P.m.ncell) {
-        mk = cell_cut_mask(P.m, a.phi + P.phi_off, cell, z);
-        a.cellmask[P.cell_off + cell] = (uint8_t)mk;
-    }
-    int tot;
-    block_excl_scan<BPLAN>(__popc(mk), &tot);
-    const double zs = block_sum<BPLAN>(z ? 1.0 : 0.0);
-    if (threadIdx.x == 0) {
-        a.blkcnt[(int64_t)p * a.max_blocks + blockIdx.x] = tot;
-        if (zs > 0.0) atomicOr(&a.zero[p], 1);
-    }
-}
-
-__global__ void __launch_bounds__(BPLAN) k_batch_cut_scan(PrepassArgs a) {
-    const int p = blockIdx.x;
-    const int64_t nb = (a.prob[p].m.ncell + BPLAN - 1) / BPLAN;
-    wg_scan_inplace<BPLAN>(a.blkcnt + (int64_t)p * a.max_blocks, nb);
-}
-
-__global__ void __launch_bounds__(BPLAN) k_batch_cut_fill(PrepassArgs a) {
-    const int p = blockIdx.y;
-    const BatchProb &P = a.prob[p];
-    const int64_t cell = (int64_t)blockIdx.x * BPLAN + threadIdx.x;
-    const int mk = cell < P.m.ncell ? a.cellmask[P.cell_off + cell] : 0;
-    const int off = block_excl_scan<BPLAN>(__popc(mk), nullptr);
-    if (cell >= P.m.ncell) return;
-    int64_t b = (int64_t)a.blkcnt[(int64_t)p * a.max_blocks + blockIdx.x] + off;
-    a.cellinfo[P.cell_off + cell] = ((uint32_t)b << 6) | (uint32_t)mk;
-    for (int k = 0; k < 6; ++k)
-        if (mk & (1 << k)) {
-            if (b < P.ncut_cap) a.cut[P.cut_off + b] = cell * 6 + k;
-            ++b;
-        }
-}
-
-__global__ void __launch_bounds__(LOCAL_BLOCK) k_batch_local(PrepassArgs a) {
-    const int64_t g = (int64_t)blockIdx.x * LOCAL_BLOCK + threadIdx.x;
-    if (g >= a.cut_total) return;
-    // the problem whose cut slots hold g: the last one with cut_off <= g
-    int lo = 0, hi = a.nprob - 1;
-    while (lo < hi) {
-        const int mid = (lo + hi + 1) >> 1;
-        if (a.prob[mid].cut_off <= g) lo = mid;
-        else hi = mid - 1;
-    }
-    const BatchProb &P = a.prob[lo];
-    const int64_t c = g - P.cut_off;
-    if (c < 0 || c >= P.ncut_cap) return;
-    LocalArgs la{P.m, a.phi + P.phi_off, a.cut + P.cut_off, P.ncut_cap, a.coef0, a.coef1, a.coef2, a.rhs_kind,
-                 a.rhs_p0, a.loc + (int64_t)LOC_N * P.cut_off, a.flags + P.cut_off, &a.perr[lo]};
-    local_p1_one(la, c);
-}
-
-// ---------------------------------------------------------------------------
-// the persistent solve
+//   k_batch_local       one thread per cut tet of any problem: local matrices and qualification
+//   k_batch_first       one thread per (cut tet, vertex): first-encounter owner
+//   k_batch_rank        per problem: owner ranks, DOF count
+//   k_batch_dofs        one thread per (cut tet, vertex)
+//   k_batch_rows<>      one wave per row: count, then (k_batch_rowptr per problem) fill
+// Threads find their problem from the offsets' table; a problem that failed a step (exact zero, capacity)
+// is skipped from there on.  512 problems of 16^3 to 64^3 cells (5.1 M cut
+// tets, 1.8 M rows): 27.0 -> 10.1 ms, local matrices 5.1, rows 1.0 + 2.1, cells 0.83 + 0.25, owners 0.5, the rest 0.3.
 // ---------------------------------------------------------------------------
 struct BatchArgs {
     const BatchProb *prob;
@@ -205,10 +113,15 @@ struct BatchArgs {
     int32_t nprob;
     int32_t *queue;             // next position in `order` (zeroed before the launch)
     const double *phi;
+    uint8_t *cellmask;          // per problem cell (cell_off layout)
+    int32_t *blkcnt;            // [nprob][max_blocks]
+    int32_t max_blocks;
+    int32_t *zero, *perr;       // per problem: exact-zero node in a cut tet; local error bits (2: all-zero sub-tet)
+    int64_t cut_total, row_total;
     uint32_t *cellinfo;
     int64_t *cut;
     uint8_t *flags;
-    double *loc;                // SoA [LOC_N][ncut] per problem
+    double *loc;                // SoA [LOC_N][ncut_cap] per problem
     int32_t *first, *slot, *dofs;
     int32_t *rowowner, *rowlen, *rowptr;
     int32_t *col;
@@ -228,9 +141,209 @@ struct BatchArgs {
     int rel;
     double inner_tol;
     int inner_max;
-    int prepass = 0;            // 1: cut lists, cell words, flags and local data come from the pre-pass
-    const int32_t *pre_zero = nullptr, *pre_err = nullptr;
 };
+
+__global__ void __launch_bounds__(BPLAN) k_batch_cut_count(BatchArgs a) {
+    const int p = blockIdx.y;
+    const BatchProb &P = a.prob[p];
+    const int64_t cell = (int64_t)blockIdx.x * BPLAN + threadIdx.x;
+    if (blockIdx.x == 0 && threadIdx.x == 0) a.stat[p].t0 = wall_clock64();
+    if ((int64_t)blockIdx.x * BPLAN >= P.m.ncell) return;
+    int mk = 0;
+    bool z = false;
+    if (cell < P.m.ncell) {
+        mk = cell_cut_mask(P.m, a.phi + P.phi_off, cell, z);
+        a.cellmask[P.cell_off + cell] = (uint8_t)mk;
+    }
+    int tot;
+    block_excl_scan<BPLAN>(__popc(mk), &tot);
+    if (threadIdx.x == 0) a.blkcnt[(int64_t)p * a.max_blocks + blockIdx.x] = tot;
+    if (z) atomicOr(&a.zero[p], 1);
+}
+
+// exclusive scan of in[0..n) into out (may alias) by a workgroup of 1024, four items a thread at a time;
+// returns the total
+constexpr int BSCAN = 1024;
+__device__ inline int64_t wg_scan4(const int32_t *in, int32_t *out, int64_t n) {
+    int64_t carry = 0;
+    for (int64_t i0 = 0; i0 < n; i0 += 4 * BSCAN) {
+        const int64_t i = i0 + 4 * threadIdx.x;
+        int v[4], s = 0;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            v[k] = i + k < n ? in[i + k] : 0;
+            s += v[k];
+        }
+        int tot;
+        int off = (int)carry + block_excl_scan<BSCAN>(s, &tot);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            if (i + k < n) out[i + k] = off;
+            off += v[k];
+        }
+        carry += tot;
+    }
+    return carry;
+}
+
+__global__ void __launch_bounds__(BSCAN) k_batch_cut_scan(BatchArgs a) {
+    const int p = blockIdx.x;
+    const BatchProb &P = a.prob[p];
+    int32_t *cnt = a.blkcnt + (int64_t)p * a.max_blocks;
+    const int64_t ncut = wg_scan4(cnt, cnt, (P.m.ncell + BPLAN - 1) / BPLAN);
+    if (threadIdx.x != 0) return;
+    BatchStat &st = a.stat[p];
+    st.ncut = (int32_t)ncut;
+    st.ndof = st.nnz = st.iters = st.outer = 0;
+    st.resid = 0.0;
+    st.status = ncut > P.ncut_cap ? DHIP_E_CAPACITY : a.zero_throw && a.zero[p] ? DHIP_E_ZERO_NODE : DHIP_OK;
+    st.t1 = st.t_asm = wall_clock64();
+}
+
+__global__ void __launch_bounds__(BPLAN) k_batch_cut_fill(BatchArgs a) {
+    const int p = blockIdx.y;
+    const BatchProb &P = a.prob[p];
+    if ((int64_t)blockIdx.x * BPLAN >= P.m.ncell || a.stat[p].status != DHIP_OK) return;
+    const int64_t cell = (int64_t)blockIdx.x * BPLAN + threadIdx.x;
+    const int mask = cell < P.m.ncell ? a.cellmask[P.cell_off + cell] : 0;
+    const int off = block_excl_scan<BPLAN>(__popc(mask), nullptr);
+    if (cell >= P.m.ncell) return;
+    int64_t b = (int64_t)a.blkcnt[(int64_t)p * a.max_blocks + blockIdx.x] + off;
+    a.cellinfo[P.cell_off + cell] = ((uint32_t)b << 6) | (uint32_t)mask;
+    for (int k = 0; k < 6; ++k)
+        if (mask & (1 << k)) a.cut[P.cut_off + b++] = cell * 6 + k;   // (the counts are within the capacity)
+}
+
+// The problem whose range of a flat index holds g, ranges starting at off(problem): the last one that starts at
+// or before g.  The wave's first index is searched for all lanes together.
+template <class F>
+__device__ __forceinline__ int batch_find(int nprob, int64_t g, F &&off) {
+    const uint32_t lo32 = __builtin_amdgcn_readfirstlane((int)(uint32_t)g);
+    const int64_t g0 = (int64_t)((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(g >> 32)) << 32 | lo32);
+    int lo = 0, hi = nprob - 1;
+    while (lo < hi) {
+        const int mid = (lo + hi + 1) >> 1;
+        if (off(mid) <= g0) lo = mid;
+        else hi = mid - 1;
+    }
+    while (lo + 1 < nprob && off(lo + 1) <= g) ++lo;
+    return lo;
+}
+
+// problem and cut tet of flat cut slot g; false for the unused capacity and failed problems
+__device__ __forceinline__ bool batch_tet(const BatchArgs &a, int64_t g, int &p, int64_t &c) {
+    p = batch_find(a.nprob, g, [&](int k) { return a.prob[k].cut_off; });
+    c = g - a.prob[p].cut_off;
+    return a.stat[p].status == DHIP_OK && c < a.stat[p].ncut;
+}
+
+__global__ void __launch_bounds__(LOCAL_BLOCK) k_batch_local(BatchArgs a) {
+    const int64_t g = (int64_t)blockIdx.x * LOCAL_BLOCK + threadIdx.x;
+    if (g >= a.cut_total) return;
+    int p;
+    int64_t c;
+    if (!batch_tet(a, g, p, c)) return;
+    const BatchProb &P = a.prob[p];
+    double *loc = a.loc + (int64_t)LOC_N * P.cut_off;
+    LocalArgs la{P.m, a.phi + P.phi_off, a.cut + P.cut_off, P.ncut_cap, a.coef0, a.coef1, a.coef2, a.rhs_kind,
+                 a.rhs_p0, loc, a.flags + P.cut_off, &a.perr[p]};
+    local_p1_one(la, c);
+    QualArgs qa{P.m, a.cut + P.cut_off, P.ncut_cap, loc, a.flags + P.cut_off, a.omit_bound};
+    qualify_one(qa, c);
+}
+
+constexpr int BFLAT = 256;
+
+__global__ void __launch_bounds__(BFLAT) k_batch_first(BatchArgs a) {
+    const int64_t g = (int64_t)blockIdx.x * BFLAT + threadIdx.x;
+    if (g >= 4 * a.cut_total) return;
+    int p;
+    int64_t c;
+    if (!batch_tet(a, g >> 2, p, c)) return;
+    const BatchProb &P = a.prob[p];
+    FirstArgs fa{P.m, a.cut + P.cut_off, a.stat[p].ncut, a.cellinfo + P.cell_off, a.flags + P.cut_off,
+                 a.first + 4 * P.cut_off, a.slot + 4 * P.cut_off};
+    first_one(fa, 4 * c + (g & 3));
+}
+
+__global__ void __launch_bounds__(BSCAN) k_batch_rank(BatchArgs a) {
+    const int p = blockIdx.x;
+    const BatchProb &P = a.prob[p];
+    BatchStat &st = a.stat[p];
+    if (st.status != DHIP_OK) return;
+    if (a.perr[p] & 2) {
+        if (threadIdx.x == 0) st.status = DHIP_E_ZERO_PATTERN;
+        return;
+    }
+    int32_t *slot = a.slot + 4 * P.cut_off;   // owner flag -> owner rank
+    const int64_t nd = wg_scan4(slot, slot, 4 * (int64_t)st.ncut);
+    if (threadIdx.x == 0) {
+        st.ndof = (int32_t)nd;
+        if (nd > P.row_cap) st.status = DHIP_E_CAPACITY;
+    }
+}
+
+__global__ void __launch_bounds__(BFLAT) k_batch_dofs(BatchArgs a) {
+    const int64_t g = (int64_t)blockIdx.x * BFLAT + threadIdx.x;
+    if (g >= 4 * a.cut_total) return;
+    int p;
+    int64_t c;
+    if (!batch_tet(a, g >> 2, p, c)) return;
+    const BatchProb &P = a.prob[p];
+    const int64_t s = 4 * c + (g & 3), o = 4 * P.cut_off;
+    const int32_t f = a.first[o + s];
+    a.dofs[o + s] = f >= 0 ? a.slot[o + f] : -1;
+    if (f == s) a.rowowner[P.row_off + a.slot[o + s]] = (int32_t)s;
+}
+
+template <bool FILL>
+__global__ void __launch_bounds__(64 * ROWW_WAVES) k_batch_rows(BatchArgs a) {
+    __shared__ RowWShared shm[ROWW_WAVES];
+    const int w = threadIdx.x >> 6;
+    const int64_t g = (int64_t)xcd_position(blockIdx.x, gridDim.x) * ROWW_WAVES + w;
+    if (g >= a.row_total) return;
+    const int p = __builtin_amdgcn_readfirstlane(
+        batch_find(a.nprob, g, [&](int k) { return a.prob[k].row_off; }));
+    const BatchProb &P = a.prob[p];
+    const BatchStat &st = a.stat[p];
+    const int64_t r = g - P.row_off;
+    if (st.status != DHIP_OK || r >= st.ndof) return;
+    RowArgs ra{P.m, a.cut + P.cut_off, P.ncut_cap, a.cellinfo + P.cell_off, a.flags + P.cut_off,
+               a.dofs + 4 * P.cut_off, a.rowowner + P.row_off, st.ndof, a.loc + (int64_t)LOC_N * P.cut_off,
+               a.rowlen + P.row_off, a.rowptr + P.row_off + p, a.col + P.nz_off, a.vm + P.nz_off, a.vl + P.nz_off,
+               a.vs + P.nz_off, a.vc + P.nz_off, a.rhs + P.row_off, a.diag + P.row_off, P.lc[0], P.lc[1], P.lc[2]};
+    row_wave<FILL>(ra, r, shm[w]);
+}
+
+__global__ void __launch_bounds__(BSCAN) k_batch_rowptr(BatchArgs a) {
+    const int p = blockIdx.x;
+    const BatchProb &P = a.prob[p];
+    BatchStat &st = a.stat[p];
+    if (st.status != DHIP_OK) return;
+    int32_t *rowptr = a.rowptr + P.row_off + p;
+    const int64_t nnz = wg_scan4(a.rowlen + P.row_off, rowptr, st.ndof);
+    if (threadIdx.x == 0) {
+        rowptr[st.ndof] = (int32_t)nnz;
+        st.nnz = (int32_t)nnz;
+        if (nnz > P.nz_cap) st.status = DHIP_E_CAPACITY;
+    }
+}
+
+// exclusive scan of a[0..n) in place by the whole workgroup; returns the total
+template <int BB>
+__device__ inline int64_t wg_scan_inplace(int32_t *a, int64_t n) {
+    int64_t carry = 0;
+    for (int64_t i0 = 0; i0 < n; i0 += BB) {
+        const int64_t i = i0 + threadIdx.x;
+        const int v = i < n ? a[i] : 0;
+        int tot;
+        const int off = block_excl_scan<BB>(v, &tot);
+        if (i < n) a[i] = (int32_t)(carry + off);
+        carry += tot;
+    }
+    __syncthreads();
+    return carry;
+}
 
 // two workgroup sums with one LDS round
 template <int BB>
@@ -301,121 +414,6 @@ __device__ __forceinline__ double sell_spmv_group(const int32_t *soff, const int
         }
     }
     return p_lam;
-}
-
-// Assembly of problem p; its stat entry carries the sizes and the status to k_batch_solve.
-template <int BB>
-__device__ void batch_problem(const BatchArgs &a, int p) {
-    __shared__ int sh_zero, sh_err;   // workgroup flags (LDS: no stale cache lines)
-    const BatchProb P = a.prob[p];
-    const MeshP m = P.m;
-    const int tid = threadIdx.x;
-    const double *phi = a.phi + P.phi_off;
-    uint32_t *cellinfo = a.cellinfo + P.cell_off;
-    int64_t *cut = a.cut + P.cut_off;
-    uint8_t *flags = a.flags + P.cut_off;
-    double *loc = a.loc + (int64_t)LOC_N * P.cut_off;
-    int32_t *first = a.first + 4 * P.cut_off, *slot = a.slot + 4 * P.cut_off, *dofs = a.dofs + 4 * P.cut_off;
-    int32_t *rowowner = a.rowowner + P.row_off, *rowlen = a.rowlen + P.row_off, *rowptr = a.rowptr + P.row_off + p;
-    int32_t *col = a.col + P.nz_off;
-    double *vm = a.vm + P.nz_off, *vl = a.vl + P.nz_off, *vs = a.vs + P.nz_off, *vc = a.vc + P.nz_off;
-    double *rhs = a.rhs + P.row_off, *diag = a.diag + P.row_off;
-    BatchStat st{};
-    st.t0 = wall_clock64();
-    st.status = DHIP_OK;
-
-    // ---- classification + compaction in cell order ----
-    if (tid == 0) {
-        sh_zero = 0;
-        sh_err = 0;
-    }
-    __syncthreads();
-    int64_t ncut = 0;
-    bool over = false;
-    if (a.prepass) {
-        ncut = P.ncut_cap;   // the planned count is exact: same level set, same classification
-        if (a.pre_zero[p]) sh_zero = 1;
-        if (a.pre_err[p] & 2) sh_err = 2;
-    }
-    for (int64_t c0 = 0; c0 < (a.prepass ? 0 : m.ncell); c0 += BB) {
-        const int64_t cell = c0 + tid;
-        int mk = 0;
-        if (cell < m.ncell) {
-            bool z;
-            mk = cell_cut_mask(m, phi, cell, z);
-            if (z) sh_zero = 1;
-        }
-        int tot;
-        const int off = block_excl_scan<BB>(__popc(mk), &tot);
-        if (cell < m.ncell) {
-            int64_t b = ncut + off;
-            cellinfo[cell] = ((uint32_t)b << 6) | (uint32_t)mk;
-            for (int k = 0; k < 6; ++k)
-                if (mk & (1 << k)) {
-                    if (b < P.ncut_cap) cut[b] = cell * 6 + k;
-                    ++b;
-                }
-        }
-        ncut += tot;
-    }
-    __syncthreads();
-    st.ncut = (int32_t)ncut;
-    if (ncut > P.ncut_cap) over = true;
-    if (a.zero_throw && sh_zero) st.status = DHIP_E_ZERO_NODE;
-    if (over) st.status = DHIP_E_CAPACITY;
-
-    int64_t nd = 0, nnz = 0;
-    if (st.status == DHIP_OK) {
-        // ---- local matrices ----
-        if (!a.prepass) {
-            LocalArgs la{m, phi, cut, ncut, a.coef0, a.coef1, a.coef2, a.rhs_kind, a.rhs_p0, loc, flags, &sh_err};
-            for (int64_t c = tid; c < ncut; c += BB) local_p1_one(la, c);
-        }
-        __syncthreads();
-        if (sh_err & 2) st.status = DHIP_E_ZERO_PATTERN;
-    }
-    if (st.status == DHIP_OK) {
-        // ---- first-encounter numbering ----
-        QualArgs qa{m, cut, ncut, loc, flags, a.omit_bound};
-        for (int64_t c = tid; c < ncut; c += BB) qualify_one(qa, c);
-        __syncthreads();
-        FirstArgs fa{m, cut, ncut, cellinfo, flags, first, slot};
-        for (int64_t s = tid; s < 4 * ncut; s += BB) first_one(fa, s);
-        __syncthreads();
-        nd = wg_scan_inplace<BB>(slot, 4 * ncut);   // slot: owner flag -> owner rank
-        if (nd > P.row_cap) st.status = DHIP_E_CAPACITY;
-    }
-    if (st.status == DHIP_OK) {
-        for (int64_t s = tid; s < 4 * ncut; s += BB) {
-            const int32_t f = first[s];
-            dofs[s] = f >= 0 ? slot[f] : -1;
-            if (f == s) rowowner[slot[s]] = (int32_t)s;
-        }
-        __syncthreads();
-        // ---- CSR rows ----
-        RowArgs ra{m, cut, ncut, cellinfo, flags, dofs, rowowner, nd, loc, rowlen, rowptr, col,
-                   vm, vl, vs, vc, rhs, diag, P.lc[0], P.lc[1], P.lc[2]};
-        for (int64_t r = tid; r < nd; r += BB) rowcount_one(ra, r);
-        __syncthreads();
-        for (int64_t r = tid; r < nd; r += BB) rowptr[r] = rowlen[r];
-        __syncthreads();
-        nnz = wg_scan_inplace<BB>(rowptr, nd);
-        if (tid == 0) rowptr[nd] = (int32_t)nnz;
-        if (nnz > P.nz_cap) st.status = DHIP_E_CAPACITY;
-        __syncthreads();
-    }
-    st.ndof = (int32_t)nd;
-    st.nnz = (int32_t)nnz;
-    if (st.status == DHIP_OK) {
-        RowArgs ra{m, cut, ncut, cellinfo, flags, dofs, rowowner, nd, loc, rowlen, rowptr, col,
-                   vm, vl, vs, vc, rhs, diag, P.lc[0], P.lc[1], P.lc[2]};
-        for (int64_t r = tid; r < nd; r += BB) rowfill_one(ra, r);
-        __syncthreads();
-        st.t_asm = wall_clock64();
-    }
-    st.t1 = wall_clock64();
-    if (tid == 0) a.stat[p] = st;
-    __syncthreads();
 }
 
 // The same PCG for a problem whose search direction does not fit the workgroup's LDS: every vector in
@@ -1015,8 +1013,8 @@ __device__ __noinline__ void batch_pcg_chip(const BatchArgs &a, int p, BatchStat
     st.status = status == 0 ? DHIP_OK : DHIP_E_NOT_CONVERGED;
 }
 
-template <int BB>
-__global__ void __launch_bounds__(BB) k_batch(BatchArgs a) {
+// The PCG of every assembled problem: problems from the second queue counter, largest first.
+__global__ void __launch_bounds__(BPT) k_batch_solve(BatchArgs a) {
     __shared__ int sh_p;
     for (;;) {
         if (threadIdx.x == 0) {
@@ -1027,24 +1025,9 @@ __global__ void __launch_bounds__(BB) k_batch(BatchArgs a) {
         const int p = sh_p;
         __syncthreads();
         if (p < 0) break;
-        batch_problem<BB>(a, p);
-    }
-}
-
-// The PCG of every assembled problem: problems from the second queue counter, largest first.
-__global__ void __launch_bounds__(BPT) k_batch_solve(BatchArgs a) {
-    __shared__ int sh_p;
-    for (;;) {
-        if (threadIdx.x == 0) {
-            const int q = atomicAdd(a.queue + 1, 1);
-            sh_p = q < a.nprob ? a.order[q] : -1;
-        }
-        __syncthreads();
-        const int p = sh_p;
-        __syncthreads();
-        if (p < 0) break;
         BatchStat st = a.stat[p];
         if (st.status == DHIP_OK) {
+            st.t_asm = wall_clock64();
             const int slots = (st.ndof + BPT - 1) / BPT;
             // the smallest size class that holds the problem; the LDS of the classes up to 27 slots fits (asserted)
             switch (slots) {

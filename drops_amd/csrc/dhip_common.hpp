@@ -166,11 +166,8 @@ struct dhip_ctx {
     // optional per-block wall-clock probe of the persistent solver
     bool probe_on = false;
     int64_t pcg_rows_per_block = 0;   // 0: one row per thread of a 512-thread block
-    int batch_threads = 256;          // workgroup size of the batched solve (128, 256, 512)
-    int batch_blocks_per_cu = 2;      // resident workgroups per CU of the batched solve
     int xcd_map = 1;                  // persistent solvers: each XCD's blocks own one contiguous run of rows
     int coherent_exchange = 2;        // persistent solvers' exchange: 0 fenced, 1 coherent atomics, 2 tagged records (FP64 PCG)
-    int batch_prepass = 0;            // batched solve: classification and local matrices over the whole grid first
     bool coop_refused = false;        // cooperative launch unavailable: same grid, regular launch
     int probe_blocks = 0;
     dhip::DevBuf probe;

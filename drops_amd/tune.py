@@ -41,13 +41,13 @@ def tune_pcg(ctx, A, b_dev, x_dev, zero_dev, n, tol=1e-8, precision=D.FP64, cand
     return choice, timings
 
 
-# (assembly threads, workgroups per CU, grid-wide pre-pass of classification and local matrices,
-#  0: threads of the PCG launch, which has one geometry)
-BATCH_CANDIDATES = ((512, 1, 0, 0), (512, 1, 1, 0), (256, 1, 0, 0), (256, 2, 1, 0))
+# the batch keys (threads, workgroups per CU, pre-pass, solve threads or 0) of a candidate; the library's batched
+# launches have one geometry, so one candidate serves
+BATCH_CANDIDATES = ((512, 1, 1, 0),)
 
 
 def tune_batch(ctx, batch, tol=1e-8, candidates=BATCH_CANDIDATES, reps=2):
-    """Workgroup size, residency and pre-pass of the batched assembly: times `reps`
+    """The batch keys among `candidates`: times `reps`
     graph replays per candidate (best of; the capture is untimed) on the caller's problem set, after
     one untimed launch, and leaves the fastest on the context.  Returns
     ((threads, blocks_per_cu, prepass, solve_threads), {candidate: seconds})."""

@@ -476,9 +476,9 @@ int dhip_ch_solve_learned(dhip_ch_t *ch, dhip_mlp_t *mlp, int32_t *iters, double
  * No reference counterpart: each problem is what a DROPS caller does once per level set --
  * IdxDescCL::CreateNumbering (misc/problem.cpp:725-745), accumulate() of the P1 interface mass,
  * Laplace-Beltrami and stabilisation accumulators (num/accumulator.h:265-268), LinComb, and
- * PCGSolverCL<JACPcCL>::Solve (num/krylovsolver.h:1805-1835) -- for a set of level sets.  One
- * workgroup owns one problem at a time (workgroup barriers only), problems are taken largest first
- * from a queue, and the solve is Jacobi PCG with FP32 inner iterations and FP64 residuals and
+ * PCGSolverCL<JACPcCL>::Solve (num/krylovsolver.h:1805-1835) -- for a set of level sets.  The
+ * assembly takes its steps over all problems together; the solve is one workgroup per problem,
+ * largest first from a queue: Jacobi PCG with FP32 inner iterations and FP64 residuals and
  * refinement from x = 0.  The assembled arrays of each problem equal those of dhip_assemble_p1. */
 typedef struct dhip_batch dhip_batch_t;
 typedef struct {
@@ -494,7 +494,7 @@ typedef struct {
     int32_t iters, outer; /* FP32 inner iterations in total, FP64 refinement steps */
     double resid;         /* final FP64 relative residual */
     double start_s, end_s;  /* device wall clock at the start and end of the problem in the last solve */
-    double assembled_s;     /* device wall clock when its system was assembled */
+    double assembled_s;     /* device wall clock when its PCG started */
 } dhip_batch_stat_t;
 /* Plans the batch: counts each problem's cut tets and cut-tet vertices on the device and sizes
  * the per-problem scratch.  phi holds all level sets (phi_count values, DHIP_HOST: copied;
@@ -503,13 +503,11 @@ int dhip_batch_create(dhip_ctx_t *ctx, int32_t nprob, const dhip_batch_problem_t
                       int64_t phi_count, int32_t where, int32_t zero_policy, const double coef[3],
                       int32_t rhs_kind, const double *rhs_param, double omit_bound, dhip_batch_t **batch);
 /* Assembles and solves every problem (relative residual tol, at most max_iter inner iterations per
- * problem): one launch that assembles, one workgroup per problem, and one that runs the PCGs, one
- * problem per CU at a time, largest first.  use_graph: capture the launches into a hipGraph on the
- * first call and replay it while the arguments stay the same.  The assembly's workgroup size and
- * residency come from dhip_tune("batch_threads" 128/256/512, "batch_blocks_per_cu" 1..8);
- * "batch_prepass" 1 runs classification, compaction and local matrices of all problems over the
- * whole grid before it (same results; 0 is the default).  The PCG has one geometry: the keys
- * "batch_split" and "batch_solve_threads" are accepted and change nothing. */
+ * problem): launches that take one assembly step over all problems each, and one that runs the PCGs,
+ * one problem per CU at a time, largest first.  use_graph: capture the launches into a hipGraph on
+ * the first call and replay it while the arguments stay the same.  The launches have one geometry:
+ * the tuning keys "batch_threads" (128/256/512), "batch_blocks_per_cu" (1..8), "batch_prepass" (0/1),
+ * "batch_split" (0/1) and "batch_solve_threads" (256/512/1024) are accepted and change nothing. */
 int dhip_batch_solve(dhip_batch_t *batch, int32_t max_iter, double tol, int32_t rel, int32_t use_graph);
 /* per-problem results of the last solve (nprob entries) */
 int dhip_batch_stats(dhip_batch_t *batch, dhip_batch_stat_t *stats);
