@@ -123,6 +123,18 @@ static void derive_tables(Tables &T) {
             for (int j = 0; j < 3; ++j) T.rp_tri[pid][tr][j] = (int8_t)(tr < ntri ? roots[tr + j] : 0);
         T.rp_bnd[pid] = (int8_t)(nz == 3);
     }
+    for (int pid = 0; pid < 81; ++pid) {
+        uint32_t w = (uint32_t)T.rp_size[pid] | (uint32_t)(T.rp_bnd[pid] != 0) << 2;
+        for (int tr = 0; tr < 2; ++tr)
+            for (int j = 0; j < 3; ++j) w |= (uint32_t)T.rp_tri[pid][tr][j] << (4 + 12 * tr + 4 * j);
+        T.rp_word[pid] = w;
+    }
+    for (int t = 0; t < 8; ++t)
+        for (int r = 0; r < 10; ++r) {
+            const int a = r < 4 ? T.lat_t[t][r] : T.edge_ab[T.sub_edge[t][r - 4]][0];
+            const int b = r < 4 ? a : T.edge_ab[T.sub_edge[t][r - 4]][1];
+            T.root_ends[t][r] = (uint8_t)(a | b << 4);
+        }
     // P2 dof (vertices 0-3, edges 0-5) -> lattice vertex
     for (int l = 0; l < 10; ++l) {
         int a = -1, b = -1;

@@ -96,21 +96,19 @@ __device__ inline double tet_volume(const double X[4][3]) {
                 v[0][2] * (v[1][0] * v[2][1] - v[1][1] * v[2][0])) / 6.0;
 }
 
-// P2 basis sum (FE_P2CL::H0..H9 + LinearCombinationCL) for the squared hat of vertex i:
-// nodal values 1 at vertex i, 0.25 at its three edges, 0 elsewhere.
-__device__ inline double hat_sq_eval(int i, const double p[4]) {
-    const double h[10] = {p[0] * (2. * p[0] - 1.), p[1] * (2. * p[1] - 1.), p[2] * (2. * p[2] - 1.),
-                          p[3] * (2. * p[3] - 1.), 4. * p[0] * p[1],         4. * p[0] * p[2],
-                          4. * p[1] * p[2],         4. * p[0] * p[3],         4. * p[1] * p[3],
-                          4. * p[2] * p[3]};
+// P2 basis sums (FE_P2CL::H0..H9 + LinearCombinationCL) for the squared hats of the four vertices: nodal
+// values 1 at vertex i, 0.25 at its three edges, 0 elsewhere, in the reference's order of the nodes.
+__device__ __forceinline__ void hat_sq_all(const double p[4], double hs[4]) {
     // edges (0,1),(0,2),(1,2),(0,3),(1,3),(2,3)
     const int ea[6] = {0, 0, 1, 0, 1, 2}, eb[6] = {1, 2, 2, 3, 3, 3};
-    double s = h[0] * (i == 0 ? 1. : 0.);
 #pragma unroll
-    for (int d = 1; d < 4; ++d) s += h[d] * (i == d ? 1. : 0.);
+    for (int i = 0; i < 4; ++i) hs[i] = p[i] * (2. * p[i] - 1.);
 #pragma unroll
-    for (int e = 0; e < 6; ++e) s += h[4 + e] * ((ea[e] == i || eb[e] == i) ? 0.25 : 0.);
-    return s;
+    for (int e = 0; e < 6; ++e) {
+        const double h = 4. * p[ea[e]] * p[eb[e]] * 0.25;
+        hs[ea[e]] += h;
+        hs[eb[e]] += h;
+    }
 }
 
 __device__ inline double rhs_fun(int kind, double p0, const double x[3]) {
@@ -398,150 +396,183 @@ __device__ inline void stab_p1(const LocalArgs &a, const double ls[10], const do
     }
 }
 
-// The local matrices of one cut tet.  ROLE < 0: every output; otherwise one group, so that four
-// waves can share a tet: 0 mass + numbering integrals, 1 Laplace-Beltrami, 2 load vector, area and
-// the flags, 3 stabilisation.  Each output is summed by the same statements in the same order in
-// every form, so the parts equal the whole bit for bit.
-template <int ROLE>
-__device__ inline void local_p1_part(const LocalArgs &a, int64_t c) {
-    constexpr bool ALL = ROLE < 0;
-    constexpr bool MASS = ALL || ROLE == 0, LB = ALL || ROLE == 1, LOAD = ALL || ROLE == 2, STAB = ALL || ROLE == 3;
-    constexpr bool FACETS = MASS || LB || LOAD;
+// The sign-pattern and lattice tables of one wave's tets in LDS (their indices differ from lane to lane), and
+// the lanes' ten level-set values, which the facets index.
+struct LocalP1Shared {
+    double ls[10][LOCAL_BLOCK];
+    double latb[10][4];
+    uint32_t rp[81];    // c_tab.rp_word
+    uint8_t ends[80];   // c_tab.root_ends
+};
+
+__device__ inline void local_p1_tables(LocalP1Shared &sh) {
+    for (int i = threadIdx.x; i < 81; i += LOCAL_BLOCK) sh.rp[i] = c_tab.rp_word[i];
+    for (int i = threadIdx.x; i < 80; i += LOCAL_BLOCK) sh.ends[i] = c_tab.root_ends[i / 10][i % 10];
+    for (int i = threadIdx.x; i < 40; i += LOCAL_BLOCK) sh.latb[i / 4][i % 4] = c_tab.lat_b[i / 4][i % 4];
+    __syncthreads();
+}
+
+// The local matrices of one cut tet, one lane per tet in a block of LOCAL_BLOCK lanes (tables staged).
+// The facets are listed first, four bits each, so that the wave runs as many facet passes as its tet of most
+// facets has (about nine) and not two for each of the eight sub-tets; every sum still takes the facets in
+// make_patch order.  Terms with a factor 0 of the reference's sums (a corner of the Quad2 rule, a squared hat's
+// other nodes) are left out and factors 1 too: neither changes a value.  Bound by FP64 issue at two waves a SIMD
+// (208 registers).  Loops over sub-tets and triangles, with the values indexed in registers lane by lane and the
+// tables read per lane from constant memory: 1,302 tets 105 -> 53 us, 88,086 tets 145 -> 78 us, 352,000 tets
+// 391 -> 214 us, 243,000 band tets 269 -> 166 us.
+__device__ inline void local_p1_one(const LocalArgs &a, int64_t c, LocalP1Shared &sh) {
+    const int lane = threadIdx.x;
     double X[4][3], ls[10];
     load_tet_geom(a.m, a.phi, a.cut[c], X, ls);
     double G1[4][3];
     const double det = p1_grad(X, G1);
+
+    // sign pattern of each sub-tet (7 bits each) and the list of facets (2 lt + triangle, 4 bits each)
+    uint32_t pos = 0, neg = 0;
+#pragma unroll
+    for (int l = 0; l < 10; ++l) {
+        pos |= ls[l] > 0. ? 1u << l : 0u;
+        neg |= ls[l] < 0. ? 1u << l : 0u;
+        sh.ls[l][lane] = ls[l];
+    }
+    uint64_t pids = 0, list = 0;
+    int nfacet = 0;
+    bool body = false;
+    for (int lt = 0; lt < 8; ++lt) {
+        int pid = 40, p3 = 1;
+        uint32_t any = 0;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const int lv = c_tab.lat_t[lt][q];
+            const uint32_t p = (pos >> lv) & 1u, n = (neg >> lv) & 1u;
+            pid += p3 * ((int)p - (int)n);
+            any |= p | n;
+            p3 *= 3;
+        }
+        body |= any == 0;
+        const int ntri = sh.rp[pid] & 3;
+        pids |= (uint64_t)pid << (7 * lt);
+        if (ntri > 0) list |= (uint64_t)(2 * lt) << (4 * nfacet++);
+        if (ntri > 1) list |= (uint64_t)(2 * lt + 1) << (4 * nfacet++);
+    }
+    if (body) {
+        atomicOr(a.err, 2);
+        a.flags[c] = 0;   // defined for the steps that run before the error is read
+        return;
+    }
+    const int64_t N = a.ncut;
+    double *L = a.loc;
+    a.flags[c] = nfacet > 0 ? 1 : (a.band ? 0x21 : 0);
+    if (nfacet == 0) {
+        for (int e = 0; e < LOC_N; ++e) L[e * N + c] = 0.;
+        // NarrowBandMatrixAccuP1CL: the stabilisation of a band tet does not need the patch
+        if (a.band) stab_p1(a, ls, G1, det, c);
+        return;
+    }
 
     // accumulators (facet-major, node-minor, as the reference's flattened quadrature sums)
     double mdiag[4] = {0., 0., 0., 0.}, moff[6] = {0., 0., 0., 0., 0., 0.};
     double lbs[10] = {0., 0., 0., 0., 0., 0., 0., 0., 0., 0.};
     double hat[4] = {0., 0., 0., 0.}, rhs[4] = {0., 0., 0., 0.};
     double area = 0.;
-    int nfacet = 0;
-    const double *fvals = (LOAD && a.rhs_kind == DHIP_RHS_VALUES) ? a.rhs_vals + a.rhs_off[c] : nullptr;
+    const double *fvals = a.rhs_kind == DHIP_RHS_VALUES ? a.rhs_vals + a.rhs_off[c] : nullptr;
 
-    for (int lt = 0; lt < 8; ++lt) {
-        int s[4];
+    for (int f = 0; f < nfacet; ++f) {
+        const int e4 = (int)(list >> (4 * f)) & 15, lt = e4 >> 1, tr = e4 & 1;
+        const uint32_t w = sh.rp[(pids >> (7 * lt)) & 127];
+        double vb[3][4];
 #pragma unroll
-        for (int q = 0; q < 4; ++q) s[q] = sgn(ls[c_tab.lat_t[lt][q]]);
-        if (!s[0] && !s[1] && !s[2] && !s[3]) {
-            if (LOAD) {
-                atomicOr(a.err, 2);
-                a.flags[c] = 0;   // defined for the steps that run before the error is read
+        for (int j = 0; j < 3; ++j) {
+            const int rep = (w >> (4 + 12 * tr + 4 * j)) & 15, en = sh.ends[10 * lt + rep];
+            const double *ba = sh.latb[en & 15];
+            if (rep < 4) {
+#pragma unroll
+                for (int cc = 0; cc < 4; ++cc) vb[j][cc] = ba[cc];
+            } else {
+                const double *bb = sh.latb[en >> 4];
+                const double va = sh.ls[en & 15][lane], alpha = va / (va - sh.ls[en >> 4][lane]);
+#pragma unroll
+                for (int cc = 0; cc < 4; ++cc) vb[j][cc] = (1.0 - alpha) * ba[cc] + alpha * bb[cc];
             }
-            return;
         }
-        const int pid = s[0] + 3 * s[1] + 9 * s[2] + 27 * s[3] + 40;
-        const int ntri = c_tab.rp_size[pid];
-        if constexpr (!FACETS) {
-            nfacet += ntri;
-            continue;
+        double absdet, nrm[3];
+        facet_qr(X, vb, absdet, nrm);
+        double af = (w & 4) ? 0.5 : 1.;
+        af *= absdet;
+        // Quad2 composite: mass + numbering integrals; its nodes are the corners and the barycentre
+#pragma unroll
+        for (int qn = 0; qn < 4; ++qn) {
+            double nb[4];
+#pragma unroll
+            for (int cc = 0; cc < 4; ++cc) {
+                if (qn < 3) {
+                    nb[cc] = vb[qn < 3 ? qn : 0][cc];
+                } else {
+                    double sv = vb[0][cc] * (1. / 3.);
+                    sv += vb[1][cc] * (1. / 3.);
+                    sv += vb[2][cc] * (1. / 3.);
+                    nb[cc] = sv;
+                }
+            }
+            const double wq = af * (qn < 3 ? 1. / 24. : 0.375);
+            double hs[4];
+            hat_sq_all(nb, hs);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                mdiag[i] += wq * (nb[i] * nb[i]);
+                hat[i] += wq * hs[i];
+            }
+            int o = 0;
+#pragma unroll
+            for (int i = 1; i < 4; ++i)
+#pragma unroll
+                for (int j = 0; j < i; ++j) moff[o++] += wq * (nb[j] * nb[i]);
         }
-        const bool bnd = c_tab.rp_bnd[pid] != 0;
-        for (int tr = 0; tr < ntri; ++tr) {
-            double vb[3][4];
-            facet_vertices(ls, lt, pid, tr, vb);
-            ++nfacet;
-            double absdet, nrm[3];
-            facet_qr(X, vb, absdet, nrm);
-            double af = bnd ? 0.5 : 1.;
-            af *= absdet;
-            // Quad2 composite: mass + numbering integrals
-            if (MASS) {
+        // Laplace-Beltrami: projected gradients per facet
+        {
+            double q[4][3];
 #pragma unroll
-                for (int qn = 0; qn < 4; ++qn) {
-                    double nb[4];
+            for (int i = 0; i < 4; ++i) {
+                const double d = dot3(G1[i], nrm);
 #pragma unroll
-                    for (int cc = 0; cc < 4; ++cc) {
-                        double sv = vb[0][cc] * c_tab.q2n[qn][0];
-                        sv += vb[1][cc] * c_tab.q2n[qn][1];
-                        sv += vb[2][cc] * c_tab.q2n[qn][2];
-                        nb[cc] = sv;
-                    }
-                    const double wq = af * c_tab.q2w[qn];
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        mdiag[i] += wq * (nb[i] * nb[i]);
-                        hat[i] += wq * hat_sq_eval(i, nb);
-                    }
-                    int o = 0;
-#pragma unroll
-                    for (int i = 1; i < 4; ++i)
-#pragma unroll
-                        for (int j = 0; j < i; ++j) moff[o++] += wq * (nb[j] * nb[i]);
-                }
+                for (int cc = 0; cc < 3; ++cc) q[i][cc] = G1[i][cc] - d * nrm[cc];
             }
-            // Laplace-Beltrami: projected gradients per facet
-            if (LB) {
-                double q[4][3];
+            int o = 0;
 #pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const double d = dot3(G1[i], nrm);
+            for (int i = 0; i < 4; ++i)
 #pragma unroll
-                    for (int cc = 0; cc < 3; ++cc) q[i][cc] = G1[i][cc] - d * nrm[cc];
+                for (int j = 0; j <= i; ++j) lbs[o++] += dot3(q[i], q[j]) * absdet;
+        }
+        // Quad5 composite: load vector and area
+#pragma unroll
+        for (int qn = 0; qn < 7; ++qn) {
+            const double wq = af * c_tab.q5w[qn];
+            area += wq;
+            if (a.rhs_kind != DHIP_RHS_NONE) {
+                double nb[4];
+#pragma unroll
+                for (int cc = 0; cc < 4; ++cc) {
+                    double sv = vb[0][cc] * c_tab.q5n[qn][0];
+                    sv += vb[1][cc] * c_tab.q5n[qn][1];
+                    sv += vb[2][cc] * c_tab.q5n[qn][2];
+                    nb[cc] = sv;
                 }
-                int o = 0;
-#pragma unroll
-                for (int i = 0; i < 4; ++i)
-#pragma unroll
-                    for (int j = 0; j <= i; ++j) lbs[o++] += dot3(q[i], q[j]) * absdet;
-            }
-            // Quad5 composite: load vector and area
-            if (LOAD) {
-#pragma unroll
-                for (int qn = 0; qn < 7; ++qn) {
-                    double nb[4];
-#pragma unroll
-                    for (int cc = 0; cc < 4; ++cc) {
-                        double sv = vb[0][cc] * c_tab.q5n[qn][0];
-                        sv += vb[1][cc] * c_tab.q5n[qn][1];
-                        sv += vb[2][cc] * c_tab.q5n[qn][2];
-                        nb[cc] = sv;
-                    }
-                    const double wq = af * c_tab.q5w[qn];
-                    area += wq * 1.;
-                    if (a.rhs_kind != DHIP_RHS_NONE) {
-                        double f;
-                        if (fvals) {
-                            f = fvals[7 * (nfacet - 1) + qn];
-                        } else {
-                            double x[3];
-                            b2w(X, nb, x);
-                            f = rhs_fun(a.rhs_kind, a.rhs_p0, x);
-                        }
-#pragma unroll
-                        for (int i = 0; i < 4; ++i) rhs[i] += wq * (f * nb[i]);
-                    }
+                double fx;
+                if (fvals) {
+                    fx = fvals[7 * f + qn];
+                } else {
+                    double x[3];
+                    b2w(X, nb, x);
+                    fx = rhs_fun(a.rhs_kind, a.rhs_p0, x);
                 }
+#pragma unroll
+                for (int i = 0; i < 4; ++i) rhs[i] += wq * (fx * nb[i]);
             }
         }
     }
 
-    const int64_t N = a.ncut;
-    double *L = a.loc;
-    if (LOAD) a.flags[c] = nfacet > 0 ? 1 : (a.band ? 0x21 : 0);
-    if (nfacet == 0) {
-        auto zero = [&](int e0, int cnt) {
-            for (int e = e0; e < e0 + cnt; ++e) L[e * N + c] = 0.;
-        };
-        if (MASS) {
-            zero(LOC_MASS, 16);
-            zero(LOC_HAT, 4);
-        }
-        if (LB) zero(LOC_LB, 16);
-        if (LOAD) {
-            zero(LOC_RHS, 4);
-            zero(LOC_AREA, 1);
-        }
-        if (STAB) {
-            zero(LOC_STAB, 16);
-            // NarrowBandMatrixAccuP1CL: the stabilisation of a band tet does not need the patch
-            if (a.band) stab_p1(a, ls, G1, det, c);
-        }
-        return;
-    }
     // mass: diagonal without alpha, off-diagonal alpha * integral
-    if (MASS) {
+    {
         int o = 0;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
@@ -556,7 +587,7 @@ __device__ inline void local_p1_part(const LocalArgs &a, int64_t c) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) L[(LOC_HAT + i) * N + c] = hat[i];
     }
-    if (LB) {
+    {
         const double fac = a.coef1 * 0.5;
         int o = 0;
 #pragma unroll
@@ -568,22 +599,18 @@ __device__ inline void local_p1_part(const LocalArgs &a, int64_t c) {
                 L[(LOC_LB + j * 4 + i) * N + c] = v;
             }
     }
-    if (LOAD) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) L[(LOC_RHS + i) * N + c] = rhs[i];
-        L[LOC_AREA * N + c] = area;
-    }
-    if (STAB) stab_p1(a, ls, G1, det, c);
+    for (int i = 0; i < 4; ++i) L[(LOC_RHS + i) * N + c] = rhs[i];
+    L[LOC_AREA * N + c] = area;
+    stab_p1(a, ls, G1, det, c);
 }
 
-__device__ inline void local_p1_one(const LocalArgs &a, int64_t c) { local_p1_part<-1>(a, c); }
-
-// One lane per cut tet.  Splitting the outputs over four waves or four launches (local_p1_part<0..3>)
-// was measured slower: the facet geometry, which every group needs, dominates the cost.
 __global__ void __launch_bounds__(LOCAL_BLOCK) k_local_p1(LocalArgs a) {
+    __shared__ LocalP1Shared sh;
+    local_p1_tables(sh);
     const int64_t c = (int64_t)blockIdx.x * LOCAL_BLOCK + threadIdx.x;
     if (c >= a.ncut) return;
-    local_p1_one(a, c);
+    local_p1_one(a, c, sh);
 }
 
 // The composite-Quad5 points of every cut tet's patch in the load vector's order (facets in

@@ -238,6 +238,8 @@ __device__ __forceinline__ bool batch_tet(const BatchArgs &a, int64_t g, int &p,
 }
 
 __global__ void __launch_bounds__(LOCAL_BLOCK) k_batch_local(BatchArgs a) {
+    __shared__ LocalP1Shared sh;
+    local_p1_tables(sh);
     const int64_t g = (int64_t)blockIdx.x * LOCAL_BLOCK + threadIdx.x;
     if (g >= a.cut_total) return;
     int p;
@@ -247,7 +249,7 @@ __global__ void __launch_bounds__(LOCAL_BLOCK) k_batch_local(BatchArgs a) {
     double *loc = a.loc + (int64_t)LOC_N * P.cut_off;
     LocalArgs la{P.m, a.phi + P.phi_off, a.cut + P.cut_off, P.ncut_cap, a.coef0, a.coef1, a.coef2, a.rhs_kind,
                  a.rhs_p0, loc, a.flags + P.cut_off, &a.perr[p]};
-    local_p1_one(la, c);
+    local_p1_one(la, c, sh);
     QualArgs qa{P.m, a.cut + P.cut_off, P.ncut_cap, loc, a.flags + P.cut_off, a.omit_bound};
     qualify_one(qa, c);
 }
