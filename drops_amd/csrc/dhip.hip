@@ -458,7 +458,7 @@ void dhip_destroy(dhip_ctx_t *c) {
                       &c->rowlen, &c->rowptr, &c->col, &c->val[0], &c->val[1], &c->val[2], &c->val[3],
                       &c->rhs, &c->diag, &c->scan_tmp, &c->red_tmp, &c->bar, &c->host_stage, &c->qual,
                       &c->gm_sval, &c->probe, &c->gm_sell_off, &c->gm_sell_col, &c->gm_sell_val, &c->gm_sell_pos,
-                      &c->gm_sell_val32, &c->qp_off, &c->qp_vals, &c->qq_first, &c->qq_gh, &c->qq_list, &c->qqp_off, &c->qqp_vals};
+                      &c->gm_sell_val32, &c->gm_pair_off, &c->gm_pair_col, &c->gm_pair_val, &c->gm_pair_pos, &c->gm_pair_row, &c->qp_off, &c->qp_vals, &c->qq_first, &c->qq_gh, &c->qq_list, &c->qqp_off, &c->qqp_vals};
     for (DevBuf *b : bufs) b->release();
     for (auto &b : c->kv) b.release();
     (void)hipStreamDestroy(c->stream);
@@ -1959,16 +1959,66 @@ int dhip_solver_probe(dhip_ctx_t *c, int32_t on, uint64_t *ticks, int32_t *nbloc
 
 }  // extern "C"
 
+// The 2 x 2 block form of a matrix [A B; C D] of one pattern (k_gmres PAIR) for nb blocks of `per` pairs: the
+// layout once per pattern, the values of every solve.
+static int gmres_pairs(dhip_ctx *c, const dhip_csr *A, const double *diag, int64_t per, unsigned nb, bool f32,
+                       GmresArgs &ga) {
+    const int64_t np = A->n / 2, nnz1 = A->nnz / 4;
+    const int spb = (int)((per + 63) / 64);
+    const uint64_t key[4] = {A->pattern_id, (uint64_t)A->n, (uint64_t)A->nnz, (uint64_t)nb};
+    if (A->pattern_id == 0 || !std::equal(key, key + 4, c->gm_pair_key)) {
+        const int64_t nsl = (int64_t)nb * spb;
+        for (int k = 0; k < 4; ++k) c->gm_pair_key[k] = 0;
+        DHIP_HIPCHK(c, c->gm_pair_off.ensure(sizeof(int32_t) * (nsl + 1)));
+        DHIP_LAUNCH(c, "gmres_pair_width", k_pair_width, blocks_for(nsl, 256), 256, 0, np, per, spb, nsl, A->rowptr,
+                    c->gm_pair_off.as<int32_t>());
+        int rc = scan_exclusive_i32(c, c->gm_pair_off.as<int32_t>(), c->gm_pair_off.as<int32_t>(), nsl, &c->gm_pair_tot);
+        if (rc) return rc;
+        DHIP_HIPCHK(c, c->gm_pair_col.ensure(sizeof(int32_t) * (c->gm_pair_tot + 1)));
+        DHIP_HIPCHK(c, c->gm_pair_pos.ensure(sizeof(int32_t) * (nnz1 + 1)));
+        DHIP_HIPCHK(c, c->gm_pair_row.ensure(sizeof(int32_t) * (nnz1 + 1)));
+        DHIP_LAUNCH(c, "gmres_pair_fill", k_pair_fill, blocks_for(np, 256), 256, 0, np, per, spb, A->rowptr, A->col,
+                    c->gm_pair_off.as<int32_t>(), c->gm_pair_col.as<int32_t>(), c->gm_pair_pos.as<int32_t>(),
+                    c->gm_pair_row.as<int32_t>());
+        if (A->pattern_id != 0) std::copy(key, key + 4, c->gm_pair_key);
+    }
+    DHIP_HIPCHK(c, c->gm_pair_val.ensure(sizeof(double) * 4 * (c->gm_pair_tot + 1)));
+    double *pv = c->gm_pair_val.as<double>();
+    float *pv32 = f32 ? c->gm_pair_val.as<float>() : nullptr;
+    DHIP_LAUNCH(c, "gmres_pair_vals", k_pair_vals, blocks_for(nnz1, 256), 256, 0, nnz1, np, c->gm_pair_tot, A->rowptr,
+                A->col, c->gm_pair_pos.as<int32_t>(), c->gm_pair_row.as<int32_t>(), A->val, diag, pv, pv32);
+    ga.sell_off = c->gm_pair_off.as<int32_t>();
+    ga.sell_col = c->gm_pair_col.as<int32_t>();
+    ga.sell_spb = spb;
+    ga.pair_val = pv;
+    ga.pair_val32 = pv32;
+    ga.pair_tot = c->gm_pair_tot;
+    return DHIP_OK;
+}
+
 // Persistent GMRES(m) on device vectors: diag == nullptr means no preconditioner.
 // f32: Arnoldi cycles on FP32 basis and matrix values inside the FP64 restart residual (k_gmres F32).
+// block2: A is [A B; C D] with one pattern in its four blocks.
 static int gmres_core(dhip_ctx *c, const dhip_csr *A, const double *diag, const double *db, double *dx, int m,
-                      int32_t *max_iter, double *tol, int32_t rel, int32_t left_pc, bool f32 = false) {
+                      int32_t *max_iter, double *tol, int32_t rel, int32_t left_pc, bool f32 = false,
+                      bool block2 = false) {
     const int64_t n = A->n;
     DHIP_HIPCHK(c, c->kv[15].ensure(sizeof(double) * (size_t)m * n + 8));
     unsigned nb = 1;
     int rpt = 1;
     int rc = persistent_geometry(c, n, &nb, &rpt);
     if (rc) return rc;
+    // The pair form where a thread has more than one row, so that the basis is not in registers, and the average
+    // block's CSR slice would not fit in LDS; up to two pairs a thread.  128,352 unknowns, one row a thread: 61 us an
+    // iteration with the register basis, 76 in pairs; 191,104 unknowns: 107 us row by row, 72 in pairs.
+    const int64_t pair_per = (n / 2 + c->cu_count - 1) / c->cu_count;
+    const bool pair = block2 && rpt > 1 && diag && !left_pc && (c->coherent_exchange || f32) && n > 0 && A->nnz > 0 &&
+                      pair_per <= 2 * PB &&
+                      ((n + nb - 1) / nb + 1) * 4 + (A->nnz / nb) * 12 + 16 > (int64_t)LDS_BYTES;
+    if (pair) {
+        rpt = pair_per <= PB ? 2 : 4;
+        nb = (unsigned)((n / 2 + pair_per - 1) / pair_per);
+    }
     DHIP_HIPCHK(c, c->bar.ensure(sizeof(SyncSlot) * (nb + 1)));
     DHIP_HIPCHK(c, c->red_tmp.ensure(sizeof(double) * 2 * (size_t)nb * KMAX + 64));
     DHIP_HIPCHK(c, c->host_stage.ensure(64));
@@ -1980,7 +2030,10 @@ static int gmres_core(dhip_ctx *c, const dhip_csr *A, const double *diag, const 
                  c->bar.as<SyncSlot>(), c->red_tmp.as<double>(), m, *max_iter, *tol, rel, left_pc ? 1 : 0,
                  outs, outd, outs + 1, nullptr, nullptr, LDS_BYTES, nullptr, nullptr, nullptr, 0};
     ga.xcd_map = c->xcd_map;
-    if (diag && !left_pc && A->nnz > 0) {
+    if (pair) {
+        rc = gmres_pairs(c, A, diag, pair_per, nb, f32, ga);
+        if (rc) return rc;
+    } else if (diag && !left_pc && A->nnz > 0) {
         DHIP_HIPCHK(c, c->gm_sval.ensure(sizeof(double) * (A->nnz + 1)));
         DHIP_LAUNCH(c, "gmres_scale", k_scale_vals, blocks_for(A->nnz, 256), 256, 0, A->nnz, A->col, A->val, diag,
                     c->gm_sval.as<double>());
@@ -1990,7 +2043,7 @@ static int gmres_core(dhip_ctx *c, const dhip_csr *A, const double *diag, const 
     // when the average block would not fit).
     const int64_t per = (n + nb - 1) / nb;
     const uint64_t key[4] = {A->pattern_id, (uint64_t)n, (uint64_t)A->nnz, (uint64_t)nb};
-    if (A->nnz > 0 && (per + 1) * 4 + (A->nnz / nb) * 12 + 16 > (int64_t)LDS_BYTES && A->pattern_id != 0 &&
+    if (!pair && A->nnz > 0 && (per + 1) * 4 + (A->nnz / nb) * 12 + 16 > (int64_t)LDS_BYTES && A->pattern_id != 0 &&
         std::equal(key, key + 4, c->gm_sell_key)) {
         // the same pattern and block layout as the last solve: only the values change
         const int spb = (int)((per + 63) / 64);
@@ -2007,7 +2060,7 @@ static int gmres_core(dhip_ctx *c, const dhip_csr *A, const double *diag, const 
         ga.sell_col = c->gm_sell_col.as<int32_t>();
         ga.sell_val = c->gm_sell_val.as<double>();
         ga.sell_spb = spb;
-    } else if (A->nnz > 0 && (per + 1) * 4 + (A->nnz / nb) * 12 + 16 > (int64_t)LDS_BYTES) {
+    } else if (!pair && A->nnz > 0 && (per + 1) * 4 + (A->nnz / nb) * 12 + 16 > (int64_t)LDS_BYTES) {
         const int spb = (int)((per + 63) / 64);
         const int64_t nsl = (int64_t)nb * spb;
         for (int k = 0; k < 4; ++k) c->gm_sell_key[k] = 0;
@@ -2054,7 +2107,11 @@ static int gmres_core(dhip_ctx *c, const dhip_csr *A, const double *diag, const 
     const void *ks_32[5] = {regv ? (const void *)k_gmres<1, KREG, true, true> : (const void *)k_gmres<1, 0, true, true>,
                             (const void *)k_gmres<2, 0, true, true>, (const void *)k_gmres<4, 0, true, true>,
                             (const void *)k_gmres<8, 0, true, true>, (const void *)k_gmres<16, 0, true, true>};
-    const void *const *ks = f32 ? ks_32 : c->coherent_exchange ? ks_c : ks_f;
+    const void *ks_p[5] = {nullptr, (const void *)k_gmres<2, 0, true, false, true>,
+                           (const void *)k_gmres<4, 0, true, false, true>, nullptr, nullptr};
+    const void *ks_p32[5] = {nullptr, (const void *)k_gmres<2, 0, true, true, true>,
+                             (const void *)k_gmres<4, 0, true, true, true>, nullptr, nullptr};
+    const void *const *ks = pair ? (f32 ? ks_p32 : ks_p) : f32 ? ks_32 : c->coherent_exchange ? ks_c : ks_f;
     const int kidx = rpt == 1 ? 0 : rpt == 2 ? 1 : rpt == 4 ? 2 : rpt == 8 ? 3 : 4;
     const size_t lds = regv ? (size_t)LDS_BYTES : persistent_lds(c, ks[kidx]);
     ga.lds_bytes = (int64_t)lds;
@@ -2269,7 +2326,7 @@ static int ch_solve_impl(dhip_ch *h, int32_t *iters, double *resid) {
     int32_t it = h->p.max_iter;
     double tol = h->p.tol;
     rc = gmres_core(c, &h->K, h->pcdiag.as<double>(), h->rhs.as<double>(), h->x.as<double>(), m, &it, &tol,
-                    h->p.rel, 0, h->precision == DHIP_FP32_IR);
+                    h->p.rel, 0, h->precision == DHIP_FP32_IR, true);
     h->prepared = false;
     h->bdf_step = 0;
     h->bdf_e = 0.0;
@@ -2578,7 +2635,7 @@ static int ch_bdf_one(dhip_ch *h, const dhip_bdf_params_t &bp, dhip_bdf_stat_t *
         int32_t it = h->p.max_iter;
         double tl = h->p.tol;
         const int r = gmres_core(c, &h->K, h->pcdiag.as<double>(), h->rhs.as<double>(), xl, m, &it, &tl, h->p.rel, 0,
-                                 h->precision == DHIP_FP32_IR);
+                                 h->precision == DHIP_FP32_IR, true);
         *acc += it;
         resid = tl;
         return r;

@@ -164,6 +164,9 @@ struct dhip_ctx {
     dhip::DevBuf gm_sell_val32;                          // its values rounded to float (FP32 Arnoldi)
     int gmres_precision = 0;                             // DHIP_FP64 or DHIP_FP32_IR for dhip_gmres*
     dhip::DevBuf gm_sell_pos;                            // SELL slot of every CSR entry
+    dhip::DevBuf gm_pair_off, gm_pair_col, gm_pair_val, gm_pair_pos, gm_pair_row;  // SELL-64 of 2 x 2 blocks
+    int64_t gm_pair_tot = 0;
+    uint64_t gm_pair_key[4] = {0, 0, 0, 0};
     uint64_t gm_sell_key[4] = {0, 0, 0, 0};              // pattern id, rows, entries, blocks of the layout
     // optional per-block wall-clock probe of the persistent solver
     bool probe_on = false;

@@ -1751,7 +1751,63 @@ struct GmresArgs {
     int sell_spb;               // slices per block
     int xcd_map = 0;            // 1: the blocks of one XCD own one contiguous run of rows
     const float *sell_val32 = nullptr;  // FP32 Arnoldi: the SELL-64 values rounded to float
+    // PAIR: SELL-64 of the 2 x 2 blocks (sell_off / sell_col of pairs), values (a_00, a_01) of entry e at
+    // pair_val[2 e], (a_10, a_11) at pair_val[2 (pair_tot + e)], scaled by the preconditioner
+    const double *pair_val = nullptr;
+    const float *pair_val32 = nullptr;
+    int64_t pair_tot = 0;
 };
+
+// SELL-64 of the 2 x 2 blocks of a matrix [A B; C D] whose four blocks share one pattern: row i of the pattern
+// is the pair (i, n + i), entry k couples it to the pair of its k-th column.  Blocks of `per` pairs as k_sell_*.
+#ifndef DHIP_SOLVER_KERNELS
+__global__ void k_pair_width(int64_t np, int64_t per, int spb, int64_t nslices, const int32_t *rp, int32_t *width) {
+    const int64_t s = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (s >= nslices) return;
+    const int64_t b = s / spb, j = s - b * spb;
+    int32_t w = 0;
+    for (int64_t l = 64 * j; l < 64 * j + 64 && l < per; ++l) {
+        const int64_t r = b * per + l;
+        if (r >= np) break;
+        const int32_t len = (rp[r + 1] - rp[r]) / 2;
+        w = len > w ? len : w;
+    }
+    width[s] = 64 * w;
+}
+
+// the pattern: column pairs, and for every pattern entry its SELL slot and its row
+__global__ void k_pair_fill(int64_t np, int64_t per, int spb, const int32_t *rp, const int32_t *col,
+                            const int32_t *off, int32_t *scol, int32_t *pos, int32_t *row) {
+    const int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (r >= np) return;
+    const int64_t b = r / per, l = r - b * per;
+    const int32_t base = off[b * spb + (l >> 6)] + (int32_t)(l & 63), e0 = rp[r], len = (rp[r + 1] - e0) / 2;
+    for (int32_t k = 0; k < len; ++k) {
+        scol[base + 64 * k] = col[e0 + k];
+        pos[e0 / 2 + k] = base + 64 * k;
+        row[e0 / 2 + k] = (int32_t)r;
+    }
+}
+
+// the values of one solve, divided by the preconditioner of their column: one lane per pattern entry
+__global__ void k_pair_vals(int64_t nnz1, int64_t np, int64_t tot, const int32_t *rp, const int32_t *col,
+                            const int32_t *pos, const int32_t *row, const double *val, const double *diag,
+                            double *pv, float *pv32) {
+    const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (e >= nnz1) return;
+    const int32_t r = row[e], e0 = rp[r], len = (rp[r + 1] - e0) / 2, f0 = rp[np + r];
+    const int64_t k = e - e0 / 2, at = pos[e];
+    const int32_t c = col[e0 + k];
+    const double d0 = diag[c], d1 = diag[np + c];
+    const double v[4] = {val[e0 + k] / d0, val[e0 + len + k] / d1, val[f0 + k] / d0, val[f0 + len + k] / d1};
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+        const int64_t o = 2 * (at + (t < 2 ? 0 : tot)) + (t & 1);
+        if (pv32) pv32[o] = (float)v[t];
+        else pv[o] = v[t];
+    }
+}
+#endif
 
 // SELL-64 layout of a CSR matrix partitioned into blocks of `per` consecutive rows: the local rows
 // of a block form slices of 64; entry k of local row l sits at off[slice] + 64 k + (l % 64), so the
@@ -1819,7 +1875,12 @@ constexpr int KREG = 50;  // basis vectors kept in registers (restart m <= KREG,
 // b - A x, the Hessenberg least squares and x stay FP64, and a cycle that meets the tolerance by
 // its estimate is accepted only when the recomputed FP64 residual meets it too (iterative
 // refinement with one GMRES cycle as the inner solve).
-template <int RPT, int KR, bool COH, bool F32 = false>
+// PAIR: a 2 x 2 block matrix with one pattern, right preconditioned (the Cahn-Hilliard system).  The unknowns of
+// a pair sit on one thread and side by side in the basis vectors, so that one column index and one 16-byte gather
+// (8 in FP32) serve four entries, and the basis is read 16 bytes at a time.  The row-wise SELL form read a
+// column index and gathered once per entry: 47 us of a 107 us iteration on 191,104 unknowns (8.7 M entries); in pairs
+// 19 of 72 (33 of 86 with a batch's columns loaded in front of its gathers instead of one batch ahead).
+template <int RPT, int KR, bool COH, bool F32 = false, bool PAIR = false>
 __global__ void __launch_bounds__(PB) k_gmres(GmresArgs a)
 #ifndef DHIP_SOLVER_KERNELS
     ;
@@ -1835,16 +1896,22 @@ __global__ void __launch_bounds__(PB) k_gmres(GmresArgs a)
     __shared__ double red_sh[KMAX + 2];
     __shared__ double msh[KMAX + 2];         // this block's partial sums
     const int64_t n = a.n;
-    const int64_t per = (n + gridDim.x - 1) / gridDim.x;
+    const int64_t nu = PAIR ? n / 2 : n;   // rows, or pairs of rows
+    const int64_t per = (nu + gridDim.x - 1) / gridDim.x;
     const unsigned range = row_range_index(a.xcd_map);
     const int64_t r0 = (int64_t)range * per;
-    const int64_t r1 = r0 + per < n ? r0 + per : n;
-    const bool right = !a.left;
-    bool in_lds;
+    const int64_t r1 = r0 + per < nu ? r0 + per : nu;
+    const bool right = PAIR || !a.left;
+    bool in_lds = false;
     // right preconditioning: the slice holds a_rc / d_c (A M v); left: plain values (M A v)
     const bool pre = right && a.diag && a.sval;
-    const Slice<BT> S = load_slice_scaled<BT>(lds, a.rp, a.col, pre ? a.sval : a.val,
-                                              (right && !pre) ? a.diag : nullptr, r0, r1, in_lds);
+    // (const: its pointers keep the LDS address space)
+    const Slice<BT> S = [&] {
+        if constexpr (PAIR) return Slice<BT>{};
+        else
+            return load_slice_scaled<BT>(lds, a.rp, a.col, pre ? a.sval : a.val,
+                                         (right && !pre) ? a.diag : nullptr, r0, r1, in_lds);
+    }();
     const bool scaled = in_lds || pre;
     const double *dg = a.diag;
     // the global CSR values of a slice that is not in LDS (FP64 in both forms)
@@ -1856,7 +1923,7 @@ __global__ void __launch_bounds__(PB) k_gmres(GmresArgs a)
     else sell_val = a.sell_val;
     const bool sell = !in_lds && sell_val;
     const int32_t *sell_col = a.sell_col;
-    const int32_t *sell_off = a.sell_off + (sell ? (int64_t)range * a.sell_spb : 0);
+    const int32_t *sell_off = a.sell_off + (sell || PAIR ? (int64_t)range * a.sell_spb : 0);
     // SELL batches: one wave per CU-quarter runs here, so a batch may hold a whole long row in
     // registers; each batch costs two dependent memory round trips (entries, then gathers)
     constexpr int GBS = KR > 0 ? 8 : (F32 ? 40 : 20);
@@ -1905,13 +1972,17 @@ __global__ void __launch_bounds__(PB) k_gmres(GmresArgs a)
     bool own[RPT];
     int64_t lr[RPT];
     double xr[RPT], wr[RPT], dr[RPT];
+    // the system's row of the thread's k-th unknown, and its place among the block's basis entries
+    auto grow = [&](int k) { return PAIR ? (int64_t)(k & 1) * nu + r0 + lr[k] : r0 + lr[k]; };
+    auto li = [&](int k) { return PAIR ? 2 * lr[k] + (k & 1) : lr[k]; };
+    const int64_t v0 = PAIR ? 2 * r0 : r0;
 #pragma unroll
     for (int k = 0; k < RPT; ++k) {
-        lr[k] = threadIdx.x + (int64_t)k * PB;
+        lr[k] = threadIdx.x + (int64_t)(PAIR ? k / 2 : k) * PB;
         own[k] = r0 + lr[k] < r1;
         if (own[k]) {
-            xr[k] = a.x[r0 + lr[k]];
-            dr[k] = dg ? dg[r0 + lr[k]] : 1.0;
+            xr[k] = a.x[grow(k)];
+            dr[k] = dg ? dg[grow(k)] : 1.0;
         }
     }
     auto prec = [&](int k, double v) { return dg ? 1.0 * v / dr[k] : v; };
@@ -1927,7 +1998,7 @@ __global__ void __launch_bounds__(PB) k_gmres(GmresArgs a)
     // Without a register basis and with the CSR slice in global memory, the first KL basis
     // vectors of the block's rows are also kept in LDS: the dots and combinations read them there
     // (each thread reads back only its own rows), the SpMV gathers read the global copy.
-    const int64_t nrb = r1 > r0 ? r1 - r0 : 0;
+    const int64_t nrb = r1 > r0 ? (r1 - r0) * (PAIR ? 2 : 1) : 0;
     int KL = 0;
     BT *vl = reinterpret_cast<BT *>(lds);
     BT *V = reinterpret_cast<BT *>(a.V);
@@ -1938,18 +2009,76 @@ __global__ void __launch_bounds__(PB) k_gmres(GmresArgs a)
         }
     }
     auto vbasis = [&](int q, int64_t l) -> double {
-        return q < KL ? vl[(size_t)q * nrb + l] : V[(size_t)q * n + r0 + l];
+        return q < KL ? vl[(size_t)q * nrb + l] : V[(size_t)q * n + v0 + l];
     };
-    auto vstore = [&](int q, int64_t r, double v, bool mine) {
+    auto vstore = [&](int q, int64_t l, double v, bool mine) {
         const BT vb = (BT)v;
         if (mine) {
-            xstore<COH>(&V[(size_t)q * n + r], vb);
-            if (q < KL) vl[(size_t)q * nrb + (r - r0)] = vb;
+            xstore<COH>(&V[(size_t)q * n + v0 + l], vb);
+            if (q < KL) vl[(size_t)q * nrb + l] = vb;
         }
         if constexpr (REGV) {
 #pragma unroll
             for (int t = 0; t < KR - 1; ++t) vreg[t] = vreg[t + 1];
             vreg[KR - 1] = (double)vb;
+        }
+    };
+    // PAIR: w = A M v over the 2 x 2 blocks
+    auto pair_spmv = [&](const BT *vi) {
+        using P2 = typename std::conditional<F32, float2, double2>::type;
+        constexpr int G = F32 ? 16 : 12;
+        const P2 *top, *bot;
+        if constexpr (F32) top = reinterpret_cast<const P2 *>(a.pair_val32);
+        else top = reinterpret_cast<const P2 *>(a.pair_val);
+        bot = top + a.pair_tot;
+        const __amdgpu_buffer_rsrc_t vr =
+            __builtin_amdgcn_make_buffer_rsrc((void *)vi, 0, (int)(n * (int64_t)sizeof(BT)), 0x00020000);
+#pragma unroll
+        for (int k = 0; k < RPT; k += 2) {
+            wr[k] = wr[k + 1] = 0.0;
+            if (!own[k]) continue;
+            const int64_t l = lr[k];
+            const int32_t base = sell_off[l >> 6] + (int32_t)(l & 63);
+            const int32_t len = (a.rp[r0 + l + 1] - a.rp[r0 + l]) / 2;
+            double s0 = 0.0, s1 = 0.0;
+            // a batch's columns are loaded one batch ahead, so that only its gathers are waited for; entries past
+            // the row's end repeat its last one and add nothing
+            int32_t cc[G];
+            auto columns = [&](int32_t q0) {
+#pragma unroll
+                for (int j = 0; j < G; ++j) {
+                    const int32_t q = q0 + j < len ? q0 + j : len - 1;
+                    cc[j] = sell_col[base + 64 * q];
+                }
+            };
+            columns(0);
+            for (int32_t q0 = 0; q0 < len; q0 += G) {
+                P2 tt[G], bb[G], xx[G];
+#pragma unroll
+                for (int j = 0; j < G; ++j) {
+                    if constexpr (F32)
+                        xx[j] = __builtin_bit_cast(P2, __builtin_amdgcn_raw_buffer_load_b64(vr, 8 * cc[j], 0, TX_SC1));
+                    else
+                        xx[j] = __builtin_bit_cast(P2, __builtin_amdgcn_raw_buffer_load_b128(vr, 16 * cc[j], 0, TX_SC1));
+                }
+#pragma unroll
+                for (int j = 0; j < G; ++j) {
+                    const int32_t q = q0 + j < len ? q0 + j : len - 1;
+                    tt[j] = top[base + 64 * q];
+                    bb[j] = bot[base + 64 * q];
+                }
+                columns(q0 + G);
+#pragma unroll
+                for (int j = 0; j < G; ++j)
+                    if (q0 + j < len) {
+                        s0 += (double)tt[j].x * (double)xx[j].x;
+                        s0 += (double)tt[j].y * (double)xx[j].y;
+                        s1 += (double)bb[j].x * (double)xx[j].x;
+                        s1 += (double)bb[j].y * (double)xx[j].y;
+                    }
+            }
+            wr[k] = s0;
+            wr[k + 1] = s1;
         }
     };
     // block sums of w . V[q] (q < K) and, with `self`, w . w as entry K
@@ -1987,7 +2116,7 @@ __global__ void __launch_bounds__(PB) k_gmres(GmresArgs a)
                     if (q < KT) {
 #pragma unroll
                         for (int k = 0; k < RPT; ++k)
-                            if (own[k]) sacc += wr[k] * (q < K ? vbasis(q, lr[k]) : wr[k]);
+                            if (own[k]) sacc += wr[k] * (q < K ? vbasis(q, li(k)) : wr[k]);
                     }
                     p[u] = sacc;
                 }
@@ -2011,7 +2140,7 @@ __global__ void __launch_bounds__(PB) k_gmres(GmresArgs a)
 #pragma unroll
         for (int k = 0; k < RPT; ++k) {
             if (!own[k]) continue;
-            const int64_t r = r0 + lr[k];
+            const int64_t r = grow(k);
             const double ax =
                 row_product<double>(a.rp, a.col, a.val, 0, r, [&](int32_t c) { return xload<COH>(&a.x[c]); });
             double rv = a.b[r] - ax;
@@ -2030,7 +2159,7 @@ __global__ void __launch_bounds__(PB) k_gmres(GmresArgs a)
     // x += (M) V y over columns 0..kk of the basis
     // w - sign * sum_{q < cnt} h_q V[q][r], subtracting in q order (registers, or gathers of 8
     // basis entries issued before their first use)
-    auto combine_V = [&](double w, int64_t r, int cnt, const double *h, double sign) {
+    auto combine_V = [&](double w, int64_t l, int cnt, const double *h, double sign) {
         if constexpr (REGV) {
             const int off = KR - nvec;
 #pragma unroll
@@ -2042,13 +2171,42 @@ __global__ void __launch_bounds__(PB) k_gmres(GmresArgs a)
             for (int c0 = 0; c0 < cnt; c0 += 8) {
                 double vv[8];
 #pragma unroll
-                for (int q = 0; q < 8; ++q) vv[q] = c0 + q < cnt ? vbasis(c0 + q, r - r0) : 0.0;
+                for (int q = 0; q < 8; ++q) vv[q] = c0 + q < cnt ? vbasis(c0 + q, l) : 0.0;
 #pragma unroll
                 for (int q = 0; q < 8; ++q)
                     if (c0 + q < cnt) w -= sign * (h[c0 + q] * vv[q]);
             }
         }
         return w;
+    };
+    // the same for every unknown of the thread (PAIR: a pair's two basis entries together)
+    auto combine_rows = [&](double (&w)[RPT], int cnt, const double *h, double sign) {
+        if constexpr (PAIR) {
+#pragma unroll
+            for (int k = 0; k < RPT; k += 2) {
+                if (!own[k]) continue;
+                const int64_t l = li(k);
+                for (int c0 = 0; c0 < cnt; c0 += 8) {
+                    double va[8], vb[8];
+#pragma unroll
+                    for (int q = 0; q < 8; ++q) {
+                        va[q] = c0 + q < cnt ? vbasis(c0 + q, l) : 0.0;
+                        vb[q] = c0 + q < cnt ? vbasis(c0 + q, l + 1) : 0.0;
+                    }
+#pragma unroll
+                    for (int q = 0; q < 8; ++q)
+                        if (c0 + q < cnt) {
+                            const double hq = sign * h[c0 + q];
+                            w[k] -= hq * va[q];
+                            w[k + 1] -= hq * vb[q];
+                        }
+                }
+            }
+        } else {
+#pragma unroll
+            for (int k = 0; k < RPT; ++k)
+                if (own[k]) w[k] = combine_V(w[k], lr[k], cnt, h, sign);
+        }
     };
     auto update_x = [&](int kk) {
         if (threadIdx.x == 0) {
@@ -2059,13 +2217,13 @@ __global__ void __launch_bounds__(PB) k_gmres(GmresArgs a)
             }
         }
         __syncthreads();
+        double z[RPT];
 #pragma unroll
-        for (int k = 0; k < RPT; ++k) {
-            if (!own[k]) continue;
-            const int64_t r = r0 + lr[k];
-            const double z = combine_V(0.0, r, kk + 1, yv, -1.0);
-            xr[k] += right ? prec(k, z) : z;
-        }
+        for (int k = 0; k < RPT; ++k) z[k] = 0.0;
+        combine_rows(z, kk + 1, yv, -1.0);
+#pragma unroll
+        for (int k = 0; k < RPT; ++k)
+            if (own[k]) xr[k] += right ? prec(k, z[k]) : z[k];
     };
 
     {
@@ -2093,7 +2251,7 @@ __global__ void __launch_bounds__(PB) k_gmres(GmresArgs a)
             nvec = 0;
 #pragma unroll
             for (int k = 0; k < RPT; ++k)
-                vstore(0, r0 + lr[k], own[k] ? wr[k] * inv : 0.0, own[k]);
+                vstore(0, li(k), own[k] ? wr[k] * inv : 0.0, own[k]);
             nvec = 1;
             if (threadIdx.x < KMAX + 1) sv[threadIdx.x] = 0.0;
             if (threadIdx.x == 0) sv[0] = beta;
@@ -2105,12 +2263,16 @@ __global__ void __launch_bounds__(PB) k_gmres(GmresArgs a)
             const BT *vi = V + (size_t)i * n;
             // w = A M v_i (right) or M A v_i (left); h1 = V^T w
             const uint64_t t_sp = a.probe ? wall_clock64() : 0;
+            if constexpr (PAIR) {
+                pair_spmv(vi);
+            } else {
 #pragma unroll
-            for (int k = 0; k < RPT; ++k) {
-                if (!own[k]) continue;
-                double w = spmv_row(lr[k], [&](int32_t c) { return xload<COH>(&vi[c]); });
-                if (!right) w = prec(k, w);
-                wr[k] = w;
+                for (int k = 0; k < RPT; ++k) {
+                    if (!own[k]) continue;
+                    double w = spmv_row(lr[k], [&](int32_t c) { return xload<COH>(&vi[c]); });
+                    if (!right) w = prec(k, w);
+                    wr[k] = w;
+                }
             }
             if (a.probe) t_spmv += wall_clock64() - t_sp;
             dots(i + 1, false, msh);
@@ -2118,12 +2280,7 @@ __global__ void __launch_bounds__(PB) k_gmres(GmresArgs a)
             if (threadIdx.x <= i) Hc[threadIdx.x] = red_sh[threadIdx.x];
             __syncthreads();
             // w1 = w - V h1; h2 = V^T w1; |w1|^2
-#pragma unroll
-            for (int k = 0; k < RPT; ++k) {
-                if (!own[k]) continue;
-                const int64_t r = r0 + lr[k];
-                wr[k] = combine_V(wr[k], r, i + 1, Hc, 1.0);
-            }
+            combine_rows(wr, i + 1, Hc, 1.0);
             dots(i + 1, true, msh);
             if (!syncv(i + 2, red_sh)) { status = 2; goto done; }
             double hn2 = red_sh[i + 1];
@@ -2132,12 +2289,9 @@ __global__ void __launch_bounds__(PB) k_gmres(GmresArgs a)
             // v_{i+1} = (w1 - V h2) / |.|
             {
                 const double inv = 1.0 / hnorm;
-                double vnew[RPT];
+                combine_rows(wr, i + 1, red_sh, 1.0);
 #pragma unroll
-                for (int k = 0; k < RPT; ++k)
-                    vnew[k] = own[k] ? combine_V(wr[k], r0 + lr[k], i + 1, red_sh, 1.0) * inv : 0.0;
-#pragma unroll
-                for (int k = 0; k < RPT; ++k) vstore(i + 1, r0 + lr[k], vnew[k], own[k]);
+                for (int k = 0; k < RPT; ++k) vstore(i + 1, li(k), own[k] ? wr[k] * inv : 0.0, own[k]);
                 nvec = i + 2;
             }
             // Hessenberg column i: h1 + h2 (one thread per entry), then the Givens rotations by one
@@ -2186,7 +2340,7 @@ __global__ void __launch_bounds__(PB) k_gmres(GmresArgs a)
         // restart: publish x, r = b - A x (left: M r)
 #pragma unroll
         for (int k = 0; k < RPT; ++k)
-            if (own[k]) xstore<COH>(&a.x[r0 + lr[k]], xr[k]);
+            if (own[k]) xstore<COH>(&a.x[grow(k)], xr[k]);
         if (!syncv(0, red_sh)) { status = 2; goto done; }
         {
             double p_rr, p_bb;
@@ -2205,7 +2359,7 @@ done:
     if (status != 2) {
 #pragma unroll
         for (int k = 0; k < RPT; ++k)
-            if (own[k]) a.x[r0 + lr[k]] = xr[k];
+            if (own[k]) a.x[grow(k)] = xr[k];
     }
     if (a.probe && threadIdx.x == 0) {
         const uint64_t total = wall_clock64() - t_start;

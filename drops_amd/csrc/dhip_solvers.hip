@@ -68,6 +68,12 @@ template __global__ void k_gmres<4, 0, true, true>(GmresArgs);
 template __global__ void k_gmres<8, 0, true, true>(GmresArgs);
 #elif DHIP_SOLVER_PART == 13
 template __global__ void k_gmres<16, 0, true, true>(GmresArgs);
+#elif DHIP_SOLVER_PART == 15
+// 2 x 2 block systems
+template __global__ void k_gmres<2, 0, true, false, true>(GmresArgs);
+template __global__ void k_gmres<4, 0, true, false, true>(GmresArgs);
+template __global__ void k_gmres<2, 0, true, true, true>(GmresArgs);
+template __global__ void k_gmres<4, 0, true, true, true>(GmresArgs);
 #elif DHIP_SOLVER_PART == 14
 template __global__ void k_pcg64_pipe<1>(PcgTxArgs);
 template __global__ void k_pcg64_pipe<2>(PcgTxArgs);

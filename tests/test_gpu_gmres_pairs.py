@@ -1,0 +1,51 @@
+"""The 2 x 2 block form of the persistent GMRES (systems whose row slices do not fit in LDS): the Cahn-Hilliard
+step of the P2 space at sizes with one and with two pairs of unknowns a thread and ragged last blocks, in FP64 and
+with FP32 Arnoldi cycles.  The solution's true residual on the step's own CSR system meets the tolerance (right
+preconditioning stops on the estimate: 1.05 for its rounding over some thousand steps), the row-wise form
+(fenced exchange) takes the same number of iterations to 2% and agrees to what the tolerance leaves (the
+conditioning turns 1e-8 into up to 1e-4 of the state)."""
+import numpy as np
+import pytest
+import scipy.sparse as sp
+
+from drops_amd import ch_run
+from drops_amd import dhip as D
+
+pytestmark = pytest.mark.gpu
+
+
+def step(ctx, ch, seed, tol=1e-8):
+    c0, mu0 = ch_run.initial_state(ch.n, seed)
+    ch.set_state(c0, mu0)
+    ch.prepare()
+    s = ch.system_host()
+    it, _, ok = ch.solve()
+    assert ok
+    x = np.concatenate(ch.state()[::-1])
+    K = sp.csr_matrix((s["val"], s["col"], s["rowptr"]))
+    assert np.linalg.norm(s["rhs"] - K @ x) <= 1.05 * tol * np.linalg.norm(s["rhs"])
+    return x, it
+
+
+@pytest.mark.parametrize("cells", [82, 97, 116])
+def test_pair_form(ctx, cells):
+    print(f"[gpu gmres] 2x2 block form, P2 torus {cells}", flush=True)
+    m, phi = ch_run.torus_mesh(cells)
+    ch = ch_run.make_stepper(ctx, m, phi, space=2)
+    assert 2 * ch.n > 131072 and (ch.n > 131072) == (cells == 116)
+    x, it = step(ctx, ch, 7)
+    again, it2 = step(ctx, ch, 7)
+    assert it2 == it and np.array_equal(again, x)
+    ch.set_precision(D.FP32_IR)
+    x32, it32 = step(ctx, ch, 7)
+    assert np.linalg.norm(x32 - x) <= 1e-3 * np.linalg.norm(x) and abs(it32 - it) <= 0.3 * it
+    ch.set_precision(D.FP64)
+    if cells == 82:
+        ctx.tune("coherent_exchange", 0)
+        try:
+            xr, itr = step(ctx, ch, 7)
+        finally:
+            ctx.tune("coherent_exchange", 2)
+        assert abs(it - itr) <= 0.02 * itr + 2
+        assert np.linalg.norm(xr - x) <= 1e-3 * np.linalg.norm(x)
+    ch.close()
