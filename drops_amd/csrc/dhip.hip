@@ -419,9 +419,10 @@ int dhip_create(dhip_ctx_t **out, int32_t device) {
     // the tagged PCG kernels' dynamic LDS (their attribute raised here, once, so that the
     // allocation-free entry point launches them as they are)
     {
-        const void *kt[6] = {(const void *)k_pcg64_tx<1>, (const void *)k_pcg64_tx<2>, (const void *)k_pcg64_tx<4>,
+        const void *kt[9] = {(const void *)k_pcg64_tx<1>, (const void *)k_pcg64_tx<2>, (const void *)k_pcg64_tx<4>,
                              (const void *)k_pcg64_pipe<1>, (const void *)k_pcg64_pipe<2>,
-                             (const void *)k_pcg64_pipe<4>};
+                             (const void *)k_pcg64_pipe<4>, (const void *)k_pcg_mixed_tx<1>,
+                             (const void *)k_pcg_mixed_tx<2>, (const void *)k_pcg_mixed_tx<4>};
         size_t lim = persistent_lds(c, kt[2]);
         for (const void *k : kt) lim = std::min(lim, persistent_lds(c, k));
         c->tx_lds = lim;
@@ -1846,8 +1847,6 @@ int dhip_pcg(dhip_ctx_t *c, const dhip_csr_t *A, int32_t pc, const double *b, do
         if (n > 0)
             DHIP_LAUNCH(c, "csr_diag", k_diag, blocks_for(n, KB), KB, 0, n, A->rowptr, A->col, A->val, diag,
                         mixed ? diag32 : nullptr);
-        if (mixed && A->nnz > 0)
-            DHIP_LAUNCH(c, "csr_to_f32", k_to_f32, blocks_for(A->nnz, KB), KB, 0, A->nnz, A->val, val32);
         DHIP_LAUNCH(c, "zero_slots", k_zero_u32, blocks_for((int64_t)nb * sizeof(SyncSlot) / 4, 256), 256, 0,
                     c->bar.as<uint32_t>(), (int)(nb * sizeof(SyncSlot) / 4));
     }
@@ -1864,15 +1863,40 @@ int dhip_pcg(dhip_ctx_t *c, const dhip_csr_t *A, int32_t pc, const double *b, do
         if (rc) return rc;
     } else if (precision == DHIP_FP32_IR) {
         if (pc != DHIP_PC_JACOBI) return set_error(c, DHIP_E_ARG, "FP32 refinement path uses the Jacobi preconditioner");
-        for (int k = 6; k < 9; ++k) DHIP_HIPCHK(c, c->kv[k].ensure(sizeof(float) * (n + 1)));
-        PcgMixArgs pa{n, A->rowptr, A->col, A->val, diag, val32, db, dx, c->kv[6].as<float>(), c->kv[7].as<float>(),
-                      c->kv[8].as<float>(), c->bar.as<SyncSlot>(), *max_iter, *tol, rel, 1e-4, 400, outs, outd,
-                      outs + 1, outs + 2};
-        pa.xcd_map = c->xcd_map;
-        const void *ks[5] = {(const void *)k_pcg_mixed<1>, (const void *)k_pcg_mixed<2>, (const void *)k_pcg_mixed<4>,
-                             (const void *)k_pcg_mixed<8>, (const void *)k_pcg_mixed<16>};
-        rc = launch_persistent(c, "pcg_mixed", ks, rpt, nb, pa);
-        if (rc) return rc;
+        SolverResult tres{};
+        tres.i[1] = 3;
+        if (c->coherent_exchange >= 2 && rpt <= 4) {
+            // tagged records (cleared first: an earlier solve's tags would match); status 3 with x untouched where a
+            // block's slice and halo exceed its LDS
+            DHIP_HIPCHK(c, c->kv[16].ensure((size_t)32 * (n + 1)));
+            DHIP_LAUNCH(c, "zero_records", k_zero_u32, blocks_for(8 * n, 256), 256, 0, c->kv[16].as<uint32_t>(),
+                        (int)(8 * n));
+            PcgMixTxArgs pt{n, A->rowptr, A->col, A->val, diag, db, dx, c->kv[16].as<uint4>(), c->bar.as<SyncSlot>(),
+                            *max_iter, *tol, rel, 1e-4, 400, outs, outd, outs + 1, outs + 2, c->xcd_map,
+                            (int64_t)c->tx_lds};
+            const void *kt[5] = {(const void *)k_pcg_mixed_tx<1>, (const void *)k_pcg_mixed_tx<2>,
+                                 (const void *)k_pcg_mixed_tx<4>, nullptr, nullptr};
+            rc = launch_persistent(c, "pcg_mixed", kt, rpt, nb, pt, c->tx_lds);
+            if (rc) return rc;
+            DHIP_HIPCHK(c, hipMemcpyAsync(&tres, outs, sizeof tres, hipMemcpyDeviceToHost, c->stream));
+            DHIP_HIPCHK(c, hipStreamSynchronize(c->stream));
+            if (tres.i[1] == 3)
+                DHIP_LAUNCH(c, "zero_slots", k_zero_u32, blocks_for((int64_t)nb * sizeof(SyncSlot) / 4, 256), 256, 0,
+                            c->bar.as<uint32_t>(), (int)(nb * sizeof(SyncSlot) / 4));
+        }
+        if (tres.i[1] == 3) {
+            if (A->nnz > 0)
+                DHIP_LAUNCH(c, "csr_to_f32", k_to_f32, blocks_for(A->nnz, KB), KB, 0, A->nnz, A->val, val32);
+            for (int k = 6; k < 9; ++k) DHIP_HIPCHK(c, c->kv[k].ensure(sizeof(float) * (n + 1)));
+            PcgMixArgs pa{n, A->rowptr, A->col, A->val, diag, val32, db, dx, c->kv[6].as<float>(), c->kv[7].as<float>(),
+                          c->kv[8].as<float>(), c->bar.as<SyncSlot>(), *max_iter, *tol, rel, 1e-4, 400, outs, outd,
+                          outs + 1, outs + 2};
+            pa.xcd_map = c->xcd_map;
+            const void *ks[5] = {(const void *)k_pcg_mixed<1>, (const void *)k_pcg_mixed<2>, (const void *)k_pcg_mixed<4>,
+                                 (const void *)k_pcg_mixed<8>, (const void *)k_pcg_mixed<16>};
+            rc = launch_persistent(c, "pcg_mixed", ks, rpt, nb, pa);
+            if (rc) return rc;
+        }
     } else {
         return set_error(c, DHIP_E_ARG, "unknown precision");
     }

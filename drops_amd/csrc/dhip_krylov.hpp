@@ -953,19 +953,23 @@ __device__ inline int block_min_int(int v) {
 // the diagonal of their column (dg != nullptr), and nvec halo arrays X[nvec][nu].  Layout:
 // lrp[nr + 1] | lcol[nzb] | bits[nwords] | pre[nwords] | U[nu] | (16-aligned) lval[nzb] | X[nvec][nu].
 // fits is the same in every thread; false: the LDS holds neither (the arrays are then unusable).
-struct TxLocal {
+template <class VT>
+struct TxLocalT {
     int32_t *lrp, *lcol, *pre, *U;
     uint32_t *bits;
-    double *lval, *X;
+    VT *lval, *X;
     int cmn, nu;
     int64_t range;
     bool fits;
 };
 
-__device__ inline TxLocal tx_local_setup(unsigned char *lds, int64_t lds_bytes, const int32_t *rp, const int32_t *col,
+using TxLocal = TxLocalT<double>;
+
+template <class VT = double>
+__device__ inline TxLocalT<VT> tx_local_setup(unsigned char *lds, int64_t lds_bytes, const int32_t *rp, const int32_t *col,
                                          const double *val, const double *dg, int64_t r0, int64_t nr, int32_t nz0,
                                          int64_t nzb, int nvec) {
-    TxLocal T{};
+    TxLocalT<VT> T{};
     int cmn = 0x7fffffff, cmx = -1;
     for (int64_t k = threadIdx.x; k < nzb; k += PB) {
         const int c = col[nz0 + k];
@@ -983,7 +987,7 @@ __device__ inline TxLocal tx_local_setup(unsigned char *lds, int64_t lds_bytes, 
     int32_t *U = pre + nwords;
     bool fits = 4 * (size_t)(nr + 1 + nzb + 2 * nwords) <= (size_t)lds_bytes;
     int nu = 0;
-    double *lval = nullptr, *X = nullptr;
+    VT *lval = nullptr, *X = nullptr;
     if (fits && nzb > 0) {
         for (int64_t w = threadIdx.x; w < nwords; w += PB) bits[w] = 0u;
         __syncthreads();
@@ -1003,9 +1007,9 @@ __device__ inline TxLocal tx_local_setup(unsigned char *lds, int64_t lds_bytes, 
         const size_t int_bytes = 4 * (size_t)(nr + 1 + nzb + 2 * nwords + nu);
         const size_t lval_off = (int_bytes + 15) & ~(size_t)15;
         // the same in every thread (the scan total)
-        fits = lval_off + 8 * (size_t)(nzb + (int64_t)nvec * nu) <= (size_t)lds_bytes;
+        fits = lval_off + sizeof(VT) * (size_t)(nzb + (int64_t)nvec * nu) <= (size_t)lds_bytes;
         if (fits) {
-            lval = reinterpret_cast<double *>(lds + lval_off);
+            lval = reinterpret_cast<VT *>(lds + lval_off);
             X = lval + nzb;
             for (int64_t w = w0; w < w1; ++w) {
                 pre[w] = off;
@@ -1021,7 +1025,7 @@ __device__ inline TxLocal tx_local_setup(unsigned char *lds, int64_t lds_bytes, 
             for (int64_t k = threadIdx.x; k < nzb; k += PB) {
                 const int c = col[nz0 + k], d = c - cmn;
                 lcol[k] = pre[d >> 5] + __popc(bits[d >> 5] & ((1u << (d & 31)) - 1u));
-                lval[k] = dg ? val[nz0 + k] / dg[c] : val[nz0 + k];
+                lval[k] = (VT)(dg ? val[nz0 + k] / dg[c] : val[nz0 + k]);
             }
             __syncthreads();
         }
@@ -2383,6 +2387,15 @@ done:
 //         from d = 0 until |r_in| <= inner_tol or inner_max iterations
 //   update (FP64): x += |r| d
 // ---------------------------------------------------------------------------
+// Relative residual at which an FP32 inner solve stops, from the FP64 relative residual `resid` it starts at:
+// `base`, or what is left to `tol` (half of it, so that the FP64 check passes) where FP32 reaches that too.  With
+// `base` alone a solve to 1e-8 takes a third pass of 1e-4 for a factor of little over one (512 batched problems
+// 36.1 ms with `base`, 28.9 ms with what is left).
+__device__ __forceinline__ double inner_tolerance(double tol, double resid, double base) {
+    const double left = tol / resid;
+    return left >= 0.1 * base ? 0.5 * left : base;
+}
+
 struct PcgMixArgs {
     int64_t n;
     const int32_t *rp, *col;
@@ -2517,10 +2530,255 @@ __global__ void __launch_bounds__(PB) k_pcg_mixed(PcgMixArgs a)
             p_rr2 = block_sum<PB>(p_rr2);
             p_zr2 = block_sum<PB>(p_zr2);
             if (!sync_reduce<PB>(a.slots, ++gen, p_rr2, p_zr2, 0.0, red)) { fail = true; break; }
-            if (sqrt(red[0]) <= a.inner_tol) break;
+            if (sqrt(red[0]) <= inner_tolerance(a.tol, resid, a.inner_tol)) break;
             const double rho1 = rho;
             rho = red[1];
             beta = (float)(rho / rho1);
+        }
+        if (fail) { status = 2; break; }
+        // ---- FP64 refinement update, published for the next outer residual ----
+#pragma unroll
+        for (int k = 0; k < RPT; ++k) {
+            if (!own[k]) continue;
+            xr[k] += rnorm * (double)dv[k];
+            a.x[r0 + lr[k]] = xr[k];
+        }
+        if (!sync_reduce<PB>(a.slots, ++gen, 0.0, 0.0, 0.0, red)) { status = 2; break; }
+    }
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        *a.out_iter = total_it;
+        *a.out_resid = resid;
+        *a.out_status = status;
+        *a.out_outer = outer;
+    }
+}
+#endif
+
+// The mixed-precision PCG over tagged records (k_pcg64_tx's arrangement with FP32 inner vectors): r, w and s of a
+// row are one 16-byte record {r, w, s, generation}, a third of the FP64 form's, so that an inner iteration
+// waits for one device-coherent load per halo column and one reduction, both under way together; the block's
+// slice, divided by the preconditioner, and its halo are floats in LDS.  Dot products, the residual b - A x and x
+// are FP64 as in k_pcg_mixed, whose two fenced
+// reductions cost 7.5 us an inner iteration: a solve at 92 x 84 x 101 cells 8.4 -> 3.0 ms, inner_tolerance's shorter
+// last pass included.  A block whose
+// slice and halo do not fit the LDS makes every block leave with status 3 (the host then runs k_pcg_mixed).
+struct PcgMixTxArgs {
+    int64_t n;
+    const int32_t *rp, *col;
+    const double *val, *diag;
+    const double *b;
+    double *x;                  // FP64 solution (exchanged for the outer residual)
+    uint4 *T;                   // [2][n] records
+    SyncSlot *slots;
+    int max_iter;               // total inner iterations allowed
+    double tol;
+    int rel;
+    double inner_tol;
+    int inner_max;
+    int *out_iter;
+    double *out_resid;
+    int *out_status;
+    int *out_outer;
+    int xcd_map;
+    int64_t lds_bytes;
+};
+
+template <int RPT>
+__global__ void __launch_bounds__(PB) k_pcg_mixed_tx(PcgMixTxArgs a)
+#ifndef DHIP_SOLVER_KERNELS
+    ;
+#else
+{
+    extern __shared__ __align__(16) unsigned char lds[];
+    __shared__ double red_sh[SYNC_VALS];
+    bool tbad = false;   // this thread saw a timeout
+    const int64_t per = (a.n + gridDim.x - 1) / gridDim.x;
+    const int64_t r0 = (int64_t)row_range_index(a.xcd_map) * per;
+    const int64_t r1 = r0 + per < a.n ? r0 + per : a.n;
+    const int64_t nr = r1 > r0 ? r1 - r0 : 0;
+    const int32_t nz0 = nr ? a.rp[r0] : 0;
+    const int64_t nzb = nr ? (int64_t)a.rp[r1] - nz0 : 0;
+    const TxVec TV = tx_vec(a.T, a.n);
+    const TxLocalT<float> TL = tx_local_setup<float>(lds, a.lds_bytes, a.rp, a.col, a.val, a.diag, r0, nr, nz0, nzb, 3);
+    const int32_t *lrp = TL.lrp, *lcol = TL.lcol, *U = TL.U;
+    const float *lval = TL.lval;
+    const int nu = TL.nu;
+    const bool fits = TL.fits;
+    float *XR = TL.X, *XW = TL.X ? TL.X + nu : nullptr, *XS = TL.X ? TL.X + 2 * nu : nullptr;
+    auto local_of = [&](int64_t c) -> int {
+        const int64_t d = c - TL.cmn;
+        if (d < 0 || d >= TL.range) return -1;
+        const uint32_t w = TL.bits[d >> 5], m = 1u << (d & 31);
+        return (w & m) ? TL.pre[d >> 5] + __popc(w & (m - 1u)) : -1;
+    };
+    auto lds_row = [&](int64_t l, auto &&yv) {
+        const int32_t e0 = lrp[l + 1];
+        float s = 0.f;
+        for (int32_t q = lrp[l]; q < e0; ++q) s = __builtin_fmaf(lval[q], yv(lcol[q]), s);
+        return s;
+    };
+    auto publish = [&](uint32_t g, int64_t r, float rv, float wv, float sv) {
+        const u32x4 rec = {__float_as_uint(rv), __float_as_uint(wv), __float_as_uint(sv), g};
+        __builtin_amdgcn_raw_buffer_store_b128(rec, TV.rsrc, (uint32_t)(((g & 1) * a.n + r) * 16), 0, TX_SC1);
+    };
+    // The halo of generation g: the record of every distinct column not owned by the block, reloaded until
+    // its tag is g (a record is one 128-bit access; its tag word travels with it).
+    auto halo = [&](uint32_t g) {
+        for (int t = threadIdx.x; t < nu; t += PB) {
+            if (U[t] >= r0 && U[t] < r1) continue;
+            u32x4 v = tx_load_raw(TV, g, U[t]);
+            uint32_t spins = 0;
+            while (v[3] != g) {
+                if (++spins > SPIN_LIMIT) {
+                    tbad = true;
+                    break;
+                }
+                __asm__ __volatile__("" ::: "memory");   // (see k_pcg64_tx)
+                v = tx_load_raw(TV, g, U[t]);
+            }
+            XR[t] = __uint_as_float(v[0]);
+            XW[t] = __uint_as_float(v[1]);
+            XS[t] = __uint_as_float(v[2]);
+        }
+    };
+    auto collect = [&](uint32_t g) {
+        if (threadIdx.x < 64) {
+            double o[3];
+            const bool ok = slot_collect3(a.slots, g, o);
+            if (threadIdx.x == 0) {
+                red_sh[0] = o[0];
+                red_sh[1] = o[1];
+                red_sh[2] = o[2];
+                if (!ok) {
+                    tbad = true;
+                    a.slots[blockIdx.x].timeout = 1;
+                }
+            }
+        }
+        return !__syncthreads_or(tbad);
+    };
+    int status = 1, total_it = 0, outer = 0;
+    double resid = 0.0, normb = 1.0;
+    uint32_t gen = 0;   // slots' generations (sync_reduce and the tagged partials)
+    uint32_t rg = 0;    // records' generations
+    double xr[RPT], red[3];
+    float rr[RPT], ur[RPT], wr[RPT], pr[RPT], sr[RPT], dv[RPT], di[RPT];
+    int lo[RPT];
+    bool own[RPT];
+    int64_t lr[RPT];
+#pragma unroll
+    for (int k = 0; k < RPT; ++k) {
+        lr[k] = threadIdx.x + (int64_t)k * PB;
+        own[k] = lr[k] < nr;
+        lo[k] = (own[k] && fits) ? local_of(r0 + lr[k]) : -1;
+        if (own[k]) {
+            xr[k] = a.x[r0 + lr[k]];
+            di[k] = (float)a.diag[r0 + lr[k]];
+        }
+    }
+    bool first = true, fail = false;
+    for (;;) {
+        // ---- FP64 residual ----
+        double p_rr = 0.0, p_bb = 0.0, r64[RPT];
+#pragma unroll
+        for (int k = 0; k < RPT; ++k) {
+            if (!own[k]) continue;
+            const int64_t r = r0 + lr[k];
+            const double s = row_product<double>(a.rp, a.col, a.val, 0, r, [&](int32_t c) { return a.x[c]; });
+            const double bv = a.b[r];
+            r64[k] = bv - s;
+            p_rr += r64[k] * r64[k];
+            p_bb += bv * bv;
+        }
+        p_rr = block_sum<PB>(p_rr);
+        if (first) p_bb = block_sum<PB>(p_bb);
+        if (!sync_reduce<PB>(a.slots, ++gen, p_rr, p_bb, fits ? 0.0 : 1.0, red)) { status = 2; break; }
+        if (red[2] != 0.0) { status = 3; break; }
+        const double rnorm = sqrt(red[0]);
+        if (first) {
+            normb = sqrt(red[1]);
+            if (normb == 0.0 || !a.rel) normb = 1.0;
+            first = false;
+        }
+        resid = rnorm / normb;
+        if (resid <= a.tol) { status = 0; break; }
+        if (total_it >= a.max_iter) { status = 1; break; }
+        ++outer;
+        // ---- FP32 inner PCG on A d = r/|r| ----
+        const double scale = 1.0 / rnorm, itol = inner_tolerance(a.tol, resid, a.inner_tol);
+        ++rg;
+#pragma unroll
+        for (int k = 0; k < RPT; ++k) {
+            if (!own[k]) continue;
+            rr[k] = (float)(r64[k] * scale);
+            dv[k] = pr[k] = sr[k] = 0.f;
+            ur[k] = rr[k] / di[k];
+            publish(rg, r0 + lr[k], rr[k], 0.f, 0.f);
+            if (lo[k] >= 0) XR[lo[k]] = rr[k];
+        }
+        halo(rg);
+        __syncthreads();
+        double p_g = 0.0, p_d = 0.0, unused = 0.0;
+        ++rg;
+#pragma unroll
+        for (int k = 0; k < RPT; ++k) {
+            if (!own[k]) continue;
+            wr[k] = lds_row(lr[k], [&](int q) { return XR[q]; });
+            publish(rg, r0 + lr[k], rr[k], wr[k], 0.f);
+            p_g += (double)rr[k] * (double)ur[k];
+            p_d += (double)wr[k] * (double)ur[k];
+        }
+        block_sum3<PB>(p_g, p_d, unused);
+#pragma unroll
+        for (int k = 0; k < RPT; ++k)
+            if (lo[k] >= 0) {
+                XW[lo[k]] = wr[k];
+                XS[lo[k]] = 0.f;
+            }
+        ++gen;
+        if (threadIdx.x == 0) slot_publish3(a.slots, gen, p_g, p_d, 0.0);
+        double gamma = 0.0, alpha = 0.0, beta = 0.0;
+        for (int it = 0;; ++it) {
+            halo(rg);
+            if (!collect(gen)) { fail = true; break; }
+            if (it == 0) {
+                gamma = red_sh[0];
+                alpha = red_sh[0] / red_sh[1];
+            } else {
+                if (sqrt(red_sh[2]) <= itol || it == a.inner_max || total_it == a.max_iter) break;
+                const double gamma_new = red_sh[0];
+                beta = gamma_new / gamma;
+                alpha = gamma_new / (red_sh[1] - beta * gamma_new / alpha);
+                gamma = gamma_new;
+            }
+            ++total_it;
+            const float al = (float)alpha, be = (float)beta;
+            double p_g2 = 0.0, p_d2 = 0.0, p_rr2 = 0.0;
+            ++rg;
+            ++gen;
+#pragma unroll
+            for (int k = 0; k < RPT; ++k) {
+                if (!own[k]) continue;
+                pr[k] = ur[k] + be * pr[k];
+                sr[k] = wr[k] + be * sr[k];
+                dv[k] += al * pr[k];
+                rr[k] = rr[k] - al * sr[k];
+                ur[k] = rr[k] / di[k];
+                wr[k] = lds_row(lr[k], [&](int q) { return XR[q] - al * (XW[q] + be * XS[q]); });
+                publish(rg, r0 + lr[k], rr[k], wr[k], sr[k]);
+                p_g2 += (double)rr[k] * (double)ur[k];
+                p_d2 += (double)wr[k] * (double)ur[k];
+                p_rr2 += (double)rr[k] * (double)rr[k];
+            }
+            block_sum3<PB>(p_g2, p_d2, p_rr2);
+#pragma unroll
+            for (int k = 0; k < RPT; ++k)
+                if (lo[k] >= 0) {
+                    XR[lo[k]] = rr[k];
+                    XW[lo[k]] = wr[k];
+                    XS[lo[k]] = sr[k];
+                }
+            if (threadIdx.x == 0) slot_publish3(a.slots, gen, p_g2, p_d2, p_rr2);
         }
         if (fail) { status = 2; break; }
         // ---- FP64 refinement update, published for the next outer residual ----

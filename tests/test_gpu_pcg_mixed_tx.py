@@ -1,0 +1,66 @@
+"""The mixed-precision PCG over tagged records: every rows-per-thread class and the forms it hands over (eight
+rows a thread, a slice beyond the LDS, the fenced exchange), tiny and ragged systems, and solves after solves in
+one context, whose records must not be taken for this one's.  Each solution's true FP64 residual meets the
+tolerance (x 1.01: it is summed in another order here)."""
+import numpy as np
+import pytest
+import scipy.sparse as sp
+
+import cases
+from drops_amd import dhip as D
+
+pytestmark = pytest.mark.gpu
+
+
+def assembled(ctx, n):
+    m, phi = cases.c1_sphere(n)
+    ctx.mesh(m)
+    ctx.levelset(phi)
+    ctx.assemble_p1(rhs_kind=D.RHS_3XY_MINUS_X3, lc=(1.0, 1.0, m.h))
+    g = ctx.csr()
+    return sp.csr_matrix((g["comb"], g["colind"], g["rowptr"])), g["rhs"]
+
+
+def check(ctx, M, b, tol, **kw):
+    M = M.tocsr()
+    M.sort_indices()
+    A = ctx.csr_create(M.indptr, M.indices, M.data)
+    x, it, res, ok = ctx.pcg(A, b, tol=tol, precision=D.FP32_IR, **kw)
+    A.close()
+    assert ok and res <= tol and np.linalg.norm(b - M @ x) <= 1.01 * tol * np.linalg.norm(b)
+    return x, it
+
+
+@pytest.mark.parametrize("rows", [0, 100, 512, 700, 1500, 2048, 3000])
+def test_rows_per_block(ctx, rows):
+    print(f"[gpu mixed pcg] {rows} rows per block", flush=True)
+    M, b = assembled(ctx, 48)
+    ctx.tune("pcg_rows_per_block", rows)
+    try:
+        x, it = check(ctx, M, b, 1e-8)
+        assert np.array_equal(check(ctx, M, b, 1e-8)[0], x)
+        ctx.tune("coherent_exchange", 0)
+        y, it0 = check(ctx, M, b, 1e-8)
+    finally:
+        ctx.tune("pcg_rows_per_block", 0)
+        ctx.tune("coherent_exchange", 2)
+    assert np.linalg.norm(x - y) <= 1e-6 * np.linalg.norm(y) and it <= 1.2 * it0 + 20
+
+
+def test_sizes_and_tolerances(ctx):
+    print("[gpu mixed pcg] sizes", flush=True)
+    rng = np.random.default_rng(2)
+    for n in (1, 2, 63, 257, 513, 2999):
+        M = sp.diags([np.full(n, 4.0), np.full(n - 1, -1.0), np.full(n - 1, -1.0)], [0, 1, -1], format="csr")
+        M = M + sp.diags(rng.uniform(0.1, 1.0, n))
+        b = rng.normal(size=n)
+        for tol in (1e-3, 1e-6, 1e-12):
+            check(ctx, M, b, tol)
+        check(ctx, M, b, 1e-8, x0=rng.normal(size=n))
+    for n, tol in ((16, 1e-10), (33, 1e-6), (64, 1e-12)):
+        M, b = assembled(ctx, n)
+        check(ctx, M, b, tol)
+    # rows longer than a block's LDS holds: the memory form
+    M = sp.random(6000, 6000, density=0.02, random_state=3, format="csr")
+    M = M + M.T + sp.diags(np.full(6000, 200.0))
+    check(ctx, M, rng.normal(size=6000), 1e-8)
