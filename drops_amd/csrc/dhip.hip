@@ -134,6 +134,10 @@ static void derive_tables(Tables &T) {
             const int a = r < 4 ? T.lat_t[t][r] : T.edge_ab[T.sub_edge[t][r - 4]][0];
             const int b = r < 4 ? a : T.edge_ab[T.sub_edge[t][r - 4]][1];
             T.root_ends[t][r] = (uint8_t)(a | b << 4);
+            uint32_t w = T.root_ends[t][r];
+            for (int c = 0; c < 4; ++c)
+                w |= (uint32_t)T.lat_b2[a][c] << (8 + 2 * c) | (uint32_t)T.lat_b2[b][c] << (16 + 2 * c);
+            T.root_word[t][r] = w;
         }
     // P2 dof (vertices 0-3, edges 0-5) -> lattice vertex
     for (int l = 0; l < 10; ++l) {

@@ -39,6 +39,7 @@ struct Tables {
     int8_t rp_bnd[81];         // facet lies in a face of the sub-tet
     uint32_t rp_word[81];      // triangles | boundary << 2 | roots << 4 (4 bits each, triangle major)
     uint8_t root_ends[8][10];  // sub-tet and root -> lattice end points a | b << 4 (a vertex: itself twice)
+    uint32_t root_word[8][10]; // root_ends and the end points' barycentrics x 2: a | b << 4 | a's (2 bits each) << 8 | b's << 16
     int8_t lat_of_p2[10];      // lattice vertex of P2 dof (vertices, edges)
     int8_t inc[8][6];          // local index of corner delta in Kuhn tet k (-1 if absent)
     int8_t slot[6][4][4];      // neighbour slot 0..14 of (k, row vertex, col vertex)

@@ -35,7 +35,8 @@ constexpr int LOC2_MASS = 0, LOC2_LB = 100, LOC2_STAB = 200, LOC2_RHS = 300, LOC
 // row builder's lanes read a tet's row of one operator as consecutive doubles)
 __device__ __forceinline__ int64_t loc2(int e, int64_t c) { return c * LOC2_N + e; }
 constexpr int P2_MAXF = 16;
-constexpr int P2_CHUNK = 64;
+// points staged at a time: six facets' 42 points in one go, and eight waves' LDS on a CU (64: six waves)
+constexpr int P2_CHUNK = 48;
 
 // FE_P2CL::H0..H9 (num/fe.h:287-296): vertices l(2l-1), edges 4 l_a l_b
 __device__ __forceinline__ void p2_basis(const double p[4], double h[10]) {
@@ -84,44 +85,75 @@ struct LocalP2Args {
 struct P2Shared {
     double vb[P2_MAXF][3][4];
     double af[P2_MAXF];
+    double ls[10];
     double h[P2_CHUNK][10];
     double sg[P2_CHUNK][10][3];
     double w[P2_CHUNK];
     double f[P2_CHUNK];
     double U[15][10];
     double n5[15][3];   // P2 level-set unit normal at the 15 volume points
+    double G1[4][3];    // gradients of the barycentric coordinates
     int nf;
 };
 
 // Patch facets of the tet (sub-tet lt, triangle tr, in the order of make_patch) into sh.vb / sh.af,
 // lanes 0..nf-1 one facet each.  Returns the facet count, or -1 when a sub-tet lies entirely in
-// the zero level set (the reference's "full body" error).  Uniform over the wave.
+// the zero level set (the reference's "full body" error).  Uniform over the tet's lanes (a wave or a part of one).
+// Every lane lists the facets (2 lt + triangle, four bits each) from the sign masks and takes its own; the
+// level-set values a facet needs differ from lane to lane and are read from LDS.
 template <class Shared>
 __device__ inline int p2_patch_facets(Shared &sh, const double X[4][3], const double ls[10], int lane) {
-    int ntri[8], nf = 0;
+    uint32_t pos = 0, neg = 0;
+#pragma unroll
+    for (int l = 0; l < 10; ++l) {
+        pos |= ls[l] > 0. ? 1u << l : 0u;
+        neg |= ls[l] < 0. ? 1u << l : 0u;
+        if (lane == 0) sh.ls[l] = ls[l];
+    }
+    uint64_t pids = 0, list = 0;
+    int nf = 0;
     bool zero_body = false;
 #pragma unroll
     for (int lt = 0; lt < 8; ++lt) {
-        int s[4];
+        int pid = 40, p3 = 1;
+        uint32_t any = 0;
 #pragma unroll
-        for (int q = 0; q < 4; ++q) s[q] = sgn(ls[c_tab.lat_t[lt][q]]);
-        if (!s[0] && !s[1] && !s[2] && !s[3]) zero_body = true;
-        ntri[lt] = c_tab.rp_size[s[0] + 3 * s[1] + 9 * s[2] + 27 * s[3] + 40];
-        nf += ntri[lt];
+        for (int q = 0; q < 4; ++q) {
+            const int lv = c_tab.lat_t[lt][q];
+            const uint32_t p = (pos >> lv) & 1u, n = (neg >> lv) & 1u;
+            pid += p3 * ((int)p - (int)n);
+            any |= p | n;
+            p3 *= 3;
+        }
+        zero_body |= any == 0;
+        const int ntri = c_tab.rp_size[pid];
+        pids |= (uint64_t)pid << (7 * lt);
+        if (ntri > 0) list |= (uint64_t)(2 * lt) << (4 * nf++);
+        if (ntri > 1) list |= (uint64_t)(2 * lt + 1) << (4 * nf++);
     }
+    wave_sync_lds();
     if (zero_body) return -1;
     if (lane < nf) {
-        int lt = 0, tr = lane;
-        while (tr >= ntri[lt]) tr -= ntri[lt++];
-        int s[4];
-#pragma unroll
-        for (int q = 0; q < 4; ++q) s[q] = sgn(ls[c_tab.lat_t[lt][q]]);
-        const int pid = s[0] + 3 * s[1] + 9 * s[2] + 27 * s[3] + 40;
+        const int e4 = (int)(list >> (4 * lane)) & 15, lt = e4 >> 1, tr = e4 & 1;
+        const uint32_t w = c_tab.rp_word[(pids >> (7 * lt)) & 127];
         double vb[3][4];
-        facet_vertices(ls, lt, pid, tr, vb);
+#pragma unroll
+        for (int j = 0; j < 3; ++j) {
+            const int rep = (w >> (4 + 12 * tr + 4 * j)) & 15;
+            const uint32_t rw = c_tab.root_word[lt][rep];
+            double ba[4], bb[4];
+#pragma unroll
+            for (int cc = 0; cc < 4; ++cc) {
+                ba[cc] = 0.5 * (double)((rw >> (8 + 2 * cc)) & 3u);
+                bb[cc] = 0.5 * (double)((rw >> (16 + 2 * cc)) & 3u);
+            }
+            const double va = sh.ls[rw & 15], alpha = va / (va - sh.ls[(rw >> 4) & 15]);
+#pragma unroll
+            for (int cc = 0; cc < 4; ++cc) vb[j][cc] = rep < 4 ? ba[cc] : (1.0 - alpha) * ba[cc] + alpha * bb[cc];
+        }
         double absdet, nrm[3];
         facet_qr(X, vb, absdet, nrm);
-        double af = c_tab.rp_bnd[pid] ? 0.5 : 1.;
+        double af = (w & 4) ? 0.5 : 1.;
         af *= absdet;
 #pragma unroll
         for (int j = 0; j < 3; ++j)
@@ -139,7 +171,7 @@ __device__ inline void p2_stage_points(P2Shared &sh, int base, int nq, int lane,
                                        const double G1[4][3], const double v[10], int rhs_kind, double rhs_p0,
                                        const double *fvals = nullptr) {
     const int q = base + lane;
-    if (q >= nq) return;
+    if (q >= nq || lane >= P2_CHUNK) return;
     const int f = q / 7, i = q - 7 * (q / 7);
     double nb[4];
 #pragma unroll
@@ -174,6 +206,12 @@ __device__ inline void p2_stage_points(P2Shared &sh, int base, int nq, int lane,
     sh.f[lane] = fv;
 }
 
+// One wave per cut tet.  Bound by the chain of short phases in it (facets, points, pair sums, normals), each
+// waiting on the one before, with two waves a SIMD to hide it: 221 registers and 19.1 KiB of LDS both allow
+// two (168 registers for three spill 49).  What a lane picks by its own index -- a facet's level-set values, a
+// basis function's vertices -- comes from LDS or packed words: picked from registers it was a chain of selects.
+// The load and the squared basis functions ride in the pair sums (they took a loop of their own in ten lanes).
+// 96^3 torus: 645 -> 386 us, of it 200 for the facets, the joined loop and the third more waves, 58 for U.
 __global__ void __launch_bounds__(64) k_local_p2(LocalP2Args a) {
     __shared__ P2Shared sh;
     const int64_t c = blockIdx.x;
@@ -203,7 +241,8 @@ __global__ void __launch_bounds__(64) k_local_p2(LocalP2Args a) {
     // ---- composite Quad5 surface integrals ----
     int pi = 0, pj = 0;
     pair_of(lane < 55 ? lane : 0, pi, pj);
-    double am = 0., al = 0., hat = 0., rh = 0.;
+    // a diagonal pair's lane also sums its node's load; its mass integral is the squared basis function's
+    double am = 0., al = 0., rh = 0.;
     const int nq = 7 * nf;
     for (int base = 0; base < nq; base += P2_CHUNK) {
         p2_stage_points(sh, base, nq, lane, X, G1, v, a.rhs_kind, a.rhs_p0,
@@ -211,17 +250,12 @@ __global__ void __launch_bounds__(64) k_local_p2(LocalP2Args a) {
         __syncthreads();
         const int cnt = nq - base < P2_CHUNK ? nq - base : P2_CHUNK;
         if (lane < 55) {
+#pragma unroll 7
             for (int k = 0; k < cnt; ++k) {
-                const double w = sh.w[k];
-                am += w * (sh.h[k][pj] * sh.h[k][pi]);
+                const double w = sh.w[k], hi = sh.h[k][pi];
+                am += w * (sh.h[k][pj] * hi);
                 al += w * dot3(sh.sg[k][pj], sh.sg[k][pi]);
-            }
-        }
-        if (lane < 10) {
-            for (int k = 0; k < cnt; ++k) {
-                const double w = sh.w[k];
-                hat += w * (sh.h[k][lane] * sh.h[k][lane]);
-                if (a.rhs_kind != DHIP_RHS_NONE) rh += w * (sh.f[k] * sh.h[k][lane]);
+                if (a.rhs_kind != DHIP_RHS_NONE) rh += w * (sh.f[k] * hi);
             }
         }
         __syncthreads();
@@ -229,17 +263,32 @@ __global__ void __launch_bounds__(64) k_local_p2(LocalP2Args a) {
 
     // ---- normal-gradient stabilisation: U[q][d] = n(x_q) . grad h_d(x_q), Quad5 volume rule ----
     // (the normal once per point, then one lane per (point, basis function))
+    // (U's lane takes its own basis function's vertices: the gradients come from LDS, p2_grad_one's sums)
     if (lane < 15) {
         double n3[3];
         p2_unit_normal(v, c_tab.v5n[lane], G1, n3);
 #pragma unroll
         for (int cc = 0; cc < 3; ++cc) sh.n5[lane][cc] = n3[cc];
     }
+    if (lane == 15) {
+#pragma unroll
+        for (int d = 0; d < 4; ++d)
+#pragma unroll
+            for (int cc = 0; cc < 3; ++cc) sh.G1[d][cc] = G1[d][cc];
+    }
     __syncthreads();
-    for (int t = lane; t < 150; t += 64) {
-        const int q = t / 10, d = t - 10 * (t / 10);
+#pragma unroll
+    for (int r = 0; r < 3; ++r) {
+        const int t = min(lane + 64 * r, 149), q = t / 10, d = t - 10 * (t / 10);
+        // vertices a, b of basis function d (a = b = d at a vertex), four bits each from d = 0 up
+        const int va = (int)(0x2101003210ull >> (4 * d)) & 3, vb = (int)(0x3332213210ull >> (4 * d)) & 3;
+        const double pa = c_tab.v5n[q][va], pb = c_tab.v5n[q][vb];
         double g[3];
-        p2_grad_one(d, c_tab.v5n[q], G1, g);
+#pragma unroll
+        for (int cc = 0; cc < 3; ++cc) {
+            const double ga = sh.G1[va][cc], gb = sh.G1[vb][cc];
+            g[cc] = d < 4 ? (4.0 * pa - 1.0) * ga : 4.0 * pb * ga + 4.0 * pa * gb;
+        }
         sh.U[q][d] = dot3(sh.n5[q], g);
     }
     __syncthreads();
@@ -261,9 +310,9 @@ __global__ void __launch_bounds__(64) k_local_p2(LocalP2Args a) {
         L[loc2(LOC2_STAB + e1, c)] = st;
         L[loc2(LOC2_STAB + e2, c)] = st;
     }
-    if (lane < 10) {
-        L[loc2(LOC2_RHS + lane, c)] = rh;
-        L[loc2(LOC2_HAT + lane, c)] = hat;
+    if (lane < 55 && pi == pj) {
+        L[loc2(LOC2_RHS + pi, c)] = rh;
+        L[loc2(LOC2_HAT + pi, c)] = am;
     }
     if (lane == 0) a.flags[c] = 1;
 }
@@ -277,6 +326,7 @@ constexpr int HAT_TPW = 4;
 struct HatShared {
     double vb[P2_MAXF][3][4];
     double af[P2_MAXF];
+    double ls[10];
     double h[16][10];
     double w[16];
     int nq;
