@@ -155,7 +155,8 @@ struct QQShared {
     double af[2];          // (boundary ? 0.5 : 1) |det| of the facet
     double nrm[2][3];      // facet normals Q e3
     double U[2][3][2];     // Q e1, Q e2 of the facet QR
-    double w[14], ad[14], f[14], H[14][10], Gq[14][10][3];
+    double w[14], ad[14], f[14];
+    double H[7][10], Gq[7][10][3];   // one facet's points at a time
     int nf;
 };
 
@@ -252,6 +253,7 @@ __device__ inline bool qq_base_point(const QQShared &s, const QQParams &P, const
     double x[4] = {f.xcur[0], f.xcur[1], f.xcur[2], f.xcur[3]};
     const double min_step_length = 1e-7;
     for (int iter = 0;; ++iter) {
+        asm volatile("" ::: "memory");   // the tet's values stay in LDS: hoisted out of the loop they fill the registers
         qq_set_point(s, f, x);
         const double normF = sqrt(qq_dot4(f.F, f.F));
         if (iter >= P.maxiter || normF < P.tol) break;
@@ -296,6 +298,7 @@ __device__ inline bool qq_base_point(const QQShared &s, const QQParams &P, const
             double xt[4];
 #pragma unroll
             for (int i = 0; i < 4; ++i) xt[i] = x[i] - l * dx[i];
+            asm volatile("" ::: "memory");
             qq_set_point(s, f, xt);
             if (sqrt(qq_dot4(f.F, f.F)) < normF + armijo_slope * l) break;
         }
@@ -660,19 +663,19 @@ __global__ void __launch_bounds__(128) k_recovered_gradient(RecGradArgs a) {
     for (int c = 0; c < 3; ++c) a.out[3 * j + c] = g[c];
 }
 
-// mass and Laplace-Beltrami sums of pair (pi, pj) over points k0 .. k0 + 6, added to am, al in point order
+// mass and Laplace-Beltrami sums of pair (pi, pj) over points k0 .. k0 + 6 (the facet staged in H, Gq), added to am, al in point order
 __device__ __forceinline__ void qq_pair7(const QQShared &S, int k0, int pi, int pj, double &am, double &al) {
     double w[7], ad[7], hj[7], hi[7], gj[7][3], gi[7][3];
 #pragma unroll
     for (int k = 0; k < 7; ++k) {
         w[k] = S.w[k0 + k];
         ad[k] = S.ad[k0 + k];
-        hj[k] = S.H[k0 + k][pj];
-        hi[k] = S.H[k0 + k][pi];
+        hj[k] = S.H[k][pj];
+        hi[k] = S.H[k][pi];
 #pragma unroll
         for (int c = 0; c < 3; ++c) {
-            gj[k][c] = S.Gq[k0 + k][pj][c];
-            gi[k][c] = S.Gq[k0 + k][pi][c];
+            gj[k][c] = S.Gq[k][pj][c];
+            gi[k][c] = S.Gq[k][pi][c];
         }
     }
 #pragma unroll
@@ -685,7 +688,13 @@ __device__ __forceinline__ void qq_pair7(const QQShared &S, int k0, int pi, int 
 
 constexpr int QQ_TPW = 4;   // cut tets per wave (16 lanes each: a tet has at most 14 quadrature points)
 
-__global__ void __launch_bounds__(64) k_local_p2qq(LocalP2QQArgs a) {
+// Bound by the latency of each point's Newton iteration (a chain of dependent FP64 operations, square roots and
+// divisions in 7 or 14 of 16 lanes), so by how many waves a SIMD holds.  Left to itself the compiler lifts the
+// tet's 120 gradient and 30 recovered values out of the iteration: 512 registers, one wave.  The iteration reads
+// them from LDS again (the memory clobbers there), and H and Gq hold one facet at a time: 256 registers (30 of
+// the prologue's spill) and 18.2 KiB of LDS, two waves a SIMD.  128^3 sphere: 686 -> 500 us, of it 626 with the
+// registers alone, LDS then holding five waves on a CU.
+__global__ void __launch_bounds__(64, 2) k_local_p2qq(LocalP2QQArgs a) {
     __shared__ QQShared sh[QQ_TPW];
     const int lane = threadIdx.x, t = lane >> 4, j = lane & 15;
     const int64_t c = (int64_t)blockIdx.x * QQ_TPW + t;
@@ -824,9 +833,9 @@ __global__ void __launch_bounds__(64) k_local_p2qq(LocalP2QQArgs a) {
     }
     // ---- one quadrature point per lane of the tet's group ----
     const int nq = work ? 7 * nf : 0;
+    const int f = j / 7, qi = j - 7 * (j / 7);
+    double nb[4], Wi[3][3];
     if (j < nq) {
-        const int f = j / 7, qi = j - 7 * (j / 7);
-        double nb[4];
 #pragma unroll
         for (int cc = 0; cc < 4; ++cc) {
             double sv = s.vb[f][0][cc] * c_tab.q5n[qi][0];
@@ -874,7 +883,6 @@ __global__ void __launch_bounds__(64) k_local_p2qq(LocalP2QQArgs a) {
             if (!W.prepare()) {
                 bad = true;
             } else {
-                double Wi[3][3];
 #pragma unroll
                 for (int jj = 0; jj < 3; ++jj) {
                     double e[3] = {0., 0., 0.};
@@ -883,22 +891,6 @@ __global__ void __launch_bounds__(64) k_local_p2qq(LocalP2QQArgs a) {
 #pragma unroll
                     for (int r = 0; r < 3; ++r) Wi[r][jj] = e[r];
                 }
-                const double nf3[3] = {s.nrm[f][0], s.nrm[f][1], s.nrm[f][2]};
-#pragma unroll
-                for (int i = 0; i < 10; ++i) {
-                    double g[3], tt[3], r[3];
-                    qq_p1v(s, i, nb, g);
-                    const double d = nf3[0] * g[0] + nf3[1] * g[1] + nf3[2] * g[2];
-#pragma unroll
-                    for (int cc = 0; cc < 3; ++cc) tt[cc] = g[cc] - d * nf3[cc];
-                    qq_mv3(Wi, tt, r);
-#pragma unroll
-                    for (int cc = 0; cc < 3; ++cc) s.Gq[j][i][cc] = r[cc];
-                }
-                double h[10];
-                p2_basis(nb, h);
-#pragma unroll
-                for (int i = 0; i < 10; ++i) s.H[j][i] = h[i];
                 double fv = 0.;
                 if (a.pts) {
                     double y[3];
@@ -922,42 +914,65 @@ __global__ void __launch_bounds__(64) k_local_p2qq(LocalP2QQArgs a) {
     }
     if (a.pts) return;   // points mode: the base points only
     // ---- contractions in the composite order: per tet 55 pairs (i >= j) and 10 load entries ----
-    for (int task = lane; task < QQ_TPW * 65; task += 64) {
-        const int tt = task / 65, r = task - 65 * (task / 65);
+    // A facet at a time: its lanes stage their points' gradients, then every task adds its seven points.
+    constexpr int NTASK = (QQ_TPW * 65 + 63) / 64;
+    double am[NTASK], al[NTASK];   // a load task sums in am
+#pragma unroll
+    for (int u = 0; u < NTASK; ++u) am[u] = al[u] = 0.0;
+#pragma unroll 1
+    for (int fc = 0; fc < 2; ++fc) {
+        if (j < nq && f == fc) {
+            const double nf3[3] = {s.nrm[fc][0], s.nrm[fc][1], s.nrm[fc][2]};
+#pragma unroll
+            for (int i = 0; i < 10; ++i) {
+                double g[3], tt[3], r[3];
+                qq_p1v(s, i, nb, g);
+                const double d = nf3[0] * g[0] + nf3[1] * g[1] + nf3[2] * g[2];
+#pragma unroll
+                for (int cc = 0; cc < 3; ++cc) tt[cc] = g[cc] - d * nf3[cc];
+                qq_mv3(Wi, tt, r);
+#pragma unroll
+                for (int cc = 0; cc < 3; ++cc) s.Gq[qi][i][cc] = r[cc];
+            }
+            double h[10];
+            p2_basis(nb, h);
+#pragma unroll
+            for (int i = 0; i < 10; ++i) s.H[qi][i] = h[i];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int u = 0; u < NTASK; ++u) {
+            const int task = lane + 64 * u, tt = task / 65, r = task - 65 * (task / 65);
+            if (task >= QQ_TPW * 65 || sh[tt].nf <= fc) continue;
+            const QQShared &S = sh[tt];
+            if (r < 55) {
+                int pi = 0, pj = 0;
+                pair_of(r, pi, pj);
+                qq_pair7(S, 7 * fc, pi, pj, am[u], al[u]);
+            } else if (a.rhs_kind != DHIP_RHS_NONE) {
+#pragma unroll
+                for (int k = 0; k < 7; ++k) am[u] += S.w[7 * fc + k] * ((S.ad[7 * fc + k] * S.f[7 * fc + k]) * S.H[k][r - 55]);
+            }
+        }
+        __syncthreads();
+    }
+#pragma unroll
+    for (int u = 0; u < NTASK; ++u) {
+        const int task = lane + 64 * u, tt = task / 65, r = task - 65 * (task / 65);
         const int64_t ct = (int64_t)blockIdx.x * QQ_TPW + tt;
-        const QQShared &S = sh[tt];
-        if (ct >= N || S.nf <= 0) continue;
-        const int nqt = 7 * S.nf;
+        if (task >= QQ_TPW * 65 || ct >= N || sh[tt].nf <= 0) continue;
         if (r < 55) {
             int pi = 0, pj = 0;
             pair_of(r, pi, pj);
-            double am = 0.0, al = 0.0;
-            if (nqt % 7 == 0) {
-                // a facet's seven points at a time: every LDS read of the chunk is issued before the
-                // first sum, which still runs point by point in the composite order
-                for (int k0 = 0; k0 < nqt; k0 += 7) qq_pair7(S, k0, pi, pj, am, al);
-            } else {
-                for (int k = 0; k < nqt; ++k) {
-                    const double w = S.w[k], ad = S.ad[k];
-                    am += w * ((ad * S.H[k][pj]) * S.H[k][pi]);
-                    const double dq = S.Gq[k][pj][0] * S.Gq[k][pi][0] + S.Gq[k][pj][1] * S.Gq[k][pi][1] +
-                                      S.Gq[k][pj][2] * S.Gq[k][pi][2];
-                    al += w * (ad * dq);
-                }
-            }
             const int e1 = pi * 10 + pj, e2 = pj * 10 + pi;
-            L[loc2(LOC2_MASS + e1, ct)] = am;
-            L[loc2(LOC2_MASS + e2, ct)] = am;
-            L[loc2(LOC2_LB + e1, ct)] = al;
-            L[loc2(LOC2_LB + e2, ct)] = al;
+            L[loc2(LOC2_MASS + e1, ct)] = am[u];
+            L[loc2(LOC2_MASS + e2, ct)] = am[u];
+            L[loc2(LOC2_LB + e1, ct)] = al[u];
+            L[loc2(LOC2_LB + e2, ct)] = al[u];
             L[loc2(LOC2_STAB + e1, ct)] = 0.;
             L[loc2(LOC2_STAB + e2, ct)] = 0.;
         } else {
-            const int i = r - 55;
-            double rh = 0.0;
-            if (a.rhs_kind != DHIP_RHS_NONE)
-                for (int k = 0; k < nqt; ++k) rh += S.w[k] * ((S.ad[k] * S.f[k]) * S.H[k][i]);
-            L[loc2(LOC2_RHS + i, ct)] = rh;
+            L[loc2(LOC2_RHS + r - 55, ct)] = am[u];
         }
     }
     if (work && j == 0) a.flags[c] = 1;
