@@ -633,8 +633,8 @@ __global__ void __launch_bounds__(TRAIN_T) k_mlp_train(TrainArgs a) {
 }
 
 // grad[p] = sum over the block slots of part[slot][p] in float64; p = MLP_NPARAM is the loss.  64 columns
-// per block, 16 threads a column that take every 16th slot, added in order: 9 us for 256 slots (one thread a column over the 2,048 slots that
-// 32 samples a block left: 500 us).
+// per block, 16 threads a column that take every 16th slot, added in order: 9 us for 256 slots (one thread a
+// column over the 2,048 slots that 32 samples a block left: 500 us).
 constexpr int MLP_RED_G = 16;
 __global__ void __launch_bounds__(64 * MLP_RED_G) k_mlp_reduce(const float *part, int nslot, double *grad) {
     __shared__ double s[MLP_RED_G][64];
