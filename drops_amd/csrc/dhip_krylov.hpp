@@ -14,6 +14,7 @@
 // them); every other unit sees their declarations.
 
 #include "dhip_common.hpp"
+#include "dhip_txrec.hpp"
 
 #include <type_traits>
 
@@ -2555,7 +2556,7 @@ __global__ void __launch_bounds__(PB) k_pcg_mixed(PcgMixArgs a)
 #endif
 
 // The mixed-precision PCG over tagged records (k_pcg64_tx's arrangement with FP32 inner vectors): r, w and s of a
-// row are one 16-byte record {r, w, s, generation}, a third of the FP64 form's, so that an inner iteration
+// row are one 16-byte record (dhip_txrec.hpp), a third of the FP64 form's, so that an inner iteration
 // waits for one device-coherent load per halo column and one reduction, both under way together; the block's
 // slice, divided by the preconditioner, and its halo are floats in LDS.  Dot products, the residual b - A x and x
 // are FP64 as in k_pcg_mixed, whose two fenced
@@ -2618,17 +2619,17 @@ __global__ void __launch_bounds__(PB) k_pcg_mixed_tx(PcgMixTxArgs a)
         return s;
     };
     auto publish = [&](uint32_t g, int64_t r, float rv, float wv, float sv) {
-        const u32x4 rec = {__float_as_uint(rv), __float_as_uint(wv), __float_as_uint(sv), g};
+        const u32x4 rec = txm_pack<u32x4>(__float_as_uint(rv), __float_as_uint(wv), __float_as_uint(sv), g);
         __builtin_amdgcn_raw_buffer_store_b128(rec, TV.rsrc, (uint32_t)(((g & 1) * a.n + r) * 16), 0, TX_SC1);
     };
     // The halo of generation g: the record of every distinct column not owned by the block, reloaded until
-    // its tag is g (a record is one 128-bit access; its tag word travels with it).
+    // both of its halves are of generation g.
     auto halo = [&](uint32_t g) {
         for (int t = threadIdx.x; t < nu; t += PB) {
             if (U[t] >= r0 && U[t] < r1) continue;
             u32x4 v = tx_load_raw(TV, g, U[t]);
             uint32_t spins = 0;
-            while (v[3] != g) {
+            while (!txm_ready(v, g)) {
                 if (++spins > SPIN_LIMIT) {
                     tbad = true;
                     break;
@@ -2637,7 +2638,7 @@ __global__ void __launch_bounds__(PB) k_pcg_mixed_tx(PcgMixTxArgs a)
                 v = tx_load_raw(TV, g, U[t]);
             }
             XR[t] = __uint_as_float(v[0]);
-            XW[t] = __uint_as_float(v[1]);
+            XW[t] = __uint_as_float(txm_w(v));
             XS[t] = __uint_as_float(v[2]);
         }
     };
