@@ -551,7 +551,7 @@ __device__ __noinline__ void batch_pcg_memory(const BatchArgs &a, int p, BatchSt
                     }
                 }
                 block_sum2<BB>(p_rr2, p_zr2);
-                if (sqrt(p_rr2) <= inner_tolerance(a.tol, resid, a.inner_tol)) break;
+                if (sqrt(p_rr2) <= a.inner_tol) break;
                 const double rho1 = rho;
                 rho = p_zr2;
                 beta = (float)(rho / rho1);
@@ -811,7 +811,7 @@ __device__ __noinline__ void batch_pcg_chip(const BatchArgs &a, int p, BatchStat
         if (total_it >= a.max_iter) { status = 1; break; }
         ++outer;
         const double scale = 1.0 / rnorm;
-        const double inner_tol = inner_tolerance(a.tol, resid, a.inner_tol), inner_tol2 = inner_tol * inner_tol;
+        const double inner_tol2 = a.inner_tol * a.inner_tol;
         // ---- the register rows' entries and vectors ----
         BpF4 val[R][BP_Q];
         BpU2 cc[R][BP_Q];

@@ -2388,15 +2388,6 @@ done:
 //         from d = 0 until |r_in| <= inner_tol or inner_max iterations
 //   update (FP64): x += |r| d
 // ---------------------------------------------------------------------------
-// Relative residual at which an FP32 inner solve stops, from the FP64 relative residual `resid` it starts at:
-// `base`, or what is left to `tol` (half of it, so that the FP64 check passes) where FP32 reaches that too.  With
-// `base` alone a solve to 1e-8 takes a third pass of 1e-4 for a factor of little over one (512 batched problems
-// 36.1 ms with `base`, 28.9 ms with what is left).
-__device__ __forceinline__ double inner_tolerance(double tol, double resid, double base) {
-    const double left = tol / resid;
-    return left >= 0.1 * base ? 0.5 * left : base;
-}
-
 struct PcgMixArgs {
     int64_t n;
     const int32_t *rp, *col;
@@ -2531,7 +2522,7 @@ __global__ void __launch_bounds__(PB) k_pcg_mixed(PcgMixArgs a)
             p_rr2 = block_sum<PB>(p_rr2);
             p_zr2 = block_sum<PB>(p_zr2);
             if (!sync_reduce<PB>(a.slots, ++gen, p_rr2, p_zr2, 0.0, red)) { fail = true; break; }
-            if (sqrt(red[0]) <= inner_tolerance(a.tol, resid, a.inner_tol)) break;
+            if (sqrt(red[0]) <= a.inner_tol) break;
             const double rho1 = rho;
             rho = red[1];
             beta = (float)(rho / rho1);
@@ -2559,10 +2550,9 @@ __global__ void __launch_bounds__(PB) k_pcg_mixed(PcgMixArgs a)
 // row are one 16-byte record (dhip_txrec.hpp), a third of the FP64 form's, so that an inner iteration
 // waits for one device-coherent load per halo column and one reduction, both under way together; the block's
 // slice, divided by the preconditioner, and its halo are floats in LDS.  Dot products, the residual b - A x and x
-// are FP64 as in k_pcg_mixed, whose two fenced
-// reductions cost 7.5 us an inner iteration: a solve at 92 x 84 x 101 cells 8.4 -> 3.0 ms, inner_tolerance's shorter
-// last pass included.  A block whose
-// slice and halo do not fit the LDS makes every block leave with status 3 (the host then runs k_pcg_mixed).
+// are FP64 as in k_pcg_mixed, whose two fenced reductions cost 7.5 us an inner iteration: assembly and solve at
+// 92 x 84 x 101 cells 8.96 -> 4.73 ms.  A block whose slice and halo do not fit the LDS makes every block leave with
+// status 3 (the host then runs k_pcg_mixed).
 struct PcgMixTxArgs {
     int64_t n;
     const int32_t *rp, *col;
@@ -2706,7 +2696,7 @@ __global__ void __launch_bounds__(PB) k_pcg_mixed_tx(PcgMixTxArgs a)
         if (total_it >= a.max_iter) { status = 1; break; }
         ++outer;
         // ---- FP32 inner PCG on A d = r/|r| ----
-        const double scale = 1.0 / rnorm, itol = inner_tolerance(a.tol, resid, a.inner_tol);
+        const double scale = 1.0 / rnorm;
         ++rg;
 #pragma unroll
         for (int k = 0; k < RPT; ++k) {
@@ -2746,7 +2736,7 @@ __global__ void __launch_bounds__(PB) k_pcg_mixed_tx(PcgMixTxArgs a)
                 gamma = red_sh[0];
                 alpha = red_sh[0] / red_sh[1];
             } else {
-                if (sqrt(red_sh[2]) <= itol || it == a.inner_max || total_it == a.max_iter) break;
+                if (sqrt(red_sh[2]) <= a.inner_tol || it == a.inner_max || total_it == a.max_iter) break;
                 const double gamma_new = red_sh[0];
                 beta = gamma_new / gamma;
                 alpha = gamma_new / (red_sh[1] - beta * gamma_new / alpha);

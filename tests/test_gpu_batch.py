@@ -132,6 +132,21 @@ def test_batch_graph_replay_and_tiles(ctx):
     b.close()
 
 
+def test_batch_inner_solves_run_to_the_end(ctx):
+    """To 1e-6 every problem takes two inner solves of 1e-4, which end at 1e-8 (twice that for what the FP32
+    recurrence's residual and the FP64 one differ by; 5e-8 for 42,796 rows, measured 3.3e-8)."""
+    print("[gpu batch] inner solves", flush=True)
+    meshes, phi, off = small_set(12, seed=9)
+    big = KuhnMesh.box(-2.0, 2.0, 80, shift=tuple(5e-5 * np.array([1.0, 2.0, 3.0])))   # the form in memory
+    pb = big.sample_p2(sphere(radius=1.9)).ravel()
+    b = make_batch(ctx, meshes + [big], np.concatenate([phi, pb]), np.concatenate([off, [phi.size]]))
+    b.solve(tol=1e-6)
+    st = b.stats()
+    assert np.all(st["status"] == D.OK) and np.all(st["outer"] == 2) and np.all(st["resid"][:-1] <= 2e-8), st["resid"]
+    assert st["resid"][-1] <= 5e-8, st["resid"]
+    b.close()
+
+
 def test_batch_zero_node_problem_isolated(ctx):
     print("[gpu batch] exact-zero node in one problem", flush=True)
     meshes, phi, off = small_set(4, seed=7)

@@ -47,6 +47,22 @@ def test_rows_per_block(ctx, rows):
     assert np.linalg.norm(x - y) <= 1e-6 * np.linalg.norm(y) and it <= 1.2 * it0 + 20
 
 
+@pytest.mark.parametrize("exchange", [0, 2])
+def test_inner_solves_run_to_the_end(ctx, exchange):
+    """An inner solve runs to 1e-4 whatever the caller's tolerance leaves to do: to 1e-6 two of them, which end at
+    1e-8 and not below 1e-6 (twice that for what the FP32 recurrence's residual and the FP64 one differ by)."""
+    print(f"[gpu mixed pcg] inner solves, exchange {exchange}", flush=True)
+    ctx.tune("coherent_exchange", exchange)
+    try:
+        for n in (16, 48):
+            M, b = assembled(ctx, n)
+            x, _, res, ok = ctx.pcg(ctx.csr_create(M.indptr, M.indices, M.data), b, tol=1e-6, precision=D.FP32_IR)
+            assert ok and res <= 2e-8
+            assert np.linalg.norm(b - M @ x) <= 2.02e-8 * np.linalg.norm(b)
+    finally:
+        ctx.tune("coherent_exchange", 2)
+
+
 def test_sizes_and_tolerances(ctx):
     print("[gpu mixed pcg] sizes", flush=True)
     rng = np.random.default_rng(2)
