@@ -1868,10 +1868,10 @@ int dhip_pcg(dhip_ctx_t *c, const dhip_csr_t *A, int32_t pc, const double *b, do
     } else if (precision == DHIP_FP32_IR) {
         if (pc != DHIP_PC_JACOBI) return set_error(c, DHIP_E_ARG, "FP32 refinement path uses the Jacobi preconditioner");
         SolverResult tres{};
-        tres.i[1] = 3;
+        tres.i[1] = 3;   // (no iterations spent)
         if (c->coherent_exchange >= 2 && rpt <= 4) {
-            // tagged records (cleared first: an earlier solve's tags would match); status 3 with x untouched where a
-            // block's slice and halo exceed its LDS
+            // tagged records (cleared first: an earlier solve's tags would match); status 3 where a block's slice and
+            // halo exceed its LDS (x untouched) or the recurrences did not carry in FP32 (x the best so far)
             DHIP_HIPCHK(c, c->kv[16].ensure((size_t)32 * (n + 1)));
             DHIP_LAUNCH(c, "zero_records", k_zero_u32, blocks_for(8 * n, 256), 256, 0, c->kv[16].as<uint32_t>(),
                         (int)(8 * n));
@@ -1893,13 +1893,14 @@ int dhip_pcg(dhip_ctx_t *c, const dhip_csr_t *A, int32_t pc, const double *b, do
                 DHIP_LAUNCH(c, "csr_to_f32", k_to_f32, blocks_for(A->nnz, KB), KB, 0, A->nnz, A->val, val32);
             for (int k = 6; k < 9; ++k) DHIP_HIPCHK(c, c->kv[k].ensure(sizeof(float) * (n + 1)));
             PcgMixArgs pa{n, A->rowptr, A->col, A->val, diag, val32, db, dx, c->kv[6].as<float>(), c->kv[7].as<float>(),
-                          c->kv[8].as<float>(), c->bar.as<SyncSlot>(), *max_iter, *tol, rel, 1e-4, 400, outs, outd,
-                          outs + 1, outs + 2};
+                          c->kv[8].as<float>(), c->bar.as<SyncSlot>(), *max_iter - tres.i[0], *tol, rel, 1e-4, 400, outs,
+                          outd, outs + 1, outs + 2};
             pa.xcd_map = c->xcd_map;
             const void *ks[5] = {(const void *)k_pcg_mixed<1>, (const void *)k_pcg_mixed<2>, (const void *)k_pcg_mixed<4>,
                                  (const void *)k_pcg_mixed<8>, (const void *)k_pcg_mixed<16>};
             rc = launch_persistent(c, "pcg_mixed", ks, rpt, nb, pa);
             if (rc) return rc;
+            h_iter = tres.i[0];
         }
     } else {
         return set_error(c, DHIP_E_ARG, "unknown precision");
@@ -1909,7 +1910,7 @@ int dhip_pcg(dhip_ctx_t *c, const dhip_csr_t *A, int32_t pc, const double *b, do
     if (where != DHIP_DEVICE && n > 0)
         DHIP_HIPCHK(c, hipMemcpyAsync(x, dx, sizeof(double) * n, hipMemcpyDeviceToHost, c->stream));
     DHIP_HIPCHK(c, hipStreamSynchronize(c->stream));
-    h_iter = res.i[0];
+    h_iter += res.i[0];
     h_status = res.i[1];
     h_outer = res.i[2];
     h_resid = res.resid;

@@ -2551,8 +2551,14 @@ __global__ void __launch_bounds__(PB) k_pcg_mixed(PcgMixArgs a)
 // waits for one device-coherent load per halo column and one reduction, both under way together; the block's
 // slice, divided by the preconditioner, and its halo are floats in LDS.  Dot products, the residual b - A x and x
 // are FP64 as in k_pcg_mixed, whose two fenced reductions cost 7.5 us an inner iteration: assembly and solve at
-// 92 x 84 x 101 cells 8.96 -> 4.73 ms.  A block whose slice and halo do not fit the LDS makes every block leave with
-// status 3 (the host then runs k_pcg_mixed).
+// 92 x 84 x 101 cells 8.96 -> 4.73 ms.
+// Status 3: the host runs k_pcg_mixed from x, with the iterations that are left.  Every block leaves with it where a
+// block's slice and halo do not fit the LDS, and where this form's recurrences do not carry in FP32.  It carries
+// s = A p along and takes (p, A p) as (w, u) - beta gamma / alpha, which cancels where beta is large; on
+// matrices whose condition number is beyond FP32 the difference can come out zero, negative or without a value, where
+// k_pcg_mixed, which forms A p, still converges.  So a pass ends at a step length that is not positive and finite
+// (with d as it was before it) and is the last one here, and so is a pass whose FP64 residual is neither half of the
+// one it started from nor within twice of what the recurrence says.  A pass that made the residual larger is taken back.
 struct PcgMixTxArgs {
     int64_t n;
     const int32_t *rp, *col;
@@ -2667,7 +2673,10 @@ __global__ void __launch_bounds__(PB) k_pcg_mixed_tx(PcgMixTxArgs a)
             di[k] = (float)a.diag[r0 + lr[k]];
         }
     }
-    bool first = true, fail = false;
+    bool first = true, fail = false, broke = false;
+    double before = 0.0, claim = 0.0, xp[RPT];   // the last pass: residual and x it started from, its recurrence's residual
+#pragma unroll
+    for (int k = 0; k < RPT; ++k) xp[k] = own[k] ? xr[k] : 0.0;
     for (;;) {
         // ---- FP64 residual ----
         double p_rr = 0.0, p_bb = 0.0, r64[RPT];
@@ -2686,6 +2695,7 @@ __global__ void __launch_bounds__(PB) k_pcg_mixed_tx(PcgMixTxArgs a)
         if (!sync_reduce<PB>(a.slots, ++gen, p_rr, p_bb, fits ? 0.0 : 1.0, red)) { status = 2; break; }
         if (red[2] != 0.0) { status = 3; break; }
         const double rnorm = sqrt(red[0]);
+        const bool start = first;
         if (first) {
             normb = sqrt(red[1]);
             if (normb == 0.0 || !a.rel) normb = 1.0;
@@ -2693,6 +2703,15 @@ __global__ void __launch_bounds__(PB) k_pcg_mixed_tx(PcgMixTxArgs a)
         }
         resid = rnorm / normb;
         if (resid <= a.tol) { status = 0; break; }
+        if (!start && (broke || !(rnorm <= fmax(0.5 * before, 2.0 * claim)))) {
+            if (!(rnorm <= before)) {
+#pragma unroll
+                for (int k = 0; k < RPT; ++k)
+                    if (own[k]) a.x[r0 + lr[k]] = xp[k];
+            }
+            status = 3;
+            break;
+        }
         if (total_it >= a.max_iter) { status = 1; break; }
         ++outer;
         // ---- FP32 inner PCG on A d = r/|r| ----
@@ -2742,8 +2761,10 @@ __global__ void __launch_bounds__(PB) k_pcg_mixed_tx(PcgMixTxArgs a)
                 alpha = gamma_new / (red_sh[1] - beta * gamma_new / alpha);
                 gamma = gamma_new;
             }
-            ++total_it;
             const float al = (float)alpha, be = (float)beta;
+            broke = !(al > 0.f && al <= 3.402823466e38f);   // the same in every thread of the grid
+            if (broke) break;
+            ++total_it;
             double p_g2 = 0.0, p_d2 = 0.0, p_rr2 = 0.0;
             ++rg;
             ++gen;
@@ -2773,9 +2794,12 @@ __global__ void __launch_bounds__(PB) k_pcg_mixed_tx(PcgMixTxArgs a)
         }
         if (fail) { status = 2; break; }
         // ---- FP64 refinement update, published for the next outer residual ----
+        before = rnorm;
+        claim = rnorm * sqrt(red_sh[2]);
 #pragma unroll
         for (int k = 0; k < RPT; ++k) {
             if (!own[k]) continue;
+            xp[k] = xr[k];
             xr[k] += rnorm * (double)dv[k];
             a.x[r0 + lr[k]] = xr[k];
         }

@@ -12,11 +12,11 @@ from drops_amd import dhip as D
 pytestmark = pytest.mark.gpu
 
 
-def assembled(ctx, n):
+def assembled(ctx, n, lc=None):
     m, phi = cases.c1_sphere(n)
     ctx.mesh(m)
     ctx.levelset(phi)
-    ctx.assemble_p1(rhs_kind=D.RHS_3XY_MINUS_X3, lc=(1.0, 1.0, m.h))
+    ctx.assemble_p1(rhs_kind=D.RHS_3XY_MINUS_X3, lc=lc or (1.0, 1.0, m.h))
     g = ctx.csr()
     return sp.csr_matrix((g["comb"], g["colind"], g["rowptr"])), g["rhs"]
 
@@ -80,3 +80,46 @@ def test_sizes_and_tolerances(ctx):
     M = sp.random(6000, 6000, density=0.02, random_state=3, format="csr")
     M = M + M.T + sp.diags(np.full(6000, 200.0))
     check(ctx, M, rng.normal(size=6000), 1e-8)
+
+
+def ill_conditioned(rng):
+    """A dense symmetric positive definite matrix with a condition number up to 1e8, half of them scaled by
+    rows and columns over six decades, and a right-hand side."""
+    n, k = int(rng.choice([8, 16, 40])), 10.0 ** rng.uniform(4, 8)
+    Q, _ = np.linalg.qr(rng.normal(size=(n, n)))
+    ev = np.exp(rng.uniform(0.0, np.log(k), n))
+    A = (Q * ev) @ Q.T
+    if rng.random() < 0.5:
+        s = 10.0 ** rng.uniform(-3, 3, n)
+        A = s[:, None] * A * s[None, :]
+    A = (A + A.T) / 2
+    return sp.csr_matrix(A), rng.normal(size=n) if rng.random() < 0.5 else A @ rng.normal(size=n)
+
+
+@pytest.mark.parametrize("seed", [11, 12])
+def test_condition_beyond_fp32(ctx, seed):
+    """Where the single-reduction recurrences lose the step length in FP32 the solve goes on in the two-reduction
+    form: what converges there (the fenced exchange runs it from the start) converges, to the same tolerance and
+    within twice the iterations and two passes of 400.  Dense matrices, and operators without stabilisation."""
+    print(f"[gpu mixed pcg] condition numbers beyond FP32, seed {seed}", flush=True)
+    rng = np.random.default_rng(seed)
+    systems = [ill_conditioned(rng) for _ in range(80)]
+    systems += [assembled(ctx, 32, lc) for lc in ((1.0, 1.0, 0.0), (1.0, 0.0, 0.0), (1e-3, 1.0, 0.0))]
+    worse = converged = 0
+    for M, b in systems:
+        A = ctx.csr_create(M.indptr, M.indices, M.data)
+        got = {}
+        for exchange in (0, 2):
+            ctx.tune("coherent_exchange", exchange)
+            try:
+                got[exchange] = ctx.pcg(A, b, tol=1e-8, max_iter=8000, precision=D.FP32_IR, raise_on_fail=False)
+            finally:
+                ctx.tune("coherent_exchange", 2)
+        A.close()
+        (x, it, _, ok), (_, it0, _, ok0) = got[2], got[0]
+        assert np.all(np.isfinite(x)) or not ok0
+        if ok:
+            assert np.linalg.norm(b - M @ x) <= 1.01e-8 * np.linalg.norm(b)
+        converged += ok0
+        worse += bool(ok0 and (not ok or it > 2 * it0 + 800))
+    assert converged >= 50 and worse == 0, (converged, worse)
