@@ -2826,13 +2826,13 @@ static int mlp_features_impl(dhip_mlp *q, const double *const hist[4], int32_t n
 // gradient (double, q->grad) and loss of a minibatch
 static int mlp_grad_impl(dhip_mlp *q, const float *X, const float *T, const int32_t *idx, int64_t B) {
     dhip_ctx *c = q->ctx;
-    // four waves of 16 samples a block, one block per CU at most (the blocks walk the tiles)
+    // 64 samples a block at a time, one block per CU at most (the blocks walk the tiles)
     const int64_t blocks = std::min<int64_t>((B + TSW * TW - 1) / (TSW * TW), c->cu_count);
-    DHIP_HIPCHK(c, q->part.ensure(sizeof(float) * (size_t)blocks * (MLP_NPARAM + 1)));
-    TrainArgs ta{X, T, idx, B, q->theta.as<float>(), q->part.as<float>()};
+    DHIP_HIPCHK(c, q->part.ensure(sizeof(double) * (size_t)blocks * (MLP_NPARAM + 1)));
+    TrainArgs ta{X, T, idx, B, q->theta.as<float>(), q->part.as<double>()};
     DHIP_LAUNCH(c, "mlp_train", k_mlp_train, (unsigned)blocks, TRAIN_T, TRAIN_LDS, ta);
     DHIP_LAUNCH(c, "mlp_reduce", k_mlp_reduce, blocks_for(MLP_NPARAM + 1, 64), 64 * MLP_RED_G, 0,
-                q->part.as<float>(), (int)blocks, q->grad.as<double>());
+                q->part.as<double>(), (int)blocks, q->grad.as<double>());
     return DHIP_OK;
 }
 

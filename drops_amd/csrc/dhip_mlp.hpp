@@ -8,8 +8,8 @@
 //   k_mlp_infer     matrix cores: one wave per 16 DOFs, v_mfma_f32_16x16x32_bf16 for every layer
 //                   (bf16 weights and layer inputs, float32 accumulation); weights staged in LDS.
 //   k_mlp_train     matrix cores: 16 samples per wave, forward with k_mlp_infer's rounding points,
-//                   backward in float32, gradients accumulated in registers over the wave's tiles;
-//                   a block's gradient goes to its own slot (no atomics).
+//                   backward in float32, gradients of at most 32 samples in float32 and their sums in
+//                   float64; a block's gradient goes to its own slot (no atomics).
 //   k_mlp_reduce    gradient = sum of the block slots in slot order; k_mlp_adam the update.
 #pragma once
 
@@ -287,8 +287,8 @@ __global__ void __launch_bounds__(64 * INFER_WAVES) k_mlp_infer(const float *X, 
 // ---------------------------------------------------------------------------------------------
 // training
 //
-// One wave owns 16 samples at a time and keeps them in registers from the forward pass to the last
-// weight gradient; nothing waits for another wave until the block's gradients are added up.
+// One wave owns 16 samples at a time, a block 64, and keeps them in registers from the forward pass to the last
+// weight gradient.
 //   * Products are taken with the units as the matrix rows and the samples as the columns, so a lane
 //     holds units 16 t + 4 q + i (q = lane / 16, i = 0..3) of sample lane % 16, and that register file is
 //     the B operand of the next product when its contraction index is enumerated in the same order: the
@@ -296,14 +296,17 @@ __global__ void __launch_bounds__(64 * INFER_WAVES) k_mlp_infer(const float *X, 
 //   * Forward: bf16 weights and layer inputs, v_mfma_f32_16x16x32_bf16 (as k_mlp_infer).  Backward: the
 //     float32 deltas meet float32 copies of the rounded weights and inputs in v_mfma_f32_16x16x4_f32, so
 //     no operand is rounded further.
-//   * Weight gradients contract over the samples: delta and layer input go through LDS once per layer
-//     (rows of 68 floats: the lanes' four sample rows 4 q + kk lie 16 banks apart), into 160
-//     accumulators that live as long as the wave.
-// A block adds its waves' sums in LDS and writes one slot; k_mlp_reduce adds the slots in float64.
+//   * Weight gradients contract over the block's samples: delta and layer input go through LDS once per layer
+//     (rows of 68 floats: the lanes' four sample rows 4 q + kk lie 16 banks apart) and each wave takes
+//     one tile row of every gradient over all 64 samples, so that its sums are few enough to be kept
+//     in float64.  The matrix cores add 32 samples in float32, which then go into the float64 sums: the error does
+//     not grow with the minibatch.  Two sets of tiles in turn, one barrier a layer: a set is written again only
+//     after the barrier behind its readers.
+// A block's sums go to one float64 slot; k_mlp_reduce adds the slots.
 // Bound by the float32 matrix rate and the tanh evaluations, about 9,500 matrix cycles per 16 samples.
-// At 65,536 samples on 256 CUs 82 us (27 of it the staged weights, the block sums and the launch, 13.5 per
-// tile of a wave); 32 samples a block with every product on the vector units and one slot per 32 samples
-// took 350 us.
+// At 65,536 samples on 256 CUs 90 us (81 with every product of a wave's own samples and its sums over all its tiles
+// in float32: an entry's error was 1e-6 there and 1.5e-5 for 2^20 equal samples, now 5e-7 for any number);
+// 32 samples a block with every product on the vector units and one slot per 32 samples took 350 us.
 constexpr int TW = 4;               // waves per block
 constexpr int TRAIN_T = 64 * TW;    // threads per block
 constexpr int TSW = 16;             // samples per wave and pass
@@ -314,7 +317,7 @@ struct TrainArgs {
     const int32_t *idx;       // minibatch sample ids
     int64_t B;                // minibatch size
     const float *theta;
-    float *part;              // [blocks][MLP_NPARAM + 1] (last: loss)
+    double *part;             // [blocks][MLP_NPARAM + 1] (last: loss)
 };
 
 // bf16 forward weights as A fragments of v_mfma_f32_16x16x32_bf16: [fragment][lane][8].
@@ -325,12 +328,19 @@ struct TrainShared {
     float w2[MLP_H * TLD], w3[MLP_H * TLD];   // rounded weights [out][in] for the backward products
     float w4[MLP_NO * MLP_H];
     float bias[3 * MLP_H + MLP_NO];
-    __align__(16) float dz[TW][TSW * TLD], in[TW][TSW * TLD];
-    __align__(16) float theta[MLP_NPARAM];
+    float dy[MLP_NO][TW * TSW];
+    struct Tiles {
+        __align__(16) float dz[TW][TSW * TLD], in[TW][TSW * TLD];
+    };
+    Tiles tiles0;
+    union {
+        Tiles tiles1;
+        __align__(16) float theta[MLP_NPARAM];   // until the weights are staged
+        double sums[TW][2 * MLP_H + MLP_NO + 1]; // the waves' bias gradients and losses at the end
+    };
 };
-// the waves' gradients at the end take the same LDS
-constexpr size_t TRAIN_LDS = sizeof(TrainShared) > sizeof(float) * TW * (MLP_NPARAM + 1)
-                                 ? sizeof(TrainShared) : sizeof(float) * TW * (MLP_NPARAM + 1);
+constexpr size_t TRAIN_LDS = sizeof(TrainShared);
+static_assert(TRAIN_LDS <= 160 * 1024, "k_mlp_train's LDS");
 
 // weight of out unit n at in unit k (layer 1: k >= 12 is padding; layer 4: n >= 2)
 __device__ inline float train_weight(const float *th, int layer, int n, int k) {
@@ -389,18 +399,10 @@ __global__ void __launch_bounds__(TRAIN_T) k_mlp_train(TrainArgs a) {
     if (t < MLP_NO) sh.bias[3 * MLP_H + t] = theta[MLP_B4 + t];
     __syncthreads();
 
-    floatx4_t g1[4], g2[4][4], g3[4][4], g4[4];   // dW tiles [out tile][in tile]; layer 1's column 12 is its bias
-    float gb2[16], gb3[16], gb4[2] = {0.f, 0.f}, loss = 0.f;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        g1[i] = g4[i] = floatx4_t{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int j = 0; j < 4; ++j) g2[i][j] = g3[i][j] = floatx4_t{0.f, 0.f, 0.f, 0.f};
-    }
-#pragma unroll
-    for (int i = 0; i < 16; ++i) gb2[i] = gb3[i] = 0.f;
+    // the wave's dW tiles: out tile wv of layers 1 (its column 12 is the bias), 2 and 3, in tile wv of layer 4
+    double g1[1][4] = {}, g2[4][4] = {}, g3[4][4] = {}, g4[1][4] = {};
+    double gb2[16] = {}, gb3[16] = {}, gb4[2] = {}, loss = 0.0;   // over the lane's samples
 
-    float *dz = sh.dz[wv], *in = sh.in[wv];
     auto frag = [&](int f) { return *reinterpret_cast<const bf16x8_t *>(&sh.frag[(f * 64 + lane) * 8]); };
     // tanh of a layer's products, in place
     auto activate = [&](float (&h)[4][4], const float *b) {
@@ -436,21 +438,28 @@ __global__ void __launch_bounds__(TRAIN_T) k_mlp_train(TrainArgs a) {
             *reinterpret_cast<floatx4_t *>(&buf[col * TLD + 16 * nt + 4 * q]) = x;
         }
     };
-    // g[nt][kt] += dz^T in over the wave's 16 samples (sample 4 q + kk at step kk)
-    auto weight_grad = [&](floatx4_t (&g)[4][4]) {
+    // g[kt] += A^T B over the block's samples, A(k) the lane's entry of sample row k of the wave's out tile, B(k, kt) of
+    // the layer input's tile kt; 32 samples in float32
+    auto weight_grad = [&](auto &g, auto &&A, auto &&B) {
+        constexpr int NK = sizeof(g) / sizeof(g[0]);
 #pragma unroll
-        for (int kk = 0; kk < 4; ++kk) {
-            float av[4], bv[4];
+        for (int w0 = 0; w0 < TW; w0 += 2) {
+            floatx4_t acc[NK];
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                av[i] = dz[(4 * q + kk) * TLD + 16 * i + col];
-                bv[i] = in[(4 * q + kk) * TLD + 16 * i + col];
-            }
+            for (int kt = 0; kt < NK; ++kt) acc[kt] = floatx4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int nt = 0; nt < 4; ++nt)
+            for (int w = w0; w < w0 + 2; ++w)
 #pragma unroll
-                for (int kt = 0; kt < 4; ++kt)
-                    g[nt][kt] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[nt], bv[kt], g[nt][kt], 0, 0, 0);
+                for (int kk = 0; kk < 4; ++kk) {
+                    const float av = A(w, 4 * q + kk);
+#pragma unroll
+                    for (int kt = 0; kt < NK; ++kt)
+                        acc[kt] = __builtin_amdgcn_mfma_f32_16x16x4f32(av, B(w, 4 * q + kk, kt), acc[kt], 0, 0, 0);
+                }
+#pragma unroll
+            for (int kt = 0; kt < NK; ++kt)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) g[kt][i] += (double)acc[kt][i];
         }
     };
     // delta of the layer below: (W^T d) (1 - h^2), the contraction index n = 16 nt + 4 q + i from d's registers
@@ -472,9 +481,9 @@ __global__ void __launch_bounds__(TRAIN_T) k_mlp_train(TrainArgs a) {
             for (int i = 0; i < 4; ++i) out[kt][i] = acc[kt][i] * (1.f - h[kt][i] * h[kt][i]);
     };
 
-    const int64_t ntile = (a.B + TSW - 1) / TSW;
-    for (int64_t tile = (int64_t)blockIdx.x * TW + wv; tile < ntile; tile += (int64_t)gridDim.x * TW) {
-        const int64_t g = tile * TSW + col;
+    const int64_t ntile = (a.B + TSW * TW - 1) / (TSW * TW);
+    for (int64_t tile = blockIdx.x; tile < ntile; tile += gridDim.x) {   // the same for every wave of the block
+        const int64_t g = tile * (TSW * TW) + TSW * wv + col;
         const int64_t sid = g < a.B ? (int64_t)a.idx[g] : -1;
         // features 8 q .. 8 q + 7 of the lane's sample (12 real ones, zero padding)
         float x0[8];
@@ -517,12 +526,16 @@ __global__ void __launch_bounds__(TRAIN_T) k_mlp_train(TrainArgs a) {
                 const float y = __shfl(d[o], col, 64) + sh.bias[3 * MLP_H + o];
                 const float r = sid >= 0 ? y - tv[o] : 0.f;
                 dy[o] = r / (float)a.B;
-                if (q == 0) loss += 0.5f * r * r;
-                if (q == 0) gb4[o] += dy[o];
+                if (q == 0) {
+                    loss += (double)(0.5f * r * r);
+                    gb4[o] += (double)dy[o];
+                    sh.dy[o][TSW * wv + col] = dy[o];
+                }
             }
         }
         // layer 4: weights and the delta of layer 3
-        store(in, h3, true);
+        TrainShared::Tiles &t0 = sh.tiles0, &t1 = sh.tiles1;
+        store(t0.in[wv], h3, true);
         float d3[4][4], d2[4][4], d1[4][4];
 #pragma unroll
         for (int nt = 0; nt < 4; ++nt)
@@ -531,53 +544,40 @@ __global__ void __launch_bounds__(TRAIN_T) k_mlp_train(TrainArgs a) {
                 const int n = 16 * nt + 4 * q + i;
                 const float v = __fmaf_rn(dy[1], sh.w4[MLP_H + n], dy[0] * sh.w4[n]);
                 d3[nt][i] = v * (1.f - h3[nt][i] * h3[nt][i]);
-                gb3[4 * nt + i] += d3[nt][i];
+                gb3[4 * nt + i] += (double)d3[nt][i];
             }
-        wave_sync_lds();
-#pragma unroll
-        for (int kk = 0; kk < 4; ++kk) {
-            const float e0 = __shfl(dy[0], 4 * q + kk, 64), e1 = __shfl(dy[1], 4 * q + kk, 64);
-            const float av = col == 0 ? e0 : col == 1 ? e1 : 0.f;
-#pragma unroll
-            for (int kt = 0; kt < 4; ++kt)
-                g4[kt] = __builtin_amdgcn_mfma_f32_16x16x4f32(av, in[(4 * q + kk) * TLD + 16 * kt + col], g4[kt], 0, 0, 0);
-        }
-        wave_sync_lds();
+        __syncthreads();
+        weight_grad(g4, [&](int w, int k) { return col < MLP_NO ? sh.dy[col < MLP_NO ? col : 0][TSW * w + k] : 0.f; },
+                    [&](int w, int k, int) { return t0.in[w][k * TLD + 16 * wv + col]; });
         // layer 3
-        store(in, h2, true);
-        store(dz, d3, false);
-        wave_sync_lds();
-        weight_grad(g3);
-        wave_sync_lds();
+        store(t1.in[wv], h2, true);
+        store(t1.dz[wv], d3, false);
         backward(sh.w3, d3, h2, d2);
 #pragma unroll
-        for (int e = 0; e < 16; ++e) gb2[e] += d2[e >> 2][e & 3];
+        for (int e = 0; e < 16; ++e) gb2[e] += (double)d2[e >> 2][e & 3];
+        __syncthreads();
+        weight_grad(g3, [&](int w, int k) { return t1.dz[w][k * TLD + 16 * wv + col]; },
+                    [&](int w, int k, int kt) { return t1.in[w][k * TLD + 16 * kt + col]; });
         // layer 2
-        store(in, h1, true);
-        store(dz, d2, false);
-        wave_sync_lds();
-        weight_grad(g2);
-        wave_sync_lds();
+        store(t0.in[wv], h1, true);
+        store(t0.dz[wv], d2, false);
         backward(sh.w2, d2, h1, d1);
+        __syncthreads();
+        weight_grad(g2, [&](int w, int k) { return t0.dz[w][k * TLD + 16 * wv + col]; },
+                    [&](int w, int k, int kt) { return t0.in[w][k * TLD + 16 * kt + col]; });
         // layer 1: inputs 0..11, a one in column 12 for the bias
-        store(dz, d1, false);
+        store(t1.dz[wv], d1, false);
         if (q < 2) {
 #pragma unroll
-            for (int x = 0; x < 8; ++x) in[col * TLD + 8 * q + x] = 8 * q + x == MLP_NF ? 1.f : x0[x];
+            for (int x = 0; x < 8; ++x) t1.in[wv][col * TLD + 8 * q + x] = 8 * q + x == MLP_NF ? 1.f : x0[x];
         }
-        wave_sync_lds();
-#pragma unroll
-        for (int kk = 0; kk < 4; ++kk) {
-            const float bv = in[(4 * q + kk) * TLD + col];
-#pragma unroll
-            for (int nt = 0; nt < 4; ++nt)
-                g1[nt] = __builtin_amdgcn_mfma_f32_16x16x4f32(dz[(4 * q + kk) * TLD + 16 * nt + col], bv, g1[nt], 0, 0, 0);
-        }
-        wave_sync_lds();
+        __syncthreads();
+        weight_grad(g1, [&](int w, int k) { return t1.dz[w][k * TLD + 16 * wv + col]; },
+                    [&](int w, int k, int) { return t1.in[w][k * TLD + col]; });
     }
 
-    // sums over the 16 lanes that share units
-    auto over_samples = [&](float v) {
+    // sums over the 16 lanes that share units, then over the waves in their order
+    auto over_samples = [&](double v) {
 #pragma unroll
         for (int o = 8; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
         return v;
@@ -591,57 +591,52 @@ __global__ void __launch_bounds__(TRAIN_T) k_mlp_train(TrainArgs a) {
     gb4[1] = over_samples(gb4[1]);
     loss = over_samples(loss);
     __syncthreads();
-    // every wave's gradient to LDS (over the weights and tiles), then their sum in wave order
-    float *G = reinterpret_cast<float *>(train_lds) + wv * (MLP_NPARAM + 1);
+    if (col == 0) {
 #pragma unroll
-    for (int nt = 0; nt < 4; ++nt)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int n = 16 * nt + 4 * q + i;
-            if (col < MLP_NF) G[MLP_W1 + n * MLP_NF + col] = g1[nt][i];
-            else if (col == MLP_NF) G[MLP_B1 + n] = g1[nt][i];
-#pragma unroll
-            for (int kt = 0; kt < 4; ++kt) {
-                G[MLP_W2 + n * MLP_H + 16 * kt + col] = g2[nt][kt][i];
-                G[MLP_W3 + n * MLP_H + 16 * kt + col] = g3[nt][kt][i];
-            }
-            if (col == 0) {
-                G[MLP_B2 + n] = gb2[4 * nt + i];
-                G[MLP_B3 + n] = gb3[4 * nt + i];
-            }
+        for (int e = 0; e < 16; ++e) {
+            const int n = 16 * (e >> 2) + 4 * q + (e & 3);
+            sh.sums[wv][n] = gb2[e];
+            sh.sums[wv][MLP_H + n] = gb3[e];
         }
-    if (q == 0) {
-#pragma unroll
-        for (int kt = 0; kt < 4; ++kt)
-#pragma unroll
-            for (int o = 0; o < MLP_NO; ++o) G[MLP_W4 + o * MLP_H + 16 * kt + col] = g4[kt][o];
     }
     if (lane == 0) {
-        G[MLP_B4] = gb4[0];
-        G[MLP_B4 + 1] = gb4[1];
-        G[MLP_NPARAM] = loss;
+        sh.sums[wv][2 * MLP_H] = gb4[0];
+        sh.sums[wv][2 * MLP_H + 1] = gb4[1];
+        sh.sums[wv][2 * MLP_H + 2] = loss;
+    }
+    double *P = a.part + (size_t)blockIdx.x * (MLP_NPARAM + 1);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int n = 16 * wv + 4 * q + i;
+        if (col < MLP_NF) P[MLP_W1 + n * MLP_NF + col] = g1[0][i];
+        else if (col == MLP_NF) P[MLP_B1 + n] = g1[0][i];
+#pragma unroll
+        for (int kt = 0; kt < 4; ++kt) {
+            P[MLP_W2 + n * MLP_H + 16 * kt + col] = g2[kt][i];
+            P[MLP_W3 + n * MLP_H + 16 * kt + col] = g3[kt][i];
+        }
+        if (q == 0 && i < MLP_NO) P[MLP_W4 + i * MLP_H + 16 * wv + col] = g4[0][i];
     }
     __syncthreads();
-    const float *W = reinterpret_cast<const float *>(train_lds);
-    float *P = a.part + (size_t)blockIdx.x * (MLP_NPARAM + 1);
-    for (int e = t; e < MLP_NPARAM + 1; e += TRAIN_T) {
-        float v = W[e];
+    if (t < 2 * MLP_H + MLP_NO + 1) {
+        double v = sh.sums[0][t];
 #pragma unroll
-        for (int w = 1; w < TW; ++w) v += W[w * (MLP_NPARAM + 1) + e];
-        P[e] = v;
+        for (int w = 1; w < TW; ++w) v += sh.sums[w][t];
+        P[t < MLP_H ? MLP_B2 + t : t < 2 * MLP_H ? MLP_B3 + t - MLP_H : t < 2 * MLP_H + MLP_NO ? MLP_B4 + t - 2 * MLP_H
+                                                                                             : MLP_NPARAM] = v;
     }
 }
 
-// grad[p] = sum over the block slots of part[slot][p] in float64; p = MLP_NPARAM is the loss.  64 columns
-// per block, 16 threads a column that take every 16th slot, added in order: 9 us for 256 slots (one thread a
+// grad[p] = sum over the block slots of part[slot][p]; p = MLP_NPARAM is the loss.  64 columns
+// per block, 16 threads a column that take every 16th slot, added in order: 6.6 us for 256 slots (one thread a
 // column over the 2,048 slots that 32 samples a block left: 500 us).
 constexpr int MLP_RED_G = 16;
-__global__ void __launch_bounds__(64 * MLP_RED_G) k_mlp_reduce(const float *part, int nslot, double *grad) {
+__global__ void __launch_bounds__(64 * MLP_RED_G) k_mlp_reduce(const double *part, int nslot, double *grad) {
     __shared__ double s[MLP_RED_G][64];
     const int c = threadIdx.x & 63, g = threadIdx.x >> 6, p = blockIdx.x * 64 + c;
     double v = 0.0;
     if (p <= MLP_NPARAM)
-        for (int b = g; b < nslot; b += MLP_RED_G) v += (double)part[(size_t)b * (MLP_NPARAM + 1) + p];
+        for (int b = g; b < nslot; b += MLP_RED_G) v += part[(size_t)b * (MLP_NPARAM + 1) + p];
     s[g][c] = v;
     __syncthreads();
     if (g == 0 && p <= MLP_NPARAM) {
