@@ -3346,16 +3346,16 @@ int dhip_batch_solve(dhip_batch_t *b, int32_t max_iter, double tol, int32_t rel,
         hipLaunchKernelGGL(k_batch_cut_count, cells, dim3(BPLAN), 0, s, a);
         hipLaunchKernelGGL(k_batch_cut_scan, dim3(b->nprob), dim3(BSCAN), 0, s, a);
         hipLaunchKernelGGL(k_batch_cut_fill, cells, dim3(BPLAN), 0, s, a);
+        const dim3 slots(blocks_for(4 * a.cut_total, BFLAT)), rows(blocks_for(a.row_total, ROWW_WAVES));
         if (a.cut_total > 0) {
-            const dim3 slots(blocks_for(4 * a.cut_total, BFLAT)), rows(blocks_for(a.row_total, ROWW_WAVES));
             hipLaunchKernelGGL(k_batch_local, dim3(blocks_for(a.cut_total, LOCAL_BLOCK)), dim3(LOCAL_BLOCK), 0, s, a);
             hipLaunchKernelGGL(k_batch_first, slots, dim3(BFLAT), 0, s, a);
             hipLaunchKernelGGL(k_batch_rank, dim3(b->nprob), dim3(BSCAN), 0, s, a);
             hipLaunchKernelGGL(k_batch_dofs, slots, dim3(BFLAT), 0, s, a);
             hipLaunchKernelGGL(k_batch_rows<false>, rows, dim3(64 * ROWW_WAVES), 0, s, a);
-            hipLaunchKernelGGL(k_batch_rowptr, dim3(b->nprob), dim3(BSCAN), 0, s, a);
-            hipLaunchKernelGGL(k_batch_rows<true>, rows, dim3(64 * ROWW_WAVES), 0, s, a);
         }
+        hipLaunchKernelGGL(k_batch_rowptr, dim3(b->nprob), dim3(BSCAN), 0, s, a);   // (a system without rows has one too)
+        if (a.cut_total > 0) hipLaunchKernelGGL(k_batch_rows<true>, rows, dim3(64 * ROWW_WAVES), 0, s, a);
         hipLaunchKernelGGL(k_batch_solve, dim3(std::min(b->nprob, c->cu_count)), dim3(BPT), (size_t)BP_LDS, s, a);
         return hipGetLastError();
     };

@@ -147,6 +147,31 @@ def test_batch_inner_solves_run_to_the_end(ctx):
     b.close()
 
 
+def test_batch_without_cut_tets(ctx):
+    """Problems whose level set cuts nothing, among others and alone: converged with no unknowns, row pointers (0).
+    The batch before leaves its memory behind."""
+    print("[gpu batch] nothing cut", flush=True)
+    meshes, phi, off = small_set(8, seed=13)
+    empty = [KuhnMesh.box(-2.0, 2.0, n) for n in (6, 5, 9)]
+    ep = [m.sample_p2(sphere(radius=9.0)).ravel() for m in empty]
+    eo = np.concatenate([[0], np.cumsum([p.size for p in ep])[:-1]]).astype(np.int64)
+    b = make_batch(ctx, meshes + empty, np.concatenate([phi] + ep), np.concatenate([off, eo + phi.size]))
+    b.solve(tol=1e-8)
+    assert np.all(b.stats()["status"] == D.OK) and np.all(b.stats()["ndof"][:8] > 0)
+    assert all(b.problem(p)["rowptr"].tolist() == [0] for p in range(8, 11))
+    b.close()
+    b = make_batch(ctx, empty, np.concatenate(ep), eo)
+    for graph in (False, True, True):
+        b.solve(tol=1e-8, graph=graph)
+        st = b.stats()
+        assert np.all(st["status"] == D.OK)
+        for k in ("ncut", "ndof", "nnz", "iters"):
+            assert np.all(st[k] == 0)
+        for p in range(3):
+            assert b.problem(p)["rowptr"].tolist() == [0]
+    b.close()
+
+
 def test_batch_zero_node_problem_isolated(ctx):
     print("[gpu batch] exact-zero node in one problem", flush=True)
     meshes, phi, off = small_set(4, seed=7)
