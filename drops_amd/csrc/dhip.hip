@@ -3103,6 +3103,9 @@ int dhip_ch_solve_learned(dhip_ch_t *h, dhip_mlp_t *q, int32_t *iters, double *r
 // ---------------------------------------------------------------------------
 // batched problems: planning, one persistent launch per solve (optionally a replayed hipGraph)
 // ---------------------------------------------------------------------------
+// largest pinned buffer that a batch holds for the caller's copies
+static const size_t BATCH_BOUNCE = (size_t)4 << 20;
+
 struct dhip_batch {
     dhip_ctx *ctx = nullptr;
     int32_t nprob = 0;
@@ -3419,7 +3422,8 @@ int dhip_batch_problem(dhip_batch_t *b, int32_t p, int32_t *rowptr, int32_t *col
     const BatchProb &P = b->hprob[p];
     const size_t nd = (size_t)st.ndof, nz = (size_t)st.nnz;
     // through pinned memory: copies to the caller's pageable arrays would each be staged and waited for (512
-    // solutions of 3,500 rows: 20 ms, now 7.4 ms with the stat entries kept from the solve)
+    // solutions of 3,500 rows: 20 ms, now 7.4 ms with the stat entries kept from the solve); a request beyond
+    // BATCH_BOUNCE goes in pieces of it
     struct Part { void *dst; const void *src; size_t bytes; } parts[5] = {
         {rowptr, b->rowptr.as<int32_t>() + P.row_off + p, sizeof(int32_t) * (nd + 1)},
         {colind, b->col.as<int32_t>() + P.nz_off, sizeof(int32_t) * nz},
@@ -3428,27 +3432,39 @@ int dhip_batch_problem(dhip_batch_t *b, int32_t p, int32_t *rowptr, int32_t *col
         {x, b->x.as<double>() + P.row_off, sizeof(double) * nd}};
     size_t total = 0;
     for (const Part &q : parts) total += q.dst ? (q.bytes + 15) & ~(size_t)15 : 0;
-    if (total > b->bounce_bytes) {
+    const size_t want = std::min(total, BATCH_BOUNCE);
+    if (want > b->bounce_bytes) {
         if (b->bounce) (void)hipHostFree(b->bounce);
         b->bounce = nullptr;
         b->bounce_bytes = 0;
-        if (hipHostMalloc((void **)&b->bounce, total, hipHostMallocDefault) != hipSuccess)
-            return set_error(c, DHIP_E_NOMEM, "%zu bytes of pinned memory", total);
-        b->bounce_bytes = total;
+        if (hipHostMalloc((void **)&b->bounce, want, hipHostMallocDefault) != hipSuccess)
+            return set_error(c, DHIP_E_NOMEM, "%zu bytes of pinned memory", want);
+        b->bounce_bytes = want;
     }
+    struct Piece { unsigned char *dst; size_t at, bytes; };
+    std::vector<Piece> pieces;
     size_t at = 0;
+    auto drain = [&]() -> hipError_t {
+        const hipError_t e = hipStreamSynchronize(c->stream);
+        if (e != hipSuccess) return e;
+        for (const Piece &q : pieces) std::memcpy(q.dst, b->bounce + q.at, q.bytes);
+        pieces.clear();
+        at = 0;
+        return hipSuccess;
+    };
     for (const Part &q : parts) {
-        if (!q.dst || !q.bytes) continue;
-        DHIP_HIPCHK(c, hipMemcpyAsync(b->bounce + at, q.src, q.bytes, hipMemcpyDeviceToHost, c->stream));
-        at += (q.bytes + 15) & ~(size_t)15;
+        if (!q.dst) continue;
+        for (size_t done = 0; done < q.bytes;) {
+            if (at >= b->bounce_bytes) DHIP_HIPCHK(c, drain());
+            const size_t bytes = std::min(q.bytes - done, b->bounce_bytes - at);
+            DHIP_HIPCHK(c, hipMemcpyAsync(b->bounce + at, (const unsigned char *)q.src + done, bytes,
+                                          hipMemcpyDeviceToHost, c->stream));
+            pieces.push_back({(unsigned char *)q.dst + done, at, bytes});
+            done += bytes;
+            at += (bytes + 15) & ~(size_t)15;
+        }
     }
-    DHIP_HIPCHK(c, hipStreamSynchronize(c->stream));
-    at = 0;
-    for (const Part &q : parts) {
-        if (!q.dst || !q.bytes) continue;
-        std::memcpy(q.dst, b->bounce + at, q.bytes);
-        at += (q.bytes + 15) & ~(size_t)15;
-    }
+    DHIP_HIPCHK(c, drain());
     return DHIP_OK;
 }
 
