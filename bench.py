@@ -233,9 +233,8 @@ def ch_leg(cells=96, steps=200, seed=1000, cpu_steps=None, with_cpu=True, space=
 
 def batch_leg(nprob=512, seed=0, steps=3, cpu_sample=8, with_cpu=True):
     """Batched configuration: `nprob` uneven P1 problems (ellipsoids, n^3 cells with n in 16..64) assembled
-    and solved (FP32 inner PCG, FP64 refinement, rel. residual 1e-8) in one persistent launch replayed as a
-    hipGraph; workgroup geometry from the autotuner; a sample of problems checked against the oracle's FP64
-    solution and timed on the CPU port."""
+    and solved (FP32 inner PCG, FP64 refinement, rel. residual 1e-8) by launches replayed as a
+    hipGraph; a sample of problems checked against the oracle's FP64 solution and timed on the CPU port."""
     from drops_amd import batch as BT
     t0 = time.perf_counter()
     probs = BT.make_problems(nprob, seed)
@@ -244,14 +243,10 @@ def batch_leg(nprob=512, seed=0, steps=3, cpu_sample=8, with_cpu=True):
     log(f"[bench] batch: {nprob} problems, {phi.size} level-set values generated in {time.perf_counter() - t0:.1f} s")
     out = {"workload": f"{nprob} P1 trace-FEM problems (mass + LB + h*stab, f = 3xy - x^3) on ellipsoids, semi-axes "
                        f"U(0.5,1.5), random rotations, [-2,2]^3 Kuhn meshes n^3 with n in 16..64 (seed {seed}); "
-                       f"assembly + Jacobi PCG (FP32 inner, FP64 refinement) to rel. residual 1e-8 in one launch"}
+                       f"assembly + Jacobi PCG (FP32 inner, FP64 refinement) to rel. residual 1e-8"}
     with D.Context(0) as ctx:
         b = ctx.batch(meshes, phi, off, rhs_kind=D.RHS_3XY_MINUS_X3)
-        choice, timings = tune.tune_batch(ctx, b)
-        out["tuned"] = {"threads": choice[0], "blocks_per_cu": choice[1], "prepass": choice[2],
-                        "solve_threads": choice[3] or None,
-                        "candidates_ms": {f"{k[0]}x{k[1]}{'+pre' if k[2] else ''}{f'+pcg{k[3]}' if k[3] else ''}":
-                                          1e3 * v for k, v in timings.items()}}
+        b.solve(tol=1e-8)               # code object load
         b.solve(tol=1e-8, graph=True)   # capture
         ctx.profile_reset()
         ctx.profile(True)
@@ -263,7 +258,7 @@ def batch_leg(nprob=512, seed=0, steps=3, cpu_sample=8, with_cpu=True):
         ctx.profile(False)
         gms, gcnt = ctx.profile_get("batch_graph")
         st = b.stats()
-        dur = st["end_s"] - st["start_s"]
+        pcg = st["end_s"] - st["assembled_s"]   # the problems are assembled together, then solved one by one
         span = st["end_s"].max() - st["start_s"].min()
         n_ok = int((st["status"] == D.OK).sum())
         # algorithmic bytes: level set read once, then per inner iteration the FP32 matrix (value +
@@ -280,11 +275,11 @@ def batch_leg(nprob=512, seed=0, steps=3, cpu_sample=8, with_cpu=True):
                     "cut_tets_total": int(st["ncut"].sum()), "dofs_range": [int(st["ndof"].min()), int(st["ndof"].max())],
                     "inner_iters_mean": float(st["iters"].mean()), "refinements_mean": float(st["outer"].mean()),
                     "resid_max": float(st["resid"].max()), "device_span_s": float(span),
-                    "longest_problem_s": float(dur.max()), "mean_problem_s": float(dur.mean()),
-                    "assembly_share_longest": float(((st["assembled_s"] - st["start_s"]) / np.maximum(dur, 1e-12))[dur.argmax()]),
+                    "longest_pcg_s": float(pcg.max()), "mean_pcg_s": float(pcg.mean()),
+                    "assembly_s": float(st["assembled_s"].min() - st["start_s"].min()),
                     "algorithmic_gbs": alg / s_batch / 1e9, "algorithmic_frac_of_hbm_peak": alg / s_batch / 8e12})
         log(f"[bench] batch: {s_batch * 1e3:.2f} ms per batch of {nprob} ({n_ok} converged), "
-            f"longest problem {dur.max() * 1e3:.1f} ms, mean {dur.mean() * 1e3:.1f} ms")
+            f"longest PCG {pcg.max() * 1e3:.1f} ms, mean {pcg.mean() * 1e3:.1f} ms")
         if with_cpu:
             sys.path.insert(0, os.path.join(ROOT, "oracle"))
             import oracle as O

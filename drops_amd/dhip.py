@@ -491,7 +491,7 @@ class CahnHilliard:
 
 
 class Batch:
-    """Many independent P1 problems assembled and solved in one launch (dhip_batch_*).
+    """Many independent P1 problems assembled and solved in one call (dhip_batch_*).
     meshes: list of KuhnMesh; phi: one float64 array holding every problem's half-grid level set
     (host array, or a device pointer with phi_count and where=DEVICE); offsets: first value of
     each problem in phi; lcs: per problem operator combination (default (1, 1, h) of its mesh)."""
@@ -523,7 +523,7 @@ class Batch:
         self.ctx.check(self.L.dhip_batch_solve(self.h, int(max_iter), float(tol), int(rel), int(graph)))
 
     def stats(self):
-        """dict of per-problem numpy arrays: status, ncut, ndof, nnz, iters, outer, resid, start_s, end_s"""
+        """dict of per-problem numpy arrays: status, ncut, ndof, nnz, iters, outer, resid, start_s, end_s, assembled_s"""
         st = (BatchStat * self.n)()
         self.ctx.check(self.L.dhip_batch_stats(self.h, st))
         return {k: np.array([getattr(x, k) for x in st]) for k, _ in BatchStat._fields_}

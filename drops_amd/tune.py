@@ -1,4 +1,4 @@
-"""Autotuner of the persistent solvers' block geometry and exchange, and of the batched solve.
+"""Autotuner of the persistent solvers' block geometry and exchange.
 
 The persistent PCG/GMRES kernels give each block a contiguous range of rows.
 More rows per block make a block's gather phase longer; more blocks make every
@@ -41,37 +41,18 @@ def tune_pcg(ctx, A, b_dev, x_dev, zero_dev, n, tol=1e-8, precision=D.FP64, cand
     return choice, timings
 
 
-# the batch keys (threads, workgroups per CU, pre-pass, solve threads or 0) of a candidate; the library's batched
-# launches have one geometry, so one candidate serves
+# (threads, workgroups per CU, pre-pass, solve threads or 0) of the batched launches
 BATCH_CANDIDATES = ((512, 1, 1, 0),)
 
 
 def tune_batch(ctx, batch, tol=1e-8, candidates=BATCH_CANDIDATES, reps=2):
-    """The batch keys among `candidates`: times `reps`
-    graph replays per candidate (best of; the capture is untimed) on the caller's problem set, after
-    one untimed launch, and leaves the fastest on the context.  Returns
-    ((threads, blocks_per_cu, prepass, solve_threads), {candidate: seconds})."""
-    timings = {}
-    batch.solve(tol=tol)   # first launch: code object load and first-touch costs stay out of the timings
-    for threads, bpc, pre, sthreads in candidates:
-        ctx.tune("batch_threads", threads)
-        ctx.tune("batch_blocks_per_cu", bpc)
-        ctx.tune("batch_prepass", pre)
-        ctx.tune("batch_split", 1 if sthreads else 0)
-        if sthreads:
-            ctx.tune("batch_solve_threads", sthreads)
-        batch.solve(tol=tol, graph=True)   # captures this candidate's graph (untimed)
-        best = np.inf
-        for _ in range(reps):
-            t0 = time.perf_counter()
-            batch.solve(tol=tol, graph=True)
-            best = min(best, time.perf_counter() - t0)
-        timings[(threads, bpc, pre, sthreads)] = best
-    choice = min(timings, key=timings.get)
-    ctx.tune("batch_threads", choice[0])
-    ctx.tune("batch_blocks_per_cu", choice[1])
-    ctx.tune("batch_prepass", choice[2])
-    ctx.tune("batch_split", 1 if choice[3] else 0)
-    if choice[3]:
-        ctx.tune("batch_solve_threads", choice[3])
-    return choice, timings
+    """The batched launches have one geometry, so there is nothing to choose and nothing is set: returns the first
+    candidate and {it: seconds}, the best of `reps` graph replays, for programs that report them."""
+    batch.solve(tol=tol)   # code object load and first-touch costs stay out of the timing
+    batch.solve(tol=tol, graph=True)   # captures (untimed)
+    best = np.inf
+    for _ in range(reps):
+        t0 = time.perf_counter()
+        batch.solve(tol=tol, graph=True)
+        best = min(best, time.perf_counter() - t0)
+    return candidates[0], {candidates[0]: best}

@@ -109,7 +109,8 @@ int dhip_solver_probe(dhip_ctx_t *ctx, int32_t on, uint64_t *ticks, int32_t *nbl
  * (L2-scope) loads and stores of the exchanged values without fences, 2 (default) as 1 and the FP64
  * PCG with generation-tagged 16-byte records and its block's gathered values staged in LDS (the
  * same iterates bit for bit while a block's slice fits its LDS; the single-reduction kernel
- * otherwise), 3 as 2 with the FP64 PCG in the pipelined arrangement of CG (one vector of records
+ * otherwise), as are the FP32 inner iterations of DHIP_FP32_IR (single-reduction recurrences; the
+ * two-reduction form where a slice does not fit or FP32 does not carry them), 3 as 2 with the FP64 PCG in the pipelined arrangement of CG (one vector of records
  * per iteration, the wait for the block partials overlapped with the next product; iterates equal
  * CG's up to rounding, and b - A x is checked, restarting from it if needed, before it stops);
  * "gmres_precision" -- DHIP_FP64 (default) or DHIP_FP32_IR for dhip_gmres and
@@ -295,7 +296,8 @@ int dhip_axpy(dhip_ctx_t *ctx, int64_t n, double a, const double *x, double *y, 
  * iterations / final residual (relative if rel != 0).  Returns DHIP_OK on
  * convergence, DHIP_E_NOT_CONVERGED otherwise (the reference's `false`).
  * precision DHIP_FP32_IR: FP32 inner PCG sweeps inside an FP64 iterative
- * refinement loop; *max_iter then counts inner iterations. */
+ * refinement loop; *max_iter then counts inner iterations.  A sweep runs to 1e-4 of the residual it
+ * starts from, or 400 iterations. */
 int dhip_pcg(dhip_ctx_t *ctx, const dhip_csr_t *A, int32_t pc, const double *b, double *x,
              int32_t where, int32_t *max_iter, double *tol, int32_t rel, int32_t precision);
 
@@ -493,8 +495,9 @@ typedef struct {
     int32_t ncut, ndof, nnz;
     int32_t iters, outer; /* FP32 inner iterations in total, FP64 refinement steps */
     double resid;         /* final FP64 relative residual */
-    double start_s, end_s;  /* device wall clock at the start and end of the problem in the last solve */
-    double assembled_s;     /* device wall clock when its PCG started */
+    double start_s, end_s;  /* device wall clock of the last solve: start of the assembly, which all problems share,
+                             * and end of this problem's PCG (a failed one: of its classification) */
+    double assembled_s;     /* when its PCG started: its system is assembled, the larger problems have been taken */
 } dhip_batch_stat_t;
 /* Plans the batch: counts each problem's cut tets and cut-tet vertices on the device and sizes
  * the per-problem scratch.  phi holds all level sets (phi_count values, DHIP_HOST: copied;
