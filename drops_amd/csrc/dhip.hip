@@ -2039,14 +2039,16 @@ static int gmres_core(dhip_ctx *c, const dhip_csr *A, const double *diag, const 
     if (rc) return rc;
     // The pair form where a thread has more than one row, so that the basis is not in registers, and the average
     // block's CSR slice would not fit in LDS; up to two pairs a thread.  128,352 unknowns, one row a thread: 61 us an
-    // iteration with the register basis, 76 in pairs; 191,104 unknowns: 107 us row by row, 72 in pairs.
-    const int64_t pair_per = (n / 2 + c->cu_count - 1) / c->cu_count;
+    // iteration with the register basis, 76 in pairs; 191,104 unknowns: 107 us row by row, 72 in pairs.  A block
+    // takes half of the "pcg_rows_per_block" in pairs where that is set.
+    int64_t pair_per = std::max<int64_t>((n / 2 + c->cu_count - 1) / c->cu_count, (c->pcg_rows_per_block + 1) / 2);
     const bool pair = block2 && rpt > 1 && diag && !left_pc && (c->coherent_exchange || f32) && n > 0 && A->nnz > 0 &&
                       pair_per <= 2 * PB &&
                       ((n + nb - 1) / nb + 1) * 4 + (A->nnz / nb) * 12 + 16 > (int64_t)LDS_BYTES;
     if (pair) {
-        rpt = pair_per <= PB ? 2 : 4;
         nb = (unsigned)((n / 2 + pair_per - 1) / pair_per);
+        pair_per = (n / 2 + nb - 1) / nb;   // (the kernel's)
+        rpt = pair_per <= PB ? 2 : 4;
     }
     DHIP_HIPCHK(c, c->bar.ensure(sizeof(SyncSlot) * (nb + 1)));
     DHIP_HIPCHK(c, c->red_tmp.ensure(sizeof(double) * 2 * (size_t)nb * KMAX + 64));

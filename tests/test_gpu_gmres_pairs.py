@@ -40,6 +40,17 @@ def test_pair_form(ctx, cells):
     x32, it32 = step(ctx, ch, 7)
     assert np.linalg.norm(x32 - x) <= 1e-3 * np.linalg.norm(x) and abs(it32 - it) <= 0.3 * it
     ch.set_precision(D.FP64)
+    if cells == 97:   # rows per block set by the caller, one and two pairs a thread
+        for rows in (900, 1700):
+            ctx.tune("pcg_rows_per_block", rows)
+            ctx.solver_probe(True)
+            try:
+                xr, itr = step(ctx, ch, 7)
+                blocks = ctx.solver_probe(False).shape[0]
+            finally:
+                ctx.tune("pcg_rows_per_block", 0)
+            assert blocks == -(-ch.n // (rows // 2))
+            assert abs(it - itr) <= 0.02 * itr + 2 and np.linalg.norm(xr - x) <= 1e-3 * np.linalg.norm(x)
     if cells == 82:
         ctx.tune("coherent_exchange", 0)
         try:
