@@ -192,10 +192,6 @@ static void derive_tables(Tables &T) {
                                                   kuhn[k][j][2] - kuhn[k][i][2]);
     // quadrature rules (num/discretize.cpp:153-211, 234-238, 263-296; num/discretize.tpp:754-762)
     const double s15 = std::sqrt(15.0);
-    const double q2n[4][3] = {{1., 0., 0.}, {0., 1., 0.}, {0., 0., 1.}, {1. / 3., 1. / 3., 1. / 3.}};
-    std::memcpy(T.q2n, q2n, sizeof q2n);
-    T.q2w[0] = T.q2w[1] = T.q2w[2] = 1. / 24.;
-    T.q2w[3] = 0.375;
     {
         const double A1 = (6.0 - s15) / 21.0, B1 = (9.0 + 2.0 * s15) / 21.0;
         const double A2 = (6.0 + s15) / 21.0, B2 = (9.0 - 2.0 * s15) / 21.0;

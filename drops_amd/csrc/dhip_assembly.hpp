@@ -499,7 +499,8 @@ __device__ inline void local_p1_one(const LocalArgs &a, int64_t c, LocalP1Shared
         facet_qr(X, vb, absdet, nrm);
         double af = (w & 4) ? 0.5 : 1.;
         af *= absdet;
-        // Quad2 composite: mass + numbering integrals; its nodes are the corners and the barycentre
+        // Quad2 composite (num/discretize.cpp:234-238): mass + numbering integrals; its nodes are the corners (weight
+        // 1/24) and the barycentre (3/8)
 #pragma unroll
         for (int qn = 0; qn < 4; ++qn) {
             double nb[4];

@@ -49,7 +49,6 @@ struct Tables {
     int8_t p2_of27[6][27];     // P2 dof of tet k at cell node (-1 if the tet has no node there)
     int8_t slot_delta[15][3];  // neighbour offset of each slot
     double lat_b[10][4];
-    double q2n[4][3], q2w[4];  // Quad2_2DDataCL
     double q5n[7][3], q5w[7];  // Quad5_2DDataCL
     double v5n[15][4];         // Quad5DataCL nodes
     double v5c1, v5c2;         // Quad5CL::quad weights of node groups 1 and 2
