@@ -1,4 +1,4 @@
-// dhip_batch.hpp -- many independent P1 trace-FEM problems assembled and solved in one launch.
+// dhip_batch.hpp -- many independent P1 trace-FEM problems assembled and solved together.
 //
 // Each problem has its own Kuhn brick, level set and sizes.  The assembly runs step by step over all
 // problems at once with the single-problem path's per-item code (cell_cut_mask, local_p1_one, qualify_one,
@@ -105,7 +105,8 @@ __global__ void __launch_bounds__(BPLAN) k_batch_verts(const BatchProb *prob, co
 //   k_batch_rows<>      one wave per row: count, then (k_batch_rowptr per problem) fill
 // Threads find their problem from the offsets' table; a problem that failed a step (exact zero, capacity)
 // is skipped from there on.  512 problems of 16^3 to 64^3 cells (5.1 M cut
-// tets, 1.8 M rows): 27.0 -> 10.1 ms, local matrices 5.1, rows 1.0 + 2.1, cells 0.83 + 0.25, owners 0.5, the rest 0.3.
+// tets, 1.8 M rows): 27.0 -> 8.0 ms, local matrices 2.9 (5.1 before they list their facets), rows 1.1 + 2.1, cells
+// 0.83 + 0.25, owners 0.55, the rest 0.3.
 // ---------------------------------------------------------------------------
 struct BatchArgs {
     const BatchProb *prob;
@@ -592,7 +593,8 @@ __device__ __noinline__ void batch_pcg_memory(const BatchArgs &a, int p, BatchSt
 // An iteration is three barriers, two workgroup sums and the LDS gathers of the search direction (about 7
 // cycles a wave's 64 against 2 without bank conflicts).  Measured a row count's iteration with 200 problems at
 // once: 765 rows 1.9 us, 1,543 2.5, 2,471 3.4, 3,555 4.7, 4,682 9.7, 7,604 13.7, 9,372 20, 12,936 30; with
-// every vector and the matrix in memory 15 to 60 us.  512 problems of 16^3 to 64^3 cells: all PCGs 70 -> 18.5 ms.
+// every vector and the matrix in memory 15 to 60 us.  512 problems of 16^3 to 64^3 cells: all PCGs 70 -> 18.5 ms,
+// 13.4 with inner_tolerance.
 // ---------------------------------------------------------------------------
 constexpr int BPT = 512;
 constexpr int BPW = BPT / 64;
@@ -1027,7 +1029,7 @@ __device__ __noinline__ void batch_pcg_chip(const BatchArgs &a, int p, BatchStat
     st.status = status == 0 ? DHIP_OK : DHIP_E_NOT_CONVERGED;
 }
 
-// The PCG of every assembled problem: problems from the second queue counter, largest first.
+// The PCG of every assembled problem: problems from the queue, largest first.
 __global__ void __launch_bounds__(BPT) k_batch_solve(BatchArgs a) {
     __shared__ int sh_p;
     for (;;) {
@@ -1043,7 +1045,7 @@ __global__ void __launch_bounds__(BPT) k_batch_solve(BatchArgs a) {
         if (st.status == DHIP_OK) {
             st.t_asm = wall_clock64();
             const int slots = (st.ndof + BPT - 1) / BPT;
-            // the smallest size class that holds the problem; the LDS of the classes up to 27 slots fits (asserted)
+            // the smallest size class that holds the problem; the LDS of every class fits (asserted)
             switch (slots) {
                 case 0: case 1: batch_pcg_chip<1, 0, 0, false>(a, p, st); break;
                 case 2: batch_pcg_chip<2, 0, 0, false>(a, p, st); break;
